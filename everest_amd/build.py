@@ -48,23 +48,30 @@ def ext_suffix():
     return sysconfig.get_config_var("EXT_SUFFIX") or ".so"
 
 
-HIP_UNITS = ("tm_abi.hip", "tm_sweep.hip", "tm_build.hip", "tm_server.hip", "tm_batch.hip", "tm_noalloc.hip", "tm_kv_n4_single.hip", "tm_kv_n4_multi.hip",
-             "tm_kv_n4_aux.hip", "tm_kv_n8_single.hip", "tm_kv_n8_multi.hip", "tm_kv_n8_aux.hip")
+HIP_UNITS = ("tm_abi.hip", "tm_sweep.hip", "tm_build.hip", "tm_server.hip", "tm_batch.hip", "tm_noalloc.hip")
+# the mining kernel's instantiations (tm_variants.h), each compiled on its own:
+# node map, enumerate, instrumented, register cap, multi-query
+HIP_VARIANTS = [(n, 0, 0, w, m) for n in (8, 4) for w in (6, 5, 4, 1) for m in (0, 1)] + \
+               [(n, 0, 2, 1, 0) for n in (8, 4)] + [(n, e, i, 1, 0) for n in (8, 4) for e, i in ((0, 1), (1, 0))]
 
 
-def build_hip():
+def build_hip(objdir=None, out=None, variants=HIP_VARIANTS):
     """Each translation unit compiled on its own (in parallel), then linked."""
-    out = os.path.join(LIB, "libtm_hip.so")
-    objdir = os.path.join(LIB, "obj")
+    out = out or os.path.join(LIB, "libtm_hip.so")
+    objdir = objdir or os.path.join(LIB, "obj")
     os.makedirs(objdir, exist_ok=True)
 
-    def unit(src):
-        obj = os.path.join(objdir, os.path.splitext(src)[0] + ".o")
-        _run([HIPCC] + HIP_FLAGS + ["-c", "-I" + INC, "-I" + HIP_SRC, os.path.join(HIP_SRC, src), "-o", obj])
+    def unit(job):
+        src, variant = job
+        name = os.path.splitext(src)[0] + ("_%d_%d_%d_%d_%d" % variant if variant else "")
+        obj = os.path.join(objdir, name + ".o")
+        defs = ["-DTMV_VARIANT=" + ",".join(map(str, variant))] if variant else []
+        _run([HIPCC] + HIP_FLAGS + defs + ["-c", "-I" + INC, "-I" + HIP_SRC, os.path.join(HIP_SRC, src), "-o", obj])
         return obj
 
-    with ThreadPoolExecutor(max_workers=min(len(HIP_UNITS), os.cpu_count() or 4)) as ex:
-        objs = list(ex.map(unit, HIP_UNITS))
+    jobs = [("tm_kv.hip", v) for v in variants] + [(u, None) for u in HIP_UNITS]
+    with ThreadPoolExecutor(max_workers=min(len(jobs), os.cpu_count() or 4)) as ex:
+        objs = list(ex.map(unit, jobs))
     _run([HIPCC] + HIP_FLAGS + ["-shared"] + objs + ["-pthread", "-o", out])
     return out
 
@@ -102,7 +109,7 @@ def build_csr_plugin():
 
 def build_oracle():
     subprocess.check_call(["make", "-s", "-C", os.path.join(ROOT, "oracle"), "libtm_oracle.so"])
-    if os.path.isdir("/root/reference"):
+    if os.path.isfile("/root/reference/src/core/cpu/Graph.cc"):
         subprocess.check_call(["make", "-s", "-C", os.path.join(ROOT, "oracle"), "ref"])
 
 

@@ -1,5 +1,5 @@
 // tm_variants.cuh -- definition of one mining-kernel variant function
-// (included by the tm_kv_*.hip units only).
+// (included by tm_kv.hip only).
 #pragma once
 #include <string>
 

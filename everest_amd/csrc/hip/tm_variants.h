@@ -1,5 +1,5 @@
 // tm_variants.h -- the mining kernel's instantiations, each behind a plain
-// function (defined in the tm_kv_*.hip units, compiled in parallel).
+// function (tm_kv.hip, compiled once per variant, in parallel).
 //
 // A variant is named by node-map width (4 or 8), enumerate, instrumented (1:
 // reference work, 2: metered bytes),
