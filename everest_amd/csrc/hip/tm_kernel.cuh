@@ -265,14 +265,30 @@ __device__ __forceinline__ int pair_last(const tm_graph_view &g, int x, int y, i
 }
 
 // Edges x -> y with positions in (p, pend), searched in the shorter of out(x)
-// and in(y).
+// and in(y) (the list is chosen first, so the search is in the code once).
 __device__ __forceinline__ int edge_count(const tm_graph_view &g, int x, int y, int p, int pend,
                                           Meter *mt = nullptr) {
-  int olo = g.outR[x], ohi = g.outR[x + 1];
-  int ilo = g.inR[y], ihi = g.inR[y + 1];
+  const int olo = g.outR[x], ohi = g.outR[x + 1];
+  const int ilo = g.inR[y], ihi = g.inR[y + 1];
   if (mt) mt->b += 16;
-  if (ohi - olo <= ihi - ilo) return pair_count(g.outPairNbr, g.outPairPos, olo, ohi, y, p, pend, mt);
-  return pair_count(g.inPairNbr, g.inPairPos, ilo, ihi, x, p, pend, mt);
+  const bool o = ohi - olo <= ihi - ilo;
+  return pair_count(o ? g.outPairNbr : g.inPairNbr, o ? g.outPairPos : g.inPairPos, o ? olo : ilo, o ? ohi : ihi,
+                    o ? y : x, p, pend, mt);
+}
+
+// The slots [*s0, *s1) of the pair x -> y in the pair index of the shorter of
+// out(x) (*dir 0) and in(y) (*dir 1).
+__device__ __forceinline__ void pair_range(const tm_graph_view &g, int x, int y, int *s0, int *s1, int *dir,
+                                           Meter *mt = nullptr) {
+  const int olo = g.outR[x], ohi = g.outR[x + 1];
+  const int ilo = g.inR[y], ihi = g.inR[y + 1];
+  if (mt) mt->b += 16;
+  const bool o = ohi - olo <= ihi - ilo;
+  const int *pn = o ? g.outPairNbr : g.inPairNbr;
+  const int hi = o ? ohi : ihi, key = o ? y : x;
+  *dir = o ? 0 : 1;
+  *s0 = lower_bound_i(pn, o ? olo : ilo, hi, key, mt);
+  *s1 = gallop_ub(pn, *s0, hi, key, mt);
 }
 
 // Candidate list of motif edge j: slots [lo, hi) of `pos` (and `nbr` for new
@@ -291,24 +307,20 @@ __device__ __forceinline__ CandList cand_start(const tm_graph_view &g, const tm_
   L.dir = 0;
   const int kind = SP::kind(md, j);
   const int mode = SP::smode(md, j);
-  if (kind == TM_K_NEW_DST) {
-    const int x = sel(m, SP::a(md, j));
-    L.pos = g.outPos;
-    L.nbr = g.outNbr;
-    L.hi = g.outR[x + 1];
+  if (kind != TM_K_CLOSE) {
+    // a new node: the out-list of the edge's source or the in-list of its destination
+    const bool out = kind == TM_K_NEW_DST;
+    const int x = sel(m, out ? SP::a(md, j) : SP::b(md, j));
+    const int *R = out ? g.outR : g.inR;
+    L.pos = out ? g.outPos : g.inPos;
+    L.nbr = out ? g.outNbr : g.inNbr;
+    L.hi = R[x + 1];
     if (mt) mt->b += 8;
     if (mode == TM_S_OUT_SELF) L.lo = g.outSelf[p] + 1;
     else if (mode == TM_S_OUT_NEXT) L.lo = g.outNext[p];
-    else L.lo = upper_bound_i(g.outPos, g.outR[x], L.hi, p, mt);
-  } else if (kind == TM_K_NEW_SRC) {
-    const int y = sel(m, SP::b(md, j));
-    L.pos = g.inPos;
-    L.nbr = g.inNbr;
-    L.hi = g.inR[y + 1];
-    if (mt) mt->b += 8;
-    if (mode == TM_S_IN_SELF) L.lo = g.inSelf[p] + 1;
+    else if (mode == TM_S_IN_SELF) L.lo = g.inSelf[p] + 1;
     else if (mode == TM_S_IN_NEXT) L.lo = g.inNext[p];
-    else L.lo = upper_bound_i(g.inPos, g.inR[y], L.hi, p, mt);
+    else L.lo = upper_bound_i(L.pos, R[x], L.hi, p, mt);
   } else {
     const int x = sel(m, SP::a(md, j)), y = sel(m, SP::b(md, j));
     L.nbr = nullptr;
@@ -319,20 +331,9 @@ __device__ __forceinline__ CandList cand_start(const tm_graph_view &g, const tm_
       if (mt) mt->b += 8;
       L.hi = gallop_ub(g.outPairNbr, L.lo, g.outR[x + 1], y, mt);
     } else {
-      int olo = g.outR[x], ohi = g.outR[x + 1];
-      int ilo = g.inR[y], ihi = g.inR[y + 1];
-      if (mt) mt->b += 16;
       int s0, s1;
-      if (ohi - olo <= ihi - ilo) {
-        s0 = lower_bound_i(g.outPairNbr, olo, ohi, y, mt);
-        s1 = gallop_ub(g.outPairNbr, s0, ohi, y, mt);
-        L.pos = g.outPairPos;
-      } else {
-        s0 = lower_bound_i(g.inPairNbr, ilo, ihi, x, mt);
-        s1 = gallop_ub(g.inPairNbr, s0, ihi, x, mt);
-        L.pos = g.inPairPos;
-        L.dir = 1;
-      }
+      pair_range(g, x, y, &s0, &s1, &L.dir, mt);
+      L.pos = L.dir ? g.inPairPos : g.outPairPos;
       L.lo = upper_bound_i(L.pos, s0, s1, p, mt);
       L.hi = s1;
     }
@@ -362,10 +363,11 @@ __device__ __forceinline__ unsigned long long leaf_count(const tm_graph_view &g,
   // skipx: the caller knows that pair has no edge left in the window)
   const bool out = SP::kind(md, j) == TM_K_NEW_DST;
   const int base = out ? sel(m, SP::a(md, j)) : sel(m, SP::b(md, j));
-#pragma unroll
-  for (int i = 0; i < MAXN; i++) {
-    if (i >= nm || ((zmask >> i) & 1) || m[i] == skipx || (g.no_self_loops && m[i] == base)) continue;
-    c -= out ? edge_count(g, base, m[i], p, pend, mt) : edge_count(g, m[i], base, p, pend, mt);
+#pragma unroll 1
+  for (int i = 0; i < nm; i++) {
+    const int x = sel(m, i);
+    if (((zmask >> i) & 1) || x == skipx || (g.no_self_loops && x == base)) continue;
+    c -= edge_count(g, out ? base : x, out ? x : base, p, pend, mt);
   }
   return (unsigned long long)c;
 }
@@ -419,49 +421,25 @@ __device__ __forceinline__ void tail2_range(const tm_graph_view &g, const tm_mot
   const int k = SP::M(md) - 1;
   const int kind = SP::kind(md, k);
   *bdir = 0;
-  if (tail2_mode<SP>(md) == T2_JOIN) {
-    // edges between w and y at y: y's in-list when edge k is w -> y, else its out-list
-    const int w = SP::mapped(md, k - 1);
-    const bool into_y = SP::a(md, k) == w;
-    const int y = sel(m, into_y ? SP::b(md, k) : SP::a(md, k));
-    const int *pos = into_y ? g.inPos : g.outPos;
-    const int *R = into_y ? g.inR : g.outR;
-    const int e = R[y + 1];
+  const int *pos;
+  int s0, s1;
+  if (tail2_mode<SP>(md) == T2_JOIN || kind != TM_K_CLOSE) {
+    // one node's list: a new last node's, or (join) the edges between w and
+    // y at y: y's in-list when edge k is w -> y, else its out-list
+    bool in = kind == TM_K_NEW_SRC;
+    if (kind == TM_K_CLOSE) in = SP::a(md, k) == SP::mapped(md, k - 1);
+    const int y = sel(m, in ? SP::b(md, k) : SP::a(md, k));
+    const int *R = in ? g.inR : g.outR;
+    pos = in ? g.inPos : g.outPos;
+    s0 = R[y];
+    s1 = R[y + 1];
     if (mt) mt->b += 8;
-    *lo = upper_bound_i(pos, R[y], e, pa0, mt);
-    *hi = gallop_lb(pos, *lo, e, pend, mt);
-  } else if (kind == TM_K_NEW_DST) {
-    const int x = sel(m, SP::a(md, k));
-    const int e = g.outR[x + 1];
-    if (mt) mt->b += 8;
-    *lo = upper_bound_i(g.outPos, g.outR[x], e, pa0, mt);
-    *hi = gallop_lb(g.outPos, *lo, e, pend, mt);
-  } else if (kind == TM_K_NEW_SRC) {
-    const int y = sel(m, SP::b(md, k));
-    const int e = g.inR[y + 1];
-    if (mt) mt->b += 8;
-    *lo = upper_bound_i(g.inPos, g.inR[y], e, pa0, mt);
-    *hi = gallop_lb(g.inPos, *lo, e, pend, mt);
   } else {
-    const int x = sel(m, SP::a(md, k)), y = sel(m, SP::b(md, k));
-    const int olo = g.outR[x], ohi = g.outR[x + 1];
-    const int ilo = g.inR[y], ihi = g.inR[y + 1];
-    const int *pos;
-    int s0, s1;
-    if (mt) mt->b += 16;
-    if (ohi - olo <= ihi - ilo) {
-      s0 = lower_bound_i(g.outPairNbr, olo, ohi, y, mt);
-      s1 = gallop_ub(g.outPairNbr, s0, ohi, y, mt);
-      pos = g.outPairPos;
-    } else {
-      s0 = lower_bound_i(g.inPairNbr, ilo, ihi, x, mt);
-      s1 = gallop_ub(g.inPairNbr, s0, ihi, x, mt);
-      pos = g.inPairPos;
-      *bdir = 1;
-    }
-    *lo = upper_bound_i(pos, s0, s1, pa0, mt);
-    *hi = gallop_lb(pos, *lo, s1, pend, mt);
+    pair_range(g, sel(m, SP::a(md, k)), sel(m, SP::b(md, k)), &s0, &s1, bdir, mt);
+    pos = *bdir ? g.inPairPos : g.outPairPos;
   }
+  *lo = upper_bound_i(pos, s0, s1, pa0, mt);
+  *hi = gallop_lb(pos, *lo, s1, pend, mt);
 }
 
 // Matches of the last two edges whose last edge is edge k's candidate at
@@ -475,52 +453,43 @@ __device__ __forceinline__ unsigned long long tail2_item(const tm_graph_view &g,
   const int M = SP::M(md);
   const int j = M - 2, k = M - 1;
   const int nm = SP::mapped(md, j);
-  const int kk = SP::kind(md, k);
-  if (tail2_mode<SP>(md) == T2_JOIN) {
-    // q = an edge between y and z after A's first candidate: the candidates
-    // of A whose new node is z (edges between A's node and z) before it
-    const int w = SP::mapped(md, j);
-    const bool into_y = SP::a(md, k) == w;
-    const int qp = into_y ? g.inPos[slot] : g.outPos[slot];
-    const int zz = into_y ? g.inNbr[slot] : g.outNbr[slot];
-    if (mt) mt->b += 8;
-    if (in_first(m, nm, zz)) return 0ull;  // z must be a new node
-    const bool aout = SP::kind(md, j) == TM_K_NEW_DST;
-    const int *ap = aout ? g.outPos : g.inPos;
-    const int base = aout ? sel(m, SP::a(md, j)) : sel(m, SP::b(md, j));
-    if (mt) mt->b += 4;
-    const int p0 = ap[alo] - 1;
-    return (unsigned long long)(aout ? edge_count(g, base, zz, p0, qp, mt) : edge_count(g, zz, base, p0, qp, mt));
-  }
+  const int kj = SP::kind(md, j), kk = SP::kind(md, k);
+  const bool join = tail2_mode<SP>(md) == T2_JOIN;
+  // the candidate q of edge k and its other end z; in a join, an edge between
+  // y and z after A's first candidate
   int qpos, z = -1;
-  if (kk == TM_K_NEW_DST) {
-    qpos = g.outPos[slot];
-    z = g.outNbr[slot];
-  } else if (kk == TM_K_NEW_SRC) {
-    qpos = g.inPos[slot];
-    z = g.inNbr[slot];
+  if (join || kk != TM_K_CLOSE) {
+    bool in = kk == TM_K_NEW_SRC;
+    if (join) in = SP::a(md, k) == SP::mapped(md, j);
+    qpos = in ? g.inPos[slot] : g.outPos[slot];
+    z = in ? g.inNbr[slot] : g.outNbr[slot];
+    if (mt) mt->b += 8;
+    if (in_first(m, nm, z)) return 0ull;  // z must be a new node
   } else {
     qpos = bdir ? g.inPairPos[slot] : g.outPairPos[slot];
+    if (mt) mt->b += 4;
   }
-  if (mt) mt->b += kk == TM_K_CLOSE ? 4 : 8;
-  if (kk != TM_K_CLOSE && in_first(m, nm, z)) return 0ull;
-  const int kj = SP::kind(md, j);
   const int *apos = kj == TM_K_NEW_DST ? g.outPos : (kj == TM_K_NEW_SRC ? g.inPos : (adir ? g.inPairPos : g.outPairPos));
-  int r = lower_bound_i(apos, alo, ahi, qpos, mt) - alo;
-  if (r <= 0 || kj == TM_K_CLOSE) return r > 0 ? (unsigned long long)r : 0ull;
-  // edge j's candidates before q whose new node is taken: edges between
-  // A's node and that node in [first candidate, q)
+  int r = 0;
+  if (!join) {
+    r = lower_bound_i(apos, alo, ahi, qpos, mt) - alo;
+    if (r <= 0 || kj == TM_K_CLOSE) return r > 0 ? (unsigned long long)r : 0ull;
+  }
+  // edges between A's node and x in [first candidate, q): in a join those to
+  // z are the count, else those to a taken node (a mapped one, or z) are not
+  // candidates of edge j
   const int p0 = apos[alo] - 1;
   if (mt) mt->b += 4;
   const bool out = kj == TM_K_NEW_DST;
   const int base = out ? sel(m, SP::a(md, j)) : sel(m, SP::b(md, j));
-#pragma unroll
-  for (int i = 0; i < MAXN; i++) {
-    if (i >= nm || ((zmask >> i) & 1) || (g.no_self_loops && m[i] == base)) continue;
-    r -= out ? edge_count(g, base, m[i], p0, qpos, mt) : edge_count(g, m[i], base, p0, qpos, mt);
+  const int last = z >= 0 ? nm + 1 : nm;
+#pragma unroll 1
+  for (int i = join ? nm : 0; i < last; i++) {
+    const int x = i < nm ? sel(m, i) : z;
+    if (i < nm && (((zmask >> i) & 1) || (g.no_self_loops && x == base))) continue;
+    r -= edge_count(g, out ? base : x, out ? x : base, p0, qpos, mt);
   }
-  if (kk != TM_K_CLOSE) r -= out ? edge_count(g, base, z, p0, qpos, mt) : edge_count(g, z, base, p0, qpos, mt);
-  return (unsigned long long)r;
+  return (unsigned long long)(join ? -r : r);
 }
 
 // ------------------------------------- last two edges on one list (count mode)
@@ -570,10 +539,11 @@ __device__ __forceinline__ unsigned long long tail_frame_term(const tm_graph_vie
   const int base = out ? sel(m, SP::a(md, j)) : sel(m, SP::b(md, j));
   long long kp = K;
   unsigned long long c2 = 0;
-#pragma unroll
-  for (int i = 0; i < MAXN; i++) {
-    if (i >= nm || (g.no_self_loops && m[i] == base)) continue;
-    const long long n = out ? edge_count(g, base, m[i], p, pend, mt) : edge_count(g, m[i], base, p, pend, mt);
+#pragma unroll 1
+  for (int i = 0; i < nm; i++) {
+    const int x = sel(m, i);
+    if (g.no_self_loops && x == base) continue;
+    const long long n = edge_count(g, out ? base : x, out ? x : base, p, pend, mt);
     kp -= n;
     c2 += (unsigned long long)(n * (n - 1) / 2);
   }
@@ -597,7 +567,7 @@ __device__ __forceinline__ unsigned long long tail_same_pair(const tm_graph_view
   if (mt) mt->b += 8;
   const int pos = out ? g.outPos[slot] : g.inPos[slot];
   const int w = out ? g.outNbr[slot] : g.inNbr[slot];
-  return (unsigned long long)(out ? edge_count(g, base, w, pos, pend, mt) : edge_count(g, w, base, pos, pend, mt));
+  return (unsigned long long)edge_count(g, out ? base : w, out ? w : base, pos, pend, mt);
 }
 
 // The last edge k's injectivity term for one mapped node can be decided by
@@ -634,11 +604,11 @@ __device__ __forceinline__ int tail_zero_mask(const tm_graph_view &g, const tm_m
                                               int base, bool out, int p, int pend, Meter *mt = nullptr) {
   const int nm = SP::mapped(md, SP::M(md) - 2);
   int mask = 0;
-#pragma unroll
-  for (int i = 0; i < MAXN; i++) {
-    if (i >= nm) continue;
-    if (g.no_self_loops && m[i] == base) { mask |= 1 << i; continue; }
-    const int n = out ? edge_count(g, base, m[i], p, pend, mt) : edge_count(g, m[i], base, p, pend, mt);
+#pragma unroll 1
+  for (int i = 0; i < nm; i++) {
+    const int x = sel(m, i);
+    if (g.no_self_loops && x == base) { mask |= 1 << i; continue; }
+    const int n = edge_count(g, out ? base : x, out ? x : base, p, pend, mt);
     if (n == 0) mask |= 1 << i;
   }
   return mask;
@@ -657,15 +627,18 @@ __device__ __forceinline__ int tail_frame_mask(const tm_graph_view &g, const tm_
   const int j = M - 2, k = M - 1;
   const int w = SP::mapped(md, j);
   const int kj = SP::kind(md, j), kk = SP::kind(md, k);
+  int bn, out;  // the list's motif node and direction
   if (swapped) {
     if (kj == TM_K_CLOSE || tail2_mode<SP>(md) != T2_INDEP) return 0;
-    const bool out = kj == TM_K_NEW_DST;
-    return tail_zero_mask<SP>(g, md, m, out ? sel(m, SP::a(md, j)) : sel(m, SP::b(md, j)), out, p, pend, mt);
+    out = kj == TM_K_NEW_DST;
+    bn = out ? SP::a(md, j) : SP::b(md, j);
+  } else {
+    if (kk == TM_K_CLOSE) return 0;
+    out = kk == TM_K_NEW_DST;
+    bn = out ? SP::a(md, k) : SP::b(md, k);
+    if (kj != TM_K_CLOSE && bn == w) return 0;  // the list node is edge j's new node: differs per leaf
   }
-  if (kk == TM_K_CLOSE) return 0;
-  const int bn = kk == TM_K_NEW_DST ? SP::a(md, k) : SP::b(md, k);
-  if (kj != TM_K_CLOSE && bn == w) return 0;  // the list node is edge j's new node: differs per leaf
-  return tail_zero_mask<SP>(g, md, m, sel(m, bn), kk == TM_K_NEW_DST, p, pend, mt);
+  return tail_zero_mask<SP>(g, md, m, sel(m, bn), out != 0, p, pend, mt);
 }
 
 // ----------------------------- repeated edges of one graph pair (count mode)
@@ -936,6 +909,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
       __syncthreads();
       continue;
     }
+    // One partial match per lane to expand: motif edge j matched at pos (valid
+    // lanes), from the root dispatch (j = 0), the dealt candidates or the
+    // buffered survivors; the expansion itself is in the code once.
+    int j = 0, pos = 0, ridx = 0, pend = 0, tl = 0, zmk = 0, skipx = -1;
+    bool valid = false;
+    unsigned long long wi = 1;
+    int m[MAXN];
+    int e[ENUM ? MAXE : 1];
+#pragma unroll
+    for (int i = 0; i < MAXN; i++) m[i] = 0;
     if (top == 0 && sbn == 0) {
       // ---------------------------------------------------- root dispatch
       // The launch's roots form one space of 256-root blocks, query after
@@ -1033,133 +1016,52 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
       bool gvalid = false;
       if (pass || (INSTR == 1 && inq)) {
         if (mt) meter.b += 12;
-        const tm_edge e = g.Eg[r];
-        u = e.u; v = e.v; t = e.t;
+        const tm_edge ed = g.Eg[r];
+        u = ed.u; v = ed.v; t = ed.t;
         gvalid = u != v;
       }
-      bool ok = pass;
-      int m[MAXN];
-#pragma unroll
-      for (int i = 0; i < MAXN; i++) m[i] = 0;
+      valid = pass;
+      pos = r;
+      ridx = lane;
       m[0] = u; m[1] = v;
-      CandList L{g.outPos, g.outNbr, 0, 0, 0};
-      const long long tl = (long long)t + q.delta;
-      int tli = tl > 0x7fffffffll ? 0x7fffffff : (int)tl;
-      if (ok) {
-        L = cand_start<SP>(g, md, 1, m, r, mt);
-        if (mt && L.lo < L.hi) meter.b += 8;
-        ok = L.lo < L.hi && (long long)g.T[L.pos[L.lo]] <= tl;
-      }
-      int pend = 0;
+      const long long tll = (long long)t + q.delta;
+      tl = tll > 0x7fffffffll ? 0x7fffffff : (int)tll;
       if constexpr (INSTR == 1) {
         if (gvalid) {
-          const int pe = pend_of(g, tl);
+          const int pe = pend_of(g, tll);
           (SP::kind(md, 1) == TM_K_CLOSE ? rx2 : rx1) += 1;
           rp += ref_probes<SP>(g, md, 1, m, r, pe);
         }
       }
-      if (ok) {
-        pend = pend_of(g, tl, mt);
-        if (INSTR != 1) ok = (pend - r - 1) >= (M - 1);
+      if (valid) {
+        pend = pend_of(g, tll, mt);
+        if (INSTR != 1) valid = (pend - r - 1) >= (M - 1);
       }
       // (counting) the last motif edge closes the root's own two nodes: every
       // edge of a match lies at or before that pair's last edge in the
       // window, so the root's window ends there (positions and pruning time)
-      if (T2 && ok && M >= 3 && SP::kind(md, M - 1) == TM_K_CLOSE && SP::a(md, M - 1) < 2 &&
+      if (T2 && valid && M >= 3 && SP::kind(md, M - 1) == TM_K_CLOSE && SP::a(md, M - 1) < 2 &&
           SP::b(md, M - 1) < 2) {
         const int x = SP::a(md, M - 1) == 0 ? u : v, y = SP::b(md, M - 1) == 0 ? u : v;
         const int pl = pair_last(g, x, y, r, pend, mt);
         if (pl < 0) {
-          ok = false;
+          valid = false;
         } else {
           pend = pl + 1;
           if (mt) meter.b += 4;
-          tli = g.T[pl];
-          ok = (pend - r - 1) >= (M - 1);
+          tl = g.T[pl];
+          valid = (pend - r - 1) >= (M - 1);
         }
       }
-      const int last = ENUM ? M - 1 : M - 2;  // last motif edge handled per candidate
-      if (last == 0) {
-        // count mode, M == 2: edge 1 is the final edge
-        if (ok) { cnt += leaf_count<SP>(g, md, 1, m, L, r, pend, args.scan_max, -1, 0, mt); st_leaves++; }
-        continue;
-      }
-      int cb = 0, ce = 0, dir = L.dir;
-      if (ok) {
-        cb = L.lo;
-        ce = gallop_lb(L.pos, L.lo, L.hi, pend, mt);
-        ok = ce > cb;
-      }
-      // root-pair rewrite: edge 1 repeats the root's pair; expand edge 2 once
-      // from the first parallel edge, its candidates weighted by their rank
-      // among the parallel edges [a1lo, a1hi) of the window
-      int lvl0 = 0, rw = 0, p0f = r, a1lo = 0, a1hi = 0;
-      if (T2 && ok && root_pair_ok<SP>(md)) {
-        a1lo = cb;
-        a1hi = ce;
-        if (mt) meter.b += 4;
-        const int p1 = L.pos[cb];
-        const CandList L2 = cand_start<SP>(g, md, 2, m, p1, mt);
-        cb = L2.lo;
-        dir = L2.dir;
-        ce = gallop_lb(L2.pos, L2.lo, L2.hi, pend, mt);
-        ok = ce > cb;
-        lvl0 = 1;
-        rw = LV_RW;
-        p0f = p1;
-      }
-      // two-edge tail of a 3-edge motif: edge 1 is the second-to-last edge
-      int swp = 0, t2lo = 0, t2hi = 0;
-      const int pat = (T2 && M == 3) ? tail_pattern<SP>(md) : TP_NONE;
-      if (T2 && M == 3 && ok && pat != TP_NONE) {
-        cnt += tail_frame_term<SP>(g, md, pat, m, ce - cb, r, pend, mt);
-        st_leaves++;
-        if (pat == TP_SAME) ok = false; else swp = LV_PAT;
-      } else if (T2 && M == 3 && ok && ce - cb >= args.t2_min && tail2_ok<SP>(md)) {
-        int blo, bhi, bdir;
-        if (mt) meter.b += 4;
-        tail2_range<SP>(g, md, m, L.pos[cb], pend, &blo, &bhi, &bdir, mt);
-        if (2 * (bhi - blo) < ce - cb) {
-          swp = LV_SWAP | (bdir ? LV_BDIR : 0);
-          t2lo = cb; t2hi = ce;
-          cb = blo; ce = bhi;
-          ok = ce > cb;
-        }
-      }
-      int zm = 0;  // injectivity terms known to be 0 in this frame's window
-      if (T2 && M == 3 && ok && !(swp & LV_PAT)) zm = tail_frame_mask<SP>(g, md, m, (swp & LV_SWAP) != 0, ce - cb, r, pend, mt);
-      unsigned long long bm = __ballot(ok);
-      int n = __popcll(bm);
-      if (top + n > FR) { if (lane == 0) atomicOr(&sched->error, 1); break; }
-      if (ok) {
-        r_pend[lane] = pend;  // the window of this lane's root (no frame of an older root is left)
-        r_tl[lane] = tli;
-        int w = top + __popcll(bm & lt_mask);
-        f_cur[w] = cb; f_end[w] = ce; f_lvl[w] = lvl0 | (dir << 8) | swp | rw | (lane << 16) | (zm << 24);
-        if (T2 && (swp & LV_SWAP)) { sw_lo[w & (WAVE - 1)] = t2lo; sw_hi[w & (WAVE - 1)] = t2hi; }
-        if (T2) {
-          f_w[w] = 1;
-          f_p0[w] = p0f;
-          r_alo[lane] = a1lo;
-          r_ahi[lane] = a1hi;
-        }
-#pragma unroll
-        for (int i = 0; i < MAXN; i++) f_m[i * FR + w] = m[i];
-        if constexpr (ENUM) f_e[w] = r;
-      }
-      top += n;
       task_t0 = (long long)wall_clock64();
-      __syncthreads();
-      continue;
-    }
-
+    } else {
     // ------------------------------------------------------ expansion step
     const tm_query_dev &q = args.queries[qcur];
     const tm_motif_dev &md = q.m;
     const int M = SP::M(md);
     const int last = ENUM ? M - 1 : M - 2;  // last motif edge handled per candidate
     const int Ltop = top > 0 ? uni(f_lvl[top - 1] & 0xff) : -1;
-    bool flush = COMPACT && sbn > 0 && (top == 0 || Ltop != sb_level || sbn >= args.sb_flush);
+    const bool flush = COMPACT && sbn > 0 && (top == 0 || Ltop != sb_level || sbn >= args.sb_flush);
     if (T2 && !flush && top > 0) {
       // a pattern frame of 64 slots or more on top: the wave sweeps its slots
       // 64 at a time (one coalesced load of next same-pair times each; the
@@ -1185,7 +1087,35 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         continue;
       }
     }
-    if (!flush) {
+    if (flush) {
+      // ---- the buffered survivors, one per lane: the long chains of
+      // dependent loads (candidate list of the next edge, window end, leaf
+      // counts) run with every lane busy instead of once per filter step
+      j = sb_level + 1;
+      valid = lane < sbn;
+      if (valid) {
+        pos = sb_pos[lane];
+        ridx = sb_ridx[lane] & 0xff;
+        zmk = (sb_ridx[lane] >> 8) & 0xff;
+        wi = ((unsigned long long)(unsigned)sb_wh[lane] << 32) | (unsigned)sb_wl[lane];
+        pend = r_pend[ridx];
+        tl = r_tl[ridx];
+#pragma unroll
+        for (int i = 0; i < MAXN; i++) m[i] = sb_m[i * WAVE + lane];
+        if (j == M - 2) {
+          const int cr = tail_crule<SP>(md);
+          if (cr >= 0) {
+            if (mt) meter.b += 4;
+            const int rule = cr & 0xff;  // uniform: a branch, not an indexed pointer table
+            const int tn = rule == TM_T_PAIR_SELF ? g.tfirst[TM_T_PAIR_SELF][pos] : g.tfirst[TM_T_RECIP][pos];
+            if (tn > tl) skipx = sel(m, cr >> 8);
+          }
+        }
+      }
+      st_steps++;
+      sbn = 0;
+      __syncthreads();
+    } else {
     // ---- deal the next candidate slots of the topmost frames of one level
     // to the lanes (at most lim: room left in the survivor buffer)
     const int L = Ltop;
@@ -1224,12 +1154,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     const int myf = top - 1 - rank;
     st_steps++;
     st_items += total;
-    int slot = 0, pend = 0, dir = 0, tl = 0, ridx = 0, lvw = 0;
+    int slot = 0, dir = 0, lvw = 0;
     unsigned fw = 1;  // the frame's weight (counting)
-    int m[MAXN];
-    int e[ENUM ? MAXE : 1];
-#pragma unroll
-    for (int i = 0; i < MAXN; i++) m[i] = 0;
     if (has) {
       slot = f_cur[myf] + off;
       const int lv = f_lvl[myf];
@@ -1251,7 +1177,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     if (part && take < fcnt) f_cur[fi] += take;
     int ntop = top - nparts + (last_partial ? 1 : 0);
 
-    const int j = L + 1;  // motif edge of the candidates
+    j = L + 1;  // motif edge of the candidates
     const int kind = SP::kind(md, j);
     const int tmn = (j + 1 < M) ? SP::tmode(md, j + 1) : -1;  // pruning rule of edge j + 1
     // a swapped frame (two-edge tail): the slot is a candidate of the last
@@ -1271,8 +1197,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
       cnt += tail_pattern<SP>(md) == TP_STAR ? 0ull - sp : sp;
       st_leaves++;
     }
-    bool valid = false;
-    int pos = 0, tfn = 0, node = -1;
+    int tfn = 0, node = -1;
     // position, neighbour and the next edge's first-candidate time: three
     // loads at the same slot of one list, issued together
     const int lst = kind == TM_K_NEW_DST ? TM_L_OUT
@@ -1310,7 +1235,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     }
     // this candidate's weight: the frame's, times its rank among the root's
     // parallel edges (root-pair rewrite) or its offset in the pair list (pair tail)
-    unsigned long long wi = fw;
+    wi = fw;
     if (T2 && valid && (lvw & LV_RW)) {
       const int rk = lower_bound_i(g.outPairPos, r_alo[ridx], r_ahi[ridx], pos, mt) - r_alo[ridx];
       wi = (unsigned long long)rk;
@@ -1331,7 +1256,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         if (surv) {
           const int w = sbn + __popcll(bm & lt_mask);
           sb_pos[w] = pos;
-          sb_ridx[w] = ridx;
+          sb_ridx[w] = ridx | (((lvw >> 24) & 0xff) << 8);
           sb_wl[w] = (int)(unsigned)(wi & 0xffffffffull);
           sb_wh[w] = (int)(unsigned)(wi >> 32);
 #pragma unroll
@@ -1339,20 +1264,43 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         }
         sbn += ns;
         sb_level = L;
-        top = ntop;
-        __syncthreads();
-        flush = sbn > 0 && (level_done || sbn >= args.sb_flush);
       }
     }
-    if (!buffer) {
+    top = ntop;
+    if (buffer) {  // (expanded once sb_flush are held or the level is done)
+      __syncthreads();
+      continue;
+    }
     if constexpr (INSTR == 1) {
       if (valid && j + 1 < M) {
         (SP::kind(md, j + 1) == TM_K_CLOSE ? rx2 : rx1) += 1;
         rp += ref_probes<SP>(g, md, j + 1, m, pos, pend);
       }
     }
-    if (j == last) {
-      if constexpr (ENUM) {
+    valid = valid && (tmn < 0 || tfn <= tl);
+    zmk = (lvw >> 24) & 0xff;
+    if (T2 && valid && j == M - 2) {
+      const int cr = tail_crule<SP>(md);
+      if (cr >= 0) {
+        if (mt) meter.b += 4;
+        if (g.stf[(size_t)(lst * TM_NTFIRST + (cr & 0xff)) * (size_t)g.E + slot] > tl) skipx = sel(m, cr >> 8);
+      }
+    }
+    }  // deal and filter
+    }
+    // ---------------------------------------------- expand the matches at edge j
+    // One copy of these searches serves the roots, the dealt candidates and
+    // the buffered survivors, and the correction loops are not unrolled: with
+    // a copy per caller and per mapped node a variant had 390 KB of code
+    // against a 64 KB instruction cache shared by two CUs, now 44 KB (4-node
+    // count variant; 4-cycle on 8M hub edges 58.1 -> 52.4 ms, all 3-edge
+    // motifs on 100k edges 93.9 -> 86.4 ms).
+    const tm_query_dev &q = args.queries[qcur];
+    const tm_motif_dev &md = q.m;
+    const int M = SP::M(md);
+    const int last = ENUM ? M - 1 : M - 2;  // last motif edge handled per candidate
+    if constexpr (ENUM) {
+      if (j == last) {
         if (valid) {
           unsigned long long w = atomicAdd(q.count, 1ull);
           if ((long long)w < q.cap) {
@@ -1364,44 +1312,62 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
           }
           if ((long long)w + 1 >= q.cap) __hip_atomic_store(q.stop, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-      } else {
-        if (valid && (tmn < 0 || tfn <= tl)) {
-          const CandList LL = cand_start<SP>(g, md, j + 1, m, pos, mt);
-          int skipx = -1;
-          const int cr = T2 ? tail_crule<SP>(md) : -1;
-          if (cr >= 0) {
-            if (mt) meter.b += 4;
-            if (g.stf[(size_t)(lst * TM_NTFIRST + (cr & 0xff)) * (size_t)g.E + slot] > tl) skipx = sel(m, cr >> 8);
-          }
-          cnt += wi * leaf_count<SP>(g, md, j + 1, m, LL, pos, pend, args.scan_max, skipx, (lvw >> 24) & 0xff, mt);
-          st_leaves++;
-        }
+        __syncthreads();
+        continue;
       }
-      top = ntop;
-      __syncthreads();
-      continue;
     }
-    int cb = 0, ce = 0, cdir = 0;
-    int swc = 0, t2lo = 0, t2hi = 0, zm = 0;
-    if (valid && tmn >= 0) valid = tfn <= tl;
+    int cb = 0, ce = 0, cdir = 0, lvl = j, rw = 0, a1lo = 0, a1hi = 0, p0f = pos;
     if (valid) {
       const CandList LL = cand_start<SP>(g, md, j + 1, m, pos, mt);
       cb = LL.lo;
-      cdir = LL.dir;
-      ce = gallop_lb(LL.pos, LL.lo, LL.hi, pend, mt);
+      if (!ENUM && j == last) {
+        // count mode: the last motif edge's matches by range arithmetic
+        cnt += wi * leaf_count<SP>(g, md, j + 1, m, LL, pos, pend, args.scan_max, skipx, zmk, mt);
+        st_leaves++;
+      } else {
+        cdir = LL.dir;
+        ce = gallop_lb(LL.pos, LL.lo, LL.hi, pend, mt);
+      }
       valid = ce > cb;
-      const int pat = (T2 && j == M - 3) ? tail_pattern<SP>(md) : TP_NONE;
-      if (T2 && valid && j == M - 3 && j == pair_tail_edge<SP>(md)) {
+    }
+    if (!ENUM && j == last) {
+      __syncthreads();
+      continue;
+    }
+    // root-pair rewrite: edge 1 repeats the root's pair; expand edge 2 once
+    // from the first parallel edge, its candidates weighted by their rank
+    // among the parallel edges [a1lo, a1hi) of the window
+    if (T2 && j == 0 && root_pair_ok<SP>(md)) {
+      lvl = 1;
+      rw = LV_RW;
+      if (valid) {
+        a1lo = cb;
+        a1hi = ce;
+        if (mt) meter.b += 4;
+        p0f = g.outPairPos[cb];
+        const CandList L2 = cand_start<SP>(g, md, 2, m, p0f, mt);
+        cb = L2.lo;
+        cdir = L2.dir;
+        ce = gallop_lb(L2.pos, L2.lo, L2.hi, pend, mt);
+        valid = ce > cb;
+      }
+    }
+    int swc = 0, t2lo = 0, t2hi = 0, zm = 0;
+    if (T2 && valid && j == M - 3) {
+      const int pat = tail_pattern<SP>(md);
+      if (j > 0 && j == pair_tail_edge<SP>(md)) {
         swc = LV_R1;  // pair tail: the pair list after this first edge, weighted by offset
         t2lo = cb;
-      } else if (T2 && valid && j == M - 3 && pat != TP_NONE) {
+      } else if (pat != TP_NONE) {
         cnt += wi * tail_frame_term<SP>(g, md, pat, m, ce - cb, pos, pend, mt);
         st_leaves++;
         if (pat == TP_SAME) valid = false; else swc = LV_PAT;
-      } else if (T2 && valid && j == M - 3 && ce - cb >= args.t2_min && tail2_ok<SP>(md)) {
+      } else if (ce - cb >= args.t2_min && tail2_ok<SP>(md)) {
         int blo, bhi, bdir;
         if (mt) meter.b += 4;
-        tail2_range<SP>(g, md, m, LL.pos[cb], pend, &blo, &bhi, &bdir, mt);
+        const int kn = SP::kind(md, j + 1);
+        const int *ap = kn == TM_K_NEW_DST ? g.outPos : (kn == TM_K_NEW_SRC ? g.inPos : (cdir ? g.inPairPos : g.outPairPos));
+        tail2_range<SP>(g, md, m, ap[cb], pend, &blo, &bhi, &bdir, mt);
         if (2 * (bhi - blo) < ce - cb) {
           swc = LV_SWAP | (bdir ? LV_BDIR : 0);
           t2lo = cb; t2hi = ce;
@@ -1409,121 +1375,42 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
           valid = ce > cb;
         }
       }
-      if (T2 && valid && j == M - 3 && !(swc & LV_PAT))
+      if (valid && !(swc & LV_PAT))
         zm = tail_frame_mask<SP>(g, md, m, (swc & LV_SWAP) != 0, ce - cb, pos, pend, mt);
     }
-    const unsigned long long bm = __ballot(valid);
-    const int n = __popcll(bm);
-    if (ntop + n > FR) { if (lane == 0) atomicOr(&sched->error, 1); break; }
-    if (valid) {
-      int w = ntop + __popcll(bm & lt_mask);
-      f_cur[w] = cb; f_end[w] = ce; f_lvl[w] = j | (cdir << 8) | swc | (ridx << 16) | (zm << 24);
-      if (T2 && (swc & (LV_SWAP | LV_R1))) { sw_lo[w & (WAVE - 1)] = t2lo; sw_hi[w & (WAVE - 1)] = t2hi; }
-      if (T2) {
-        f_w[w] = (int)(unsigned)wi;
-        f_p0[w] = pos;
-      }
-#pragma unroll
-      for (int i = 0; i < MAXN; i++) f_m[i * FR + w] = m[i];
-      if constexpr (ENUM) {
-#pragma unroll
-        for (int i = 0; i < MAXE; i++)
-          if (i < j) f_e[i * FR + w] = e[i];
-        f_e[j * FR + w] = pos;
-      }
-    }
-    st_push += n;
-    top = ntop + n;
-    __syncthreads();
-    }  // expanded in this step
-    }  // deal and filter
-    if (flush) {
-      // ---- expand the buffered survivors, one per lane: the long chains of
-      // dependent loads (candidate list of the next edge, window end, leaf
-      // counts) run with every lane busy instead of once per filter step
-      const int j = sb_level + 1;  // motif edge of the buffered candidates
-      const bool has = lane < sbn;
-      int pos = 0, ridx = 0, pend = 0;
-      unsigned long long wi = 1;
-      int m[MAXN];
-#pragma unroll
-      for (int i = 0; i < MAXN; i++) m[i] = 0;
-      if (has) {
-        pos = sb_pos[lane];
-        ridx = sb_ridx[lane];
-        wi = ((unsigned long long)(unsigned)sb_wh[lane] << 32) | (unsigned)sb_wl[lane];
-        pend = r_pend[ridx];
-#pragma unroll
-        for (int i = 0; i < MAXN; i++) m[i] = sb_m[i * WAVE + lane];
-      }
-      st_steps++;
-      sbn = 0;
-      if (j == last) {
-        if (has) {
-          const CandList LL = cand_start<SP>(g, md, j + 1, m, pos, mt);
-          int skipx = -1;
-          const int cr = tail_crule<SP>(md);
-          if (cr >= 0) {
-            if (mt) meter.b += 4;
-            const int rule = cr & 0xff;  // uniform: a branch, not an indexed pointer table
-            const int tn = rule == TM_T_PAIR_SELF ? g.tfirst[TM_T_PAIR_SELF][pos] : g.tfirst[TM_T_RECIP][pos];
-            if (tn > r_tl[ridx]) skipx = sel(m, cr >> 8);
-          }
-          cnt += wi * leaf_count<SP>(g, md, j + 1, m, LL, pos, pend, args.scan_max, skipx, 0, mt);
-          st_leaves++;
-        }
-        __syncthreads();
-        continue;
-      }
-      int cb = 0, ce = 0, cdir = 0;
-      int swc = 0, t2lo = 0, t2hi = 0, zm = 0;
-      bool valid = has;
-      if (valid) {
-        const CandList LL = cand_start<SP>(g, md, j + 1, m, pos, mt);
-        cb = LL.lo;
-        cdir = LL.dir;
-        ce = gallop_lb(LL.pos, LL.lo, LL.hi, pend, mt);
-        valid = ce > cb;
-        const int pat = (T2 && j == M - 3) ? tail_pattern<SP>(md) : TP_NONE;
-        if (T2 && valid && j == M - 3 && j == pair_tail_edge<SP>(md)) {
-          swc = LV_R1;
-          t2lo = cb;
-        } else if (T2 && valid && j == M - 3 && pat != TP_NONE) {
-          cnt += wi * tail_frame_term<SP>(g, md, pat, m, ce - cb, pos, pend, mt);
-          st_leaves++;
-          if (pat == TP_SAME) valid = false; else swc = LV_PAT;
-        } else if (T2 && valid && j == M - 3 && ce - cb >= args.t2_min && tail2_ok<SP>(md)) {
-          int blo, bhi, bdir;
-          if (mt) meter.b += 4;
-          tail2_range<SP>(g, md, m, LL.pos[cb], pend, &blo, &bhi, &bdir, mt);
-          if (2 * (bhi - blo) < ce - cb) {
-            swc = LV_SWAP | (bdir ? LV_BDIR : 0);
-            t2lo = cb; t2hi = ce;
-            cb = blo; ce = bhi;
-            valid = ce > cb;
-          }
-        }
-        if (T2 && valid && j == M - 3 && !(swc & LV_PAT))
-          zm = tail_frame_mask<SP>(g, md, m, (swc & LV_SWAP) != 0, ce - cb, pos, pend, mt);
-      }
+    {
       const unsigned long long bm = __ballot(valid);
       const int n = __popcll(bm);
       if (top + n > FR) { if (lane == 0) atomicOr(&sched->error, 1); break; }
       if (valid) {
         const int w = top + __popcll(bm & lt_mask);
-        f_cur[w] = cb; f_end[w] = ce; f_lvl[w] = j | (cdir << 8) | swc | (ridx << 16) | (zm << 24);
+        f_cur[w] = cb; f_end[w] = ce; f_lvl[w] = lvl | (cdir << 8) | swc | rw | (ridx << 16) | (zm << 24);
         if (T2 && (swc & (LV_SWAP | LV_R1))) { sw_lo[w & (WAVE - 1)] = t2lo; sw_hi[w & (WAVE - 1)] = t2hi; }
         if (T2) {
           f_w[w] = (int)(unsigned)wi;
-          f_p0[w] = pos;
+          f_p0[w] = p0f;
         }
 #pragma unroll
         for (int i = 0; i < MAXN; i++) f_m[i * FR + w] = m[i];
+        if (j == 0) {  // the window of this lane's root (no frame of an older root is left)
+          r_pend[lane] = pend;
+          r_tl[lane] = tl;
+          if (T2) {
+            r_alo[lane] = a1lo;
+            r_ahi[lane] = a1hi;
+          }
+        }
+        if constexpr (ENUM) {
+#pragma unroll
+          for (int i = 0; i < MAXE; i++)
+            if (i < j) f_e[i * FR + w] = e[i];
+          f_e[j * FR + w] = pos;
+        }
       }
-      st_push += n;
+      if (j > 0) st_push += n;
       top += n;
       __syncthreads();
-    }  // flush
+    }
     // ---------------------------------------------- donate to idle wavefronts
     // every steal_every steps; only a wavefront that has held its current
     // task for steal_after_ticks donates: short tasks never pay for the exchange
