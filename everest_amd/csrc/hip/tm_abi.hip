@@ -211,13 +211,15 @@ __global__ void error_kernel(const tm_sched *s, int *out) {
 
 __global__ void reset_kernel(tm_sched *s, unsigned long long *counts, int *stops, int n, int grid) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < TM_STRIPES) st_dev(&s->next_chunk[i][0], 0ull);
+  if (i < TM_STRIPES) {
+    st_dev(&s->stripe[i].next, 0);
+    st_dev(&s->stripe[i].busy, (grid + TM_STRIPES - 1 - i) / TM_STRIPES);  // every wavefront starts out holding (root) work
+  }
   if (i == 0) {
     st_dev(&s->error, 0);
     st_dev(&s->abort, 0);
     st_dev(&s->pool_head, 0u);
     st_dev(&s->pool_tail, 0u);
-    st_dev(&s->busy, grid);  // every wavefront starts out holding (root) work
     st_dev(&s->waiters, 0);
     // fresh ring tags for this launch (the host clears the ring before 2^18)
     __hip_atomic_fetch_add(&s->gen, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -521,7 +523,13 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
   if (wpc < 1) wpc = 1;
   int grid = std::min(g->num_cus * wpc, s.wstats_cap);
 
-  long long total_blocks = 0, max_blocks = 0;
+  // Roots per dispatch block: about 4 blocks per wavefront, so that a small
+  // graph's roots reach every wavefront and a large one's are read 1024 at a
+  // time (100k edges, the 36 3-edge motifs: 86.4 ms with 256-root blocks in
+  // claims of 4, which 98 wavefronts took, 7.9 ms with 16-root blocks).
+  int unit_shift = 4;
+  while (unit_shift < 10 && (span >> (unit_shift + 1)) >= 4ll * grid) unit_shift++;
+  long long total_blocks = 0;
   for (int i = 0; i < nq; i++) {
     const tm_query_dev &qd = s.h_queries[q0 + i];
     int *qt = &s.h_qtab[4 * (size_t)(q0 + i)];
@@ -535,22 +543,14 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
     qt[3] = qd.m.tmode[1] | (instr == 1 ? 0 : qd.m.xmask[0] << TM_QT_XRULE_SHIFT);
     s.h_prefix[q0 + i] = total_blocks;
     if (re > rb) {
-      const long long nb = (re - (rb & ~3) + 255) / 256;
-      total_blocks += nb;
-      max_blocks = std::max(max_blocks, nb);
+      total_blocks += ((long long)re - (rb & ~3) + (1 << unit_shift) - 1) >> unit_shift;
     }
   }
   s.h_prefix[q0 + nq] = total_blocks;
   if (total_blocks < grid) grid = (int)std::max<long long>(1, total_blocks);
-  // claims of about 1/8 of one query's roots per wavefront: as fine-grained
-  // as a launch of that query alone, whatever the number of queries
-  int claim_blocks;
-  if (tune && tune->claim_blocks > 0) {
-    claim_blocks = tune->claim_blocks;
-  } else {
-    const long long c = (max_blocks + (long long)grid * 8 - 1) / ((long long)grid * 8);
-    claim_blocks = (int)std::min<long long>(std::max<long long>(c, 4), 64);
-  }
+  // a caller's claim size counts 256 roots; the library's own shrinks with the blocks left
+  const int claim_blocks =
+      (tune && tune->claim_blocks > 0) ? std::max(1, (int)(((long long)tune->claim_blocks << 8) >> unit_shift)) : 0;
 
   HIPTRY(hipMemcpyAsync(s.d_queries + q0, s.h_queries.data() + q0, sizeof(tm_query_dev) * nq,
                         hipMemcpyHostToDevice, sl.stream));
@@ -570,6 +570,7 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
   a.block_prefix = s.d_prefix + q0;
   a.nq = nq;
   a.total_blocks = total_blocks;
+  a.unit_shift = unit_shift;
   a.claim_blocks = claim_blocks;
   a.frames = frames;
   a.sb_flush = sb_flush;
@@ -586,6 +587,7 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
   a.steal_every = (tune && tune->steal_every > 0) ? tune->steal_every : 16;
   a.steal_max = (tune && tune->steal_max > 0) ? tune->steal_max : 4;
   a.idle_cap = std::max(64, g->num_cus / 2);
+  a.scouts = a.idle_cap / TM_STRIPES;
   a.steal_min = (tune && tune->steal_min > 0) ? tune->steal_min : 64;
   {
     const long long us = (tune && tune->steal_after_us > 0) ? tune->steal_after_us : 1000;

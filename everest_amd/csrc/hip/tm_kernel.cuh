@@ -27,7 +27,8 @@
 namespace tmk {
 
 constexpr int WAVE = 64;
-constexpr int TM_BLOCK = 4 * WAVE;  // roots per dispatch block (4 per lane)
+constexpr int TM_ROW = 4 * WAVE;    // roots of one 16-byte load per lane
+constexpr int TM_ROWS = 4;          // most rows of a dispatch block (1024 roots)
 constexpr int TM_ROOTS = WAVE + 1;  // window table entries: one per lane's root, one for a taken frame
 
 // ------------------------------------------------------------------ helpers
@@ -86,19 +87,6 @@ __device__ __forceinline__ bool in_first(const int (&r)[MAXN], int n, int node) 
 #pragma unroll
   for (int i = 0; i < MAXN; i++) hit |= (i < n) && (r[i] == node);
   return hit;
-}
-
-// component i (uniform) of a register quadruple, kept in registers
-__device__ __forceinline__ unsigned pick4(uint4 v, int i) {
-  const unsigned a = (unsigned)opaque((int)v.x), b = (unsigned)opaque((int)v.y);
-  const unsigned c = (unsigned)opaque((int)v.z), d = (unsigned)opaque((int)v.w);
-  return i == 0 ? a : (i == 1 ? b : (i == 2 ? c : d));
-}
-
-__device__ __forceinline__ unsigned wave_min_u32(unsigned x) {
-#pragma unroll
-  for (int o = WAVE / 2; o > 0; o >>= 1) x = min(x, (unsigned)__shfl_xor((int)x, o));
-  return x;
 }
 
 __device__ __forceinline__ int wave_incl_scan(int x, int lane) {
@@ -774,17 +762,23 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
   unsigned iter = 0;
   int qcur = -1;
   int top = 0;
-  long long claim_next = 0, claim_end = 0;  // blocks of the current claim not yet started
-  long long qb0 = 0, qb1 = 0;               // blocks of the current query
-  int blk = -1;            // first root of the block being dispatched (-1: none)
-  int quarter = 0;         // quarter of the block: this lane's root is blk + 4 lane + quarter
+  // (a launch has at most 2^30 blocks: blocks of fewer than 1024 roots are only
+  // taken while there are few)
+  int claim_next = 0, claim_end = 0;        // blocks of the current claim not yet started
+  int qb0 = 0, qb1 = 0;                     // blocks of the current query
+  int ublk = -1;           // first root of the block being dispatched (-1: none)
+  unsigned umask = 0;      // this lane's roots of the block still to expand: bit 4 k + i is root
+                           // ublk + 256 k + 4 lane + i
+  unsigned upass = 0;      // (INSTR == 1) those of them whose gaps pass
+  bool first_claim = true; // the wavefront's own first claim is not taken yet
   int cq = 0;              // query of the current chunk, and its table entry:
   int cdelta = 0, cbeg = 0, cend = 0, crule = 0;
   int cxmask = 0;          // the root's further gap rules (later edges at the root's nodes), bit per rule
-  uint4 bgap = make_uint4(0u, 0u, 0u, 0u);  // gaps of this lane's 4 roots of the block
   bool roots_done = false; // the root chunks of every query are handed out
   const int home_stripe = blockIdx.x & (TM_STRIPES - 1);
-  int stripe_off = 0;
+  int cstripe = home_stripe;  // the stripe that counts this wavefront's busy credit
+  int at_stripe = home_stripe;  // the stripe it claims from
+  bool scout = false;           // looks at the other stripes and may wait for donations
   long long task_t0 = 0;   // wall clock when the current task (root group or donated frame) began
   bool is_idle = false;    // gave up its busy credit (sched->busy starts at the grid size)
   bool waiter = false;     // counted in sched->waiters
@@ -827,9 +821,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
       // wavefronts holding work plus the records reserved and not yet
       // taken (a donor adds one before it reserves; the taker inherits it),
       // so busy == 0 means no work is left anywhere and a waiting
-      // wavefront may leave.
+      // wavefront may leave.  The count is kept per stripe, a credit staying
+      // with its stripe when a record carries it: only a holder of a stripe's
+      // credit adds to that stripe, so a stripe at 0 stays there, and all
+      // stripes read as 0, one after the other, means none is left.  (One
+      // counter for all took 24 ns per leaving wavefront, as same-address
+      // atomics do here: 95 us of every launch of 4,000.)
       if (!is_idle) {
-        if (lane == 0) add_rlx(&sched->busy, -1);
+        if (lane == 0) add_rlx(&sched->stripe[cstripe].busy, -1);
         is_idle = true;
         st_work += (unsigned long long)((long long)wall_clock64() - work_t0);
       }
@@ -839,6 +838,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         // wavefronts of this launch or of a concurrent one that have not
         // started yet always find a CU: waiting wavefronts of one launch can
         // never hold every resource while they wait for its unstarted ones
+        if (!scout) {
+          st_capexit++;
+          break;
+        }
         int w = 0;
         if (lane == 0) w = add_rlx(&sched->waiters, 1);
         if (uni(__shfl(w, 0)) >= args.idle_cap) {
@@ -863,9 +866,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         fv = (int)(unsigned)(word & 0xffffffffull);
         if (__ballot(!mine) == 0ull) { got = true; break; }
         if ((spin & 3u) == 3u) {
-          int b = 0, ab = 0;
+          int ab = 0;
+          const int b = lane < TM_STRIPES ? ld_rlx(&sched->stripe[lane].busy) : 0;
           if (lane == 0) {
-            b = ld_rlx(&sched->busy);
             ab = ld_rlx(&sched->abort);
             if (!ab && args.limit_ticks > 0 && (long long)wall_clock64() - ld_rlx(&sched->t0) > args.limit_ticks) {
               atomicOr(&sched->abort, 1);
@@ -874,7 +877,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
             }
           }
           if (uni(__shfl(ab, 0))) break;
-          if (uni(__shfl(b, 0)) == 0) break;  // every record is taken and nobody holds work
+          if (__ballot(b != 0) == 0ull) break;  // every record is taken and nobody holds work
         }
         __builtin_amdgcn_s_sleep(32);
       }
@@ -888,7 +891,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
       st_take++;
       is_idle = false;  // the record's busy credit is now this wavefront's
       work_t0 = (long long)wall_clock64();
-      const int fq = uni(__shfl(fv, 0));
+      const int fq = uni(__shfl(fv, 0)) & 0xffff;
+      cstripe = uni(__shfl(fv, 0)) >> 16;
       if (fq != qcur) {
         if (!ENUM && qcur >= 0) {
           unsigned long long sm = wave_sum64(cnt);
@@ -921,41 +925,66 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     for (int i = 0; i < MAXN; i++) m[i] = 0;
     if (top == 0 && sbn == 0) {
       // ---------------------------------------------------- root dispatch
-      // The launch's roots form one space of 256-root blocks, query after
-      // query, handed out in fixed claims over striped counters.
-      // In a block, lane l holds roots blk + 4l .. blk + 4l + 3 and their
-      // gaps under the query's start rule (one 16-byte load).  A block none
-      // of whose gaps is within delta is skipped whole; otherwise its four
-      // quarters (one root per lane) are expanded in turn, each only if some
-      // lane's root passes.
+      // The launch's roots form one space of blocks of 16 to 1024 roots
+      // (args.unit_shift), query after query.  Lane l holds roots 4 l .. 4 l + 3
+      // of each 256-root row of a block and reads their gaps under each of the
+      // query's rules with one 16-byte load, all rows of a rule in flight
+      // together; the roots that pass are kept as a bit mask per lane and
+      // expanded 64 at a time in root order, whatever lanes hold them.
       int qsel = -1;
-      bool pass = false, inq = false;
       while (qsel < 0) {
-        if (blk < 0) {
+        if (ublk < 0) {
           if (claim_next >= claim_end) {
-            // striped counters: stripe k hands out blocks [k B / S, (k+1) B / S)
-            // in claims of claim_blocks; a wavefront starts on its own stripe
-            // and moves on when it runs dry
             bool got = false;
-            while (stripe_off < TM_STRIPES) {
-              const int k = (home_stripe + stripe_off) & (TM_STRIPES - 1);
-              const long long sb = args.total_blocks * k / TM_STRIPES;
-              const long long se = args.total_blocks * (k + 1) / TM_STRIPES;
-              const long long n = args.claim_blocks;
-              long long o = 0;
-              if (lane == 0) o = (long long)atomicAdd(&sched->next_chunk[k][0], (unsigned long long)n);
-              o = sb + __shfl(o, 0);
-              if (o < se) {
-                claim_next = o;
-                claim_end = min(o + n, se);
+            while (!got) {
+              // claim `idx` of stripe k's blocks [k B / S, (k + 1) B / S): the
+              // first of each of its wavefronts by their order, the others by
+              // one atomic.  Rounds of one claim per wavefront share half of
+              // the blocks left, down to single blocks; a caller's fixed size
+              // is one round.
+              const int k = at_stripe;
+              const int sb = (int)(args.total_blocks * k / TM_STRIPES);
+              const int size = (int)(args.total_blocks * (k + 1) / TM_STRIPES) - sb;
+              const int own = ((int)gridDim.x + TM_STRIPES - 1 - k) / TM_STRIPES;  // the stripe's wavefronts
+              const int nw = max(1, own);
+              int idx = blockIdx.x / TM_STRIPES;
+              if (!first_claim) {
+                if (lane == 0) idx = own + add_rlx(&sched->stripe[k].next, 1);
+                idx = uni(idx);
+              }
+              first_claim = false;
+              // (idx stays far below the blocks of a fixed size times n: a
+              // dry stripe is tried once per wavefront)
+              int start = 0, n = args.claim_blocks;
+              if (n == 0) {
+                for (;;) {
+                  n = max(1, (int)((unsigned)(size - start) / (unsigned)(2 * nw)));
+                  if (n == 1 || idx < nw) break;
+                  start += nw * n;
+                  idx -= nw;
+                }
+              }
+              const long long at = start + (long long)idx * n;
+              if (at < size) {
+                claim_next = sb + (int)at;
+                claim_end = sb + (int)min(at + n, (long long)size);
                 got = true;
                 break;
               }
-              stripe_off++;
+              // dry.  The stripe's first wavefronts to find it so (by the
+              // claims past its end) go on to the other stripes and then wait
+              // for donations; the rest leave.  If all looked at all stripes,
+              // that alone would hold a launch for 24 ns per wavefront.
+              if (k == home_stripe && !scout) {
+                if ((at - size) / n >= args.scouts) break;
+                scout = true;
+              }
+              at_stripe = (at_stripe + 1) & (TM_STRIPES - 1);
+              if (at_stripe == home_stripe) break;
             }
             if (!got) { roots_done = true; break; }
           }
-          const long long b = claim_next++;
+          const int b = claim_next++;
           if (b < qb0 || b >= qb1) {
             // the block's query: the last q with block_prefix[q] <= b (uniform search)
             int lo = 0, hi = MULTI ? args.nq : 1;
@@ -964,42 +993,84 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
               if (args.block_prefix[mid] <= b) lo = mid; else hi = mid;
             }
             cq = lo;
-            qb0 = args.block_prefix[cq];
-            qb1 = args.block_prefix[cq + 1];
+            qb0 = (int)args.block_prefix[cq];
+            qb1 = (int)args.block_prefix[cq + 1];
             const int4 qt = *(const int4 *)(args.qtab + 4 * cq);
             cdelta = qt.x; cbeg = qt.y; cend = qt.z;
             crule = qt.w & ((1 << TM_QT_XRULE_SHIFT) - 1);
             cxmask = qt.w >> TM_QT_XRULE_SHIFT;
           }
-          blk = (cbeg & ~3) + (int)(b - qb0) * TM_BLOCK;
-          if (ENUM && ld_rlx(args.queries[cq].stop)) { blk = -1; continue; }  // enumeration cap reached
-          const int r0 = blk + 4 * lane;
-          uint4 x = *(const uint4 *)(g.rgap + (size_t)crule * (size_t)g.epad + r0);
-          for (int rr = 0; rr < TM_NTFIRST; rr++) {  // a root passes only if every rule's next edge is in the window
-            if (!((cxmask >> rr) & 1)) continue;
-            const uint4 y = *(const uint4 *)(g.rgap + (size_t)rr * (size_t)g.epad + r0);
-            x.x = max(x.x, y.x); x.y = max(x.y, y.y); x.z = max(x.z, y.z); x.w = max(x.w, y.w);
+          if (ENUM && ld_rlx(args.queries[cq].stop)) { roots_done = true; break; }  // enumeration cap reached
+          const int units = 1 << args.unit_shift;
+          ublk = (cbeg & ~3) + (b - qb0) * units;
+          // this lane's roots of the block inside the query's range
+          unsigned in = 0;
+#pragma unroll
+          for (int k = 0; k < TM_ROWS; k++) {
+            const int r0 = ublk + TM_ROW * k + 4 * lane;
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+              if (r0 + i >= cbeg && r0 + i < cend) in |= 1u << (4 * k + i);
           }
-          if (r0 < cbeg || r0 >= cend) x.x = ~0u;
-          if (r0 + 1 < cbeg || r0 + 1 >= cend) x.y = ~0u;
-          if (r0 + 2 < cbeg || r0 + 2 >= cend) x.z = ~0u;
-          if (r0 + 3 < cbeg || r0 + 3 >= cend) x.w = ~0u;
-          bgap = x;
-          st_roots += (unsigned)(min(max(cend - blk, 0), TM_BLOCK) - min(max(cbeg - blk, 0), TM_BLOCK));
-          const unsigned mn = min(min(x.x, x.y), min(x.z, x.w));
-          const bool near = cdelta >= 0 && mn <= (unsigned)cdelta;
-          if (mt) meter.b += 16 * (1 + __popc((unsigned)cxmask));  // the gap words of this lane's 4 roots
-          if (INSTR != 1 && __ballot(near) == 0ull) { blk = -1; continue; }
-          quarter = -1;
+          in &= (4 * lane < units ? 0xfu : 0u) | (units > TM_ROW ? 0xffffu : 0u);
+          if (units == 2 * TM_ROW) in &= 0xffu;
+          st_roots += (unsigned)(min(max(cend - ublk, 0), units) - min(max(cbeg - ublk, 0), units));
+          // a root passes if under every rule its next edge is in the window:
+          // edge 1's rule, then the others while some root is left
+          umask = in;
+          unsigned rules = (unsigned)cxmask;
+          int rr = crule;
+          for (;;) {
+            uint4 x[TM_ROWS];
+            const unsigned *gap = g.rgap + (size_t)rr * (size_t)g.epad;
+#pragma unroll
+            for (int k = 0; k < TM_ROWS; k++) {
+              // (a row starting before cend <= E ends inside the padded array)
+              x[k] = make_uint4(~0u, ~0u, ~0u, ~0u);
+              if (units > TM_ROW * k && ublk + TM_ROW * k < cend) x[k] = *(const uint4 *)(gap + ublk + TM_ROW * k + 4 * lane);
+            }
+            if (mt) meter.b += 16;
+            unsigned ok = 0;
+#pragma unroll
+            for (int k = 0; k < TM_ROWS; k++) {
+              const unsigned d = (unsigned)cdelta;
+              ok |= ((x[k].x <= d ? 1u : 0u) | (x[k].y <= d ? 2u : 0u) | (x[k].z <= d ? 4u : 0u) | (x[k].w <= d ? 8u : 0u)) << (4 * k);
+            }
+            umask &= ok;
+            if (rules == 0 || __ballot(umask != 0) == 0ull) break;
+            rr = __ffs(rules) - 1;
+            rules &= rules - 1;
+          }
+          if (INSTR == 1) { upass = umask; umask = in; }
         }
-        if (++quarter == 4) { blk = -1; continue; }
-        const int r = blk + 4 * lane + quarter;
-        const unsigned lg = pick4(bgap, quarter);
-        inq = r >= cbeg && r < cend;
-        pass = inq && cdelta >= 0 && lg <= (unsigned)cdelta;
-        if (__ballot(pass) != 0ull || (INSTR == 1 && __ballot(inq) != 0ull)) qsel = cq;
+        if (__ballot(umask != 0) == 0ull) { ublk = -1; continue; }
+        qsel = cq;
       }
       if (qsel < 0) continue;  // every root chunk is handed out
+      // lane l takes the l-th root left in the block
+      const int pc = __popc(umask);
+      const int incl = wave_incl_scan(pc, lane);
+      const int have = uni(__shfl(incl, WAVE - 1));
+      const int taken = min(have, WAVE);
+      int own = 0;  // the lane that holds it: as many as have their roots before it
+#pragma unroll
+      for (int d = WAVE / 2; d > 0; d >>= 1)
+        if (__shfl(incl, own + d - 1) <= lane) own += d;
+      own = min(own, WAVE - 1);
+      unsigned om = (unsigned)__shfl((int)umask, own);
+      const unsigned opass = (unsigned)__shfl((int)upass, own);
+      const int skip = lane - __shfl(incl - pc, own);
+      for (int i = 0; i < skip && lane < taken; i++) om &= om - 1;
+      const int bit = __ffs(om) - 1;
+      const int r = ublk + ((bit >> 2) << 8) + 4 * own + (bit & 3);
+      const bool inq = lane < taken;
+      const bool pass = inq && (INSTR != 1 || ((opass >> bit) & 1));
+      if (have <= WAVE) {
+        ublk = -1;
+      } else {
+        const int mine = min(max(taken - (incl - pc), 0), pc);
+        for (int i = 0; i < mine; i++) umask &= umask - 1;
+      }
       if (qsel != qcur) {
         if (!ENUM && qcur >= 0) {
           unsigned long long sm = wave_sum64(cnt);
@@ -1011,10 +1082,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
       const tm_query_dev &q = args.queries[qcur];
       const tm_motif_dev &md = q.m;
       const int M = SP::M(md);
-      const int r = blk + 4 * lane + quarter;
       int u = 0, v = 0, t = 0;
       bool gvalid = false;
-      if (pass || (INSTR == 1 && inq)) {
+      if (inq) {
         if (mt) meter.b += 12;
         const tm_edge ed = g.Eg[r];
         u = ed.u; v = ed.v; t = ed.t;
@@ -1439,7 +1509,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         unsigned t = 0;
         int ok = 1;
         if (lane == 0) {
-          add_rlx(&sched->busy, 1);  // the record's credit, before it can be seen
+          add_rlx(&sched->stripe[cstripe].busy, 1);  // the record's credit, before it can be seen
           t = atomicAdd(&sched->pool_tail, 1u);
           const unsigned lap = t >> args.pool_shift;
           if (lap > 0) {
@@ -1469,7 +1539,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         unsigned long long *rec = args.pool + (size_t)(t & (unsigned)(args.pool_cap - 1)) * TM_POOL_FIELDS;
         if (lane < TM_POOL_FIELDS) {
           int v = 0;
-          if (lane == 0) v = qcur;
+          if (lane == 0) v = qcur | (cstripe << 16);
           else if (lane == 2) v = mid;
           else {
             int *src = frame_field(lane, b);
@@ -1494,7 +1564,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     for (int q = lane; q < args.nq; q += WAVE)
       if (q_cnt[q]) atomicAdd(args.queries[q].count, q_cnt[q]);
   if (!is_idle) st_work += (unsigned long long)((long long)wall_clock64() - work_t0);
-  if (lane == 0 && !is_idle) add_rlx(&sched->busy, -1);  // left early holding work (error or deadline)
+  if (lane == 0 && !is_idle) add_rlx(&sched->stripe[cstripe].busy, -1);  // left early holding work (error or deadline)
   if (lane == 0 && waiter) add_rlx(&sched->waiters, -1);
   // work counters: plain stores into this wavefront's own slot, summed by a
   // one-block kernel after the launch (no same-address atomics from every wave)

@@ -40,11 +40,11 @@ constexpr size_t kOffWstats = kOffStops + up(sizeof(int) * kMaxQ);
 constexpr size_t kOffPool = kOffWstats + up(sizeof(unsigned long long) * TM_NSTATS * (size_t)kMaxWaves);
 constexpr size_t kOffPoolDone = kOffPool + up(sizeof(unsigned long long) * TM_POOL_FIELDS * ((size_t)1 << kPoolShift));
 constexpr size_t kBytes = kOffPoolDone + up(sizeof(unsigned) * ((size_t)1 << kPoolShift));
-static_assert(kBytes == TM_NOALLOC_SCRATCH_BYTES, "TM_NOALLOC_SCRATCH_BYTES out of date");
+static_assert(kBytes <= TM_NOALLOC_SCRATCH_BYTES && kBytes + 4096 > TM_NOALLOC_SCRATCH_BYTES, "TM_NOALLOC_SCRATCH_BYTES out of date");
 
 // The scratch array: one copy per GPU the library runs on, held until the
 // process ends.
-static __device__ __align__(256) unsigned char scratch[kBytes];
+static __device__ __align__(256) unsigned char scratch[TM_NOALLOC_SCRATCH_BYTES];
 
 __global__ void zero_kernel(unsigned long long *p, size_t n) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;

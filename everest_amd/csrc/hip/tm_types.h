@@ -108,10 +108,15 @@ typedef struct {
   int *stop;                  // set once cap rows are claimed: no more roots of this query
 } tm_query_dev;
 
-#define TM_STRIPES 8  // root-block counters, one 128-byte line each (one per XCD slot)
+#define TM_STRIPES 8  // root-block and busy counters, one 128-byte line each (one per XCD slot)
 
 typedef struct {
-  unsigned long long next_chunk[TM_STRIPES][16];  // blocks claimed per stripe
+  struct {
+    int next;                 // claims after the wavefronts' first ones
+    int pad0[15];
+    int busy;                 // wavefronts holding work + records reserved and not yet taken
+    int pad1[15];
+  } stripe[TM_STRIPES];
   int error;        // bit 0: frame stack overflow, bit 1: empty frame, bit 2: deadline passed,
                     // bit 3: a donated frame never became ready
   int abort;        // set once the deadline passed: every wavefront stops
@@ -123,8 +128,6 @@ typedef struct {
   int pad0[31];
   unsigned int pool_tail;  // donated records reserved so far
   int pad1[31];
-  int busy;         // wavefronts holding work + records reserved and not yet taken
-  int pad2[31];
   int waiters;      // wavefronts waiting for donations (at most idle_cap)
   int pad4[31];
   int gen;          // launch generation of the donation ring: the reset kernel advances it,
@@ -133,7 +136,8 @@ typedef struct {
 } tm_sched;
 
 // A frame donated by a busy wavefront to an idle one: fields q, lvl, cur,
-// end, (unused), pend, tl, m[TM_MAXN], e[TM_MAXE], each stored as a 64-bit word
+// end, (unused), pend, tl, m[TM_MAXN], e[TM_MAXE] (q's word also carries the
+// stripe of the record's busy credit), each stored as a 64-bit word
 // (tag << 32 | value) with device-scope atomic stores, so a taker knows the
 // record is complete when every word carries the tag it expects: no fences,
 // no cache invalidation.  Records live in a ring of pool_cap slots; record r
@@ -170,13 +174,15 @@ typedef struct {
   const tm_query_dev *queries;
   // 4 ints per query: (delta, root_beg, root_end, start rule of edge 1)
   const int *qtab;
-  // The launch's roots as one space of 256-root blocks, query after query:
-  // query q owns blocks [block_prefix[q], block_prefix[q + 1]), its block i
-  // starting at root (root_beg & ~3) + 256 i (nq + 1 entries).
+  // The launch's roots as one space of blocks of 1 << unit_shift roots (16 to
+  // 1024), query after query: query q owns blocks [block_prefix[q],
+  // block_prefix[q + 1]), its block i starting at root (root_beg & ~3) +
+  // (i << unit_shift) (nq + 1 entries).
   const long long *block_prefix;
   int nq;
   long long total_blocks;
-  int claim_blocks;           // blocks per claim (the same for every query of the launch)
+  int unit_shift;
+  int claim_blocks;           // blocks per claim (0: shrinking with the blocks left)
   int frames;                 // LDS frame capacity per wavefront
   int scan_max;               // last-edge ranges up to this size are scanned
   int sb_flush;               // counting: survivors buffered before a full-width expansion (0: none buffered)
@@ -190,6 +196,7 @@ typedef struct {
   int pool_shift;             // log2(pool_cap)
   int steal_every;            // busy wavefronts look for idle ones every this many steps
   int steal_max;              // frames donated per look
+  int scouts;                 // wavefronts per stripe that look at the other stripes when theirs is dry
   int idle_cap;               // most wavefronts kept waiting on tickets without records
   int steal_min;              // a donated half holds at least this many candidates
   long long steal_after_ticks; // a task donates only after running this long (wall clock)

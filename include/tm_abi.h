@@ -61,10 +61,10 @@ typedef struct tm_host_graph {
 /* Launch parameters; zero fields take the library defaults (occupancy-limited
  * waves up to 32 per CU, scan_max 16, no time
  * limit, steal_every 16, steal_max 4, steal_min 64, steal_after_us 1000,
- * claim_blocks: about 8 claims of one query's roots per wavefront). */
+ * claim_blocks: claims that shrink with the roots left). */
 typedef struct tm_tuning {
   int32_t waves_per_cu;  /* resident wavefronts per CU in the persistent grid */
-  int32_t claim_blocks;  /* 256-root blocks per claim of the root schedule */
+  int32_t claim_blocks;  /* roots per claim of the root schedule, in units of 256 */
   int32_t scan_max;      /* last-edge ranges up to this size are scanned, larger ones use the pair index */
   int32_t time_limit_ms; /* abort the launch after this wall time on the device (0 = no limit) */
   int32_t steal_every;   /* busy wavefronts look for idle ones every this many steps */

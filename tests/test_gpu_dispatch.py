@@ -1,0 +1,39 @@
+"""Root dispatch of the mining kernel: blocks of 16 to 1024 roots, claims that
+shrink with the blocks left or have a caller's size, the first of each
+wavefront without an atomic.  Counts over root ranges that begin and end
+inside a block, on one wavefront up to a full grid, equal the oracle's."""
+import numpy as np
+import pytest
+
+from oracle import oracle, prep
+from helpers import random_graph
+
+pytestmark = pytest.mark.gpu
+
+# edges: a few blocks of 16, around 256 x 4 wavefronts' worth of them, and (with one wavefront per CU,
+# so 4 x 256 blocks are wanted) blocks of 32, 256 and 1024 roots
+SIZES = [17, 65, 1023, 4097, 40_003, 270_001, 1_060_007]
+
+
+@pytest.mark.parametrize("E", SIZES)
+def test_root_ranges(E):
+    from everest_amd import abi
+    rng = np.random.default_rng(E)
+    U, V, T = random_graph(rng, E, max(4, E // 6), 4 * E)
+    g = prep.preprocess(U, V, T)
+    dg = abi.DeviceGraph.from_dict(g)
+    cases = [([(0, 1, 0), (1, 2, 1)], 40), ([(0, 1, 0), (2, 0, 1), (1, 3, 2)], 60)]
+    ranges = [(0, -1), (1, E - 3), (3, E), (E // 3 + 1, 2 * E // 3 + 2), (E // 2, E // 2 + 1), (E // 2, E // 2)]
+    for mot, delta in cases:
+        for beg, end in ranges:
+            want = oracle.count(g, mot, delta, beg, end, nthreads=4)
+            for tune in (dict(), dict(waves_per_cu=1), dict(waves_per_cu=1, claim_blocks=1), dict(claim_blocks=3)):
+                print("E", E, "motif", mot, "roots", beg, end, tune, flush=True)
+                assert dg.count(mot, delta, beg, end, tune=abi.tuning(**tune)) == want, (mot, beg, end, tune)
+        # several queries' ranges in one launch, a short one between long ones
+        qs = [(mot, delta), (mot, 0), ([(0, 1, 0), (0, 1, 1)], delta), (mot, delta)]
+        want = [oracle.count(g, m, d, nthreads=4) for m, d in qs]
+        for tune in (dict(batch_mode=1), dict(batch_mode=2, waves_per_cu=1), dict(batch_mode=2, claim_blocks=2)):
+            print("E", E, "batch", tune, flush=True)
+            assert dg.batch_count(qs, tune=abi.tuning(**tune)) == want, tune
+    dg.close()
