@@ -482,7 +482,8 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
     const int sb = flush > 0 ? (4 + nmap) * tmk::WAVE : 0;  // position, root, weight (2), node map
     const int t2 = counting ? 2 * tmk::WAVE : 0;             // two-edge tail side table
     const int roots = (counting ? 4 : 2) * tmk::TM_ROOTS;    // window, and the root-pair list (counting)
-    return (frames * per_frame + roots + sb + t2) * (int)sizeof(int) + nq * (int)sizeof(unsigned long long);
+    const int swept = 2 * tmk::WAVE;                         // long frames' candidates
+    return (frames * per_frame + roots + sb + t2 + swept) * (int)sizeof(int) + nq * (int)sizeof(unsigned long long);
   };
   int wpe = 0;  // register cap of the counting kernel: 1 (none), 4 (128 VGPRs), 5 (96) or 6 (80)
   if (tune && tune->waves_per_simd_hint > 0) {

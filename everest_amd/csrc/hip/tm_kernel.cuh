@@ -29,6 +29,7 @@ namespace tmk {
 constexpr int WAVE = 64;
 constexpr int TM_ROW = 4 * WAVE;    // roots of one 16-byte load per lane
 constexpr int TM_ROWS = 4;          // most rows of a dispatch block (1024 roots)
+constexpr int TM_SWEEP = 8;         // 64-slot chunks of a long frame whose rule times are read together
 constexpr int TM_ROOTS = WAVE + 1;  // window table entries: one per lane's root, one for a taken frame
 
 // ------------------------------------------------------------------ helpers
@@ -739,8 +740,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
   // deepest level are pushed in one step, at most 64 of them)
   int *sw_lo = sb_m + (COMPACT ? MAXN * WAVE : 0);
   int *sw_hi = sw_lo + (T2 ? WAVE : 0);
+  // candidates of long frames that passed their rules: slot and frame
+  int *sl_slot = sw_hi + (T2 ? WAVE : 0);
+  int *sl_frame = sl_slot + WAVE;
   // per-query counts of this wavefront, flushed once at the end
-  unsigned long long *q_cnt = (unsigned long long *)(sw_hi + (T2 ? WAVE : 0));
+  unsigned long long *q_cnt = (unsigned long long *)(sl_frame + WAVE);
   for (int q = lane; q < args.nq; q += WAVE) q_cnt[q] = 0;
   __syncthreads();
 
@@ -1184,48 +1188,149 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
       sbn = 0;
       __syncthreads();
     } else {
-    // ---- deal the next candidate slots of the topmost frames of one level
-    // to the lanes (at most lim: room left in the survivor buffer)
     const int L = Ltop;
-    const int lim = COMPACT ? WAVE - sbn : WAVE;
-    const int fi = top - 1 - lane;
-    int fcnt = 0;
-    if (fi >= 0) {
-      int lv = f_lvl[fi];
-      if ((lv & 0xff) == L) fcnt = f_end[fi] - f_cur[fi];
+    j = L + 1;  // motif edge of the candidates
+    const int kind = SP::kind(md, j);
+    const int tmn = (j + 1 < M) ? SP::tmode(md, j + 1) : -1;  // pruning rule of edge j + 1
+    // further rules: each later edge (k >= j + 2) at a node of this edge
+    // needs that node's next edge after this position in the window (not
+    // in the instrumented kernel, which follows the reference's search tree)
+    const unsigned xm = INSTR == 1 ? 0u : (unsigned)SP::xmask(md, j);
+    const int lim = COMPACT ? WAVE - sbn : WAVE;  // (room left in the survivor buffer)
+    // ---- a long frame on top whose candidates have a pruning rule: most
+    // fail it (0.5% pass in 0->1, 0->2, 2->3 on 64M edges), so the rules'
+    // times alone are read, TM_SWEEP x 64 slots in flight, over as many such
+    // frames as it takes to collect a wavefront's worth of candidates that
+    // pass; those go on below as if dealt.  The general deal costs 4.3 us of
+    // dependent LDS traffic per 64 candidates: that query 348 ms, 68 ms so.
+    int nl = 0;
+    if (INSTR != 1 && (tmn >= 0 || xm != 0)) {
+      const int r0 = tmn >= 0 ? tmn : __ffs(xm) - 1;
+      const unsigned rules = xm & ~(1u << r0);
+      bool full = false, moved = false;
+      while (!full && top > 0) {
+        const int ft = top - 1;
+        const int lvt = uni(f_lvl[ft]);
+        const int c0 = uni(f_cur[ft]), c1 = uni(f_end[ft]);
+        const int tlt = uni(r_tl[(lvt >> 16) & 0xff]);
+        if (c1 - c0 < WAVE || (lvt & (LV_SWAP | LV_PAT | 0xff)) != L) break;
+        const int lt = kind == TM_K_NEW_DST ? TM_L_OUT
+                       : (kind == TM_K_NEW_SRC ? TM_L_IN : ((lvt & LV_DIR) ? TM_L_INPAIR : TM_L_OUTPAIR));
+        const int *stl = g.stf + (size_t)(lt * TM_NTFIRST) * (size_t)g.E;
+        int sl = c0;
+        while (!full && sl < c1) {
+          int x[TM_SWEEP];
+          unsigned long long om[TM_SWEEP];  // of each chunk, the slots that pass
+          const int *st = stl + (size_t)r0 * (size_t)g.E + sl + lane;
+#pragma unroll
+          for (int k = 0; k < TM_SWEEP; k++) x[k] = sl + WAVE * k + lane < c1 ? st[WAVE * k] : 0x7fffffff;
+          if (mt) meter.b += 4 * (unsigned)max(0, min(TM_SWEEP, (c1 - sl + WAVE - 1 - lane) / WAVE));
+          unsigned long long any = 0;
+#pragma unroll
+          for (int k = 0; k < TM_SWEEP; k++) {
+            om[k] = __ballot(x[k] <= tlt && sl + WAVE * k + lane < c1);
+            any |= om[k];
+          }
+          for (unsigned rr = rules; rr != 0 && any != 0ull; rr &= rr - 1) {
+            st = stl + (size_t)(__ffs(rr) - 1) * (size_t)g.E + sl + lane;
+#pragma unroll
+            for (int k = 0; k < TM_SWEEP; k++) {
+              x[k] = 0x7fffffff;
+              if ((om[k] >> lane) & 1) {
+                if (mt) meter.b += 4;
+                x[k] = st[WAVE * k];
+              }
+            }
+            any = 0;
+#pragma unroll
+            for (int k = 0; k < TM_SWEEP; k++) {
+              om[k] &= __ballot(x[k] <= tlt);
+              any |= om[k];
+            }
+          }
+#pragma unroll
+          for (int k = 0; k < TM_SWEEP; k++) {
+            if (full || sl >= c1) continue;
+            const int n = __popcll(om[k]);
+            if (nl + n > lim) {
+              full = true;
+              continue;
+            }
+            if ((om[k] >> lane) & 1) {
+              const int w = nl + __popcll(om[k] & lt_mask);
+              sl_slot[w] = sl + lane;
+              sl_frame[w] = ft;
+            }
+            nl += n;
+            sl = min(sl + WAVE, c1);
+          }
+        }
+        st_items += (unsigned long long)(sl - c0);
+        moved |= sl != c0;
+        if (sl < c1) {
+          if (lane == 0) f_cur[ft] = sl;
+        } else {
+          top = ft;  // (its words stay in place until the next push)
+        }
+      }
+      __syncthreads();
+      if (nl == 0 && moved) {
+        st_steps++;
+        continue;
+      }
     }
-    int incl = wave_incl_scan(fcnt, lane);
-    int excl = incl - fcnt;
-    int total = uni(__shfl(incl, WAVE - 1));
-    if (total > lim) total = lim;
-    if (total <= 0) {  // a frame on the stack is never empty; stop rather than spin
-      if (lane == 0) atomicOr(&sched->error, 2);
-      break;
-    }
-    const bool part = (fcnt > 0) && (excl < lim);
-    const unsigned long long pm = __ballot(part);
-    const int nparts = __popcll(pm);
-    int take = part ? min(fcnt, lim - excl) : 0;
-    const bool last_partial = __ballot(part && take < fcnt) != 0ull;
-
-    int rank, off;
-    if (uni(__shfl(fcnt, 0)) >= lim) {
-      rank = 0; off = lane;
+    int slot = 0, myf = 0, ntop = top;
+    bool has = lane < nl;
+    if (nl > 0) {
+      if (has) {
+        slot = sl_slot[lane];
+        myf = sl_frame[lane];
+      }
     } else {
-      unsigned long long sm = wave_or64(part ? (1ull << excl) : 0ull);
-      unsigned long long le = (lane == 63) ? ~0ull : ((2ull << lane) - 1ull);
-      rank = __popcll(sm & le) - 1;
-      if (rank < 0) rank = 0;
-      off = lane - __shfl(excl, rank);
+      // ---- deal the next candidate slots of the topmost frames of one level
+      // to the lanes
+      const int fi = top - 1 - lane;
+      int fcnt = 0;
+      if (fi >= 0) {
+        int lv = f_lvl[fi];
+        if ((lv & 0xff) == L) fcnt = f_end[fi] - f_cur[fi];
+      }
+      int incl = wave_incl_scan(fcnt, lane);
+      int excl = incl - fcnt;
+      int total = uni(__shfl(incl, WAVE - 1));
+      if (total > lim) total = lim;
+      if (total <= 0) {  // a frame on the stack is never empty; stop rather than spin
+        if (lane == 0) atomicOr(&sched->error, 2);
+        break;
+      }
+      const bool part = (fcnt > 0) && (excl < lim);
+      const int nparts = __popcll(__ballot(part));
+      int take = part ? min(fcnt, lim - excl) : 0;
+      const bool last_partial = __ballot(part && take < fcnt) != 0ull;
+
+      int rank, off;
+      if (uni(__shfl(fcnt, 0)) >= lim) {
+        rank = 0; off = lane;
+      } else {
+        unsigned long long sm = wave_or64(part ? (1ull << excl) : 0ull);
+        unsigned long long le = (lane == 63) ? ~0ull : ((2ull << lane) - 1ull);
+        rank = __popcll(sm & le) - 1;
+        if (rank < 0) rank = 0;
+        off = lane - __shfl(excl, rank);
+      }
+      has = lane < total;
+      myf = top - 1 - rank;
+      if (has) slot = f_cur[myf] + off;
+      st_items += total;
+      __syncthreads();
+      // consume: the deepest participating frame may stay with an advanced cursor
+      if (part && take < fcnt) f_cur[fi] += take;
+      ntop = top - nparts + (last_partial ? 1 : 0);
     }
-    const bool has = lane < total;
-    const int myf = top - 1 - rank;
     st_steps++;
-    st_items += total;
-    int slot = 0, dir = 0, lvw = 0;
+    int dir = 0, lvw = 0;
     unsigned fw = 1;  // the frame's weight (counting)
     if (has) {
-      slot = f_cur[myf] + off;
       const int lv = f_lvl[myf];
       lvw = lv;
       if (T2) fw = (unsigned)f_w[myf];
@@ -1241,13 +1346,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
       }
     }
     __syncthreads();
-    // consume: the deepest participating frame may stay with an advanced cursor
-    if (part && take < fcnt) f_cur[fi] += take;
-    int ntop = top - nparts + (last_partial ? 1 : 0);
-
-    j = L + 1;  // motif edge of the candidates
-    const int kind = SP::kind(md, j);
-    const int tmn = (j + 1 < M) ? SP::tmode(md, j + 1) : -1;  // pruning rule of edge j + 1
     // a swapped frame (two-edge tail): the slot is a candidate of the last
     // edge; its matches with the earlier candidates of edge j are counted here
     const bool swp = T2 && has && (lvw & LV_SWAP);
@@ -1265,23 +1363,20 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
       cnt += tail_pattern<SP>(md) == TP_STAR ? 0ull - sp : sp;
       st_leaves++;
     }
-    int tfn = 0, node = -1;
+    int tfn = 0, tx = 0, node = -1;
     // position, neighbour and the next edge's first-candidate time: three
     // loads at the same slot of one list, issued together
     const int lst = kind == TM_K_NEW_DST ? TM_L_OUT
                     : (kind == TM_K_NEW_SRC ? TM_L_IN : (dir ? TM_L_INPAIR : TM_L_OUTPAIR));
     if (has && !swp && !patf) {
-      if (tmn >= 0) tfn = g.stf[(size_t)(lst * TM_NTFIRST + tmn) * (size_t)g.E + slot];
-      // further rules: each later edge (k >= j + 2) at a node of this edge
-      // needs that node's next edge after this position in the window (not
-      // in the instrumented kernel, which follows the reference's search tree)
-      const int xm = INSTR == 1 ? 0 : SP::xmask(md, j);
-      // position, neighbour (new node), the next edge's time and the further rules' times
-      if (mt) meter.b += 4 * (1 + (kind != TM_K_CLOSE ? 1 : 0) + (tmn >= 0 ? 1 : 0) + __popc((unsigned)xm));
-      int tx = -0x7fffffff - 1;
+      // position, neighbour (new node); unless swept, the next edge's time and the further rules' times
+      if (mt) meter.b += kind != TM_K_CLOSE ? 8 : 4;
+      if (mt && nl == 0) meter.b += 4 * ((tmn >= 0 ? 1 : 0) + __popc(xm));
+      tfn = tx = -0x7fffffff - 1;
+      if (nl == 0 && tmn >= 0) tfn = g.stf[(size_t)(lst * TM_NTFIRST + tmn) * (size_t)g.E + slot];
 #pragma unroll
       for (int rr = 0; rr < TM_NTFIRST; rr++)
-        if ((xm >> rr) & 1) tx = max(tx, g.stf[(size_t)(lst * TM_NTFIRST + rr) * (size_t)g.E + slot]);
+        if (nl == 0 && ((xm >> rr) & 1)) tx = max(tx, g.stf[(size_t)(lst * TM_NTFIRST + rr) * (size_t)g.E + slot]);
       if (kind == TM_K_NEW_DST) {
         pos = g.outPos[slot]; node = g.outNbr[slot];
         valid = !in_first(m, SP::mapped(md, j), node);
