@@ -4,8 +4,9 @@
 // Graph residency: a graph is uploaded once and stays in HBM with the
 // reference arrays (Eg, in/out CSR, Euid) plus indexes built on the device at
 // upload: packed times T, neighbour arrays aligned with the CSR position
-// lists, a per-node (neighbour, position)-sorted copy of each list (the pair
-// index), and a time-bucket index for the window end.
+// lists, a per-node (neighbour, position)-sorted copy of each out-list (the
+// pair index) with a hash table of its pairs, and a time-bucket index for the
+// window end.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
@@ -41,7 +42,7 @@ tm_status fail(tm_status s, const std::string &msg) {
 __global__ void aux_kernel(const tm_edge *__restrict__ Eg, const int *__restrict__ outPos,
                            const int *__restrict__ inPos, int E, int *__restrict__ T,
                            int *__restrict__ outNbr, int *__restrict__ inNbr,
-                           unsigned long long *__restrict__ okey, unsigned long long *__restrict__ ikey) {
+                           unsigned long long *__restrict__ okey) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= E) return;
   T[i] = Eg[i].t;
@@ -52,7 +53,6 @@ __global__ void aux_kernel(const tm_edge *__restrict__ Eg, const int *__restrict
   int pi = inPos[i];
   tm_edge ei = Eg[pi];
   inNbr[i] = ei.u;
-  ikey[i] = ((unsigned long long)(unsigned)ei.v << 32) | (unsigned)ei.u;
 }
 
 // slot of each position inside the list that holds it
@@ -167,6 +167,41 @@ __global__ void sprev_kernel(const tm_edge *__restrict__ Eg, const int *__restri
     if (ps > outR[e.u] && outPairNbr[ps - 1] == e.v) prev = outPairPos[ps - 1];
     sprev[(size_t)k * E + s] = prev;
   }
+}
+
+// Distinct pairs of the sorted pair keys (a run of equal keys each).
+__global__ void __launch_bounds__(256) heads_kernel(const unsigned long long *__restrict__ k, int n,
+                                                    unsigned long long *count) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int c = __syncthreads_count(i < n && (i == 0 || k[i] != k[i - 1]));
+  if (threadIdx.x == 0 && c) atomicAdd(count, (unsigned long long)c);
+}
+
+// The pair table's entries: the first slot of each run claims a place by its
+// key and writes the run's slots.
+__global__ void pair_table_kernel(const unsigned long long *__restrict__ k, int n, unsigned long long *tab,
+                                  unsigned mask) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n || (i > 0 && k[i] == k[i - 1])) return;
+  const unsigned long long key = k[i];
+  int hi = i + 1;  // the run's end, galloping
+  for (int step = 1; hi < n && k[hi] == key; step <<= 1) {
+    int lo = hi + 1, e = (int)min((long long)hi + step, (long long)n);
+    if (e < n && k[e] == key) { hi = e; continue; }
+    while (lo < e) {
+      const int mid = (lo + e) >> 1;
+      if (k[mid] == key) lo = mid + 1; else e = mid;
+    }
+    hi = lo;
+    break;
+  }
+  const int x = (int)(unsigned)(key >> 32), y = (int)(unsigned)key;
+  const unsigned long long word = ((unsigned long long)(unsigned)y << 32) | (unsigned)x;  // {x, y} in memory
+  for (unsigned h = tm_pair_hash(x, y) & mask;; h = (h + 1) & mask)
+    if (atomicCAS(tab + 2 * (size_t)h, ~0ull, word) == ~0ull) {
+      tab[2 * (size_t)h + 1] = ((unsigned long long)(unsigned)hi << 32) | (unsigned)i;
+      return;
+    }
 }
 
 __global__ void low_word_kernel(const unsigned long long *__restrict__ k, int *__restrict__ out, int n) {
@@ -1029,8 +1064,6 @@ tm_status tm_graph_upload(int32_t device, const tm_host_graph *hg, tm_graph **ou
   ALLOC(vw.inNbr, e4);
   ALLOC(vw.outPairNbr, e4);
   ALLOC(vw.outPairPos, e4);
-  ALLOC(vw.inPairNbr, e4);
-  ALLOC(vw.inPairPos, e4);
   ALLOC(vw.Euid, e4);
   ALLOC(vw.outSelf, e4);
   ALLOC(vw.inSelf, e4);
@@ -1040,7 +1073,7 @@ tm_status tm_graph_upload(int32_t device, const tm_host_graph *hg, tm_graph **ou
   for (int k = 0; k < TM_NTFIRST; k++) {
     ALLOC(vw.tfirst[k], e4);
   }
-  ALLOC(vw.stf, e4 * 4 * TM_NTFIRST);
+  ALLOC(vw.stf, e4 * 3 * TM_NTFIRST);
   ALLOC(vw.sprev, e4 * 2);
   vw.epad = (int)(((long long)E + 255) / 256 * 256 + 256);
   ALLOC(vw.rgap, sizeof(unsigned) * (size_t)vw.epad * TM_NTFIRST);
@@ -1066,22 +1099,20 @@ tm_status tm_graph_upload(int32_t device, const tm_host_graph *hg, tm_graph **ou
   H2D(vw.Euid, hg->Euid, e4);
 #undef H2D
   // temporaries for the pair index
-  unsigned long long *okey = nullptr, *ikey = nullptr, *skey = nullptr;
+  unsigned long long *okey = nullptr, *skey = nullptr;
   void *tmp = nullptr;
   size_t tmp_bytes = 0;
   auto free_tmp = [&]() {
     if (okey) (void)hipFree(okey);
-    if (ikey) (void)hipFree(ikey);
     if (skey) (void)hipFree(skey);
     if (tmp) (void)hipFree(tmp);
   };
 #define TMPCHK(expr) \
   if ((he = (expr)) != hipSuccess) { free_tmp(); return cleanup(fail(he == hipErrorOutOfMemory ? TM_ERR_NOMEM : TM_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(he))); }
   TMPCHK(hipMalloc(&okey, sizeof(unsigned long long) * (size_t)E));
-  TMPCHK(hipMalloc(&ikey, sizeof(unsigned long long) * (size_t)E));
   TMPCHK(hipMalloc(&skey, sizeof(unsigned long long) * (size_t)E));
   hipLaunchKernelGGL(aux_kernel, dim3((E + 255) / 256), dim3(256), 0, s, vw.Eg, vw.outPos, vw.inPos, E,
-                     (int *)vw.T, (int *)vw.outNbr, (int *)vw.inNbr, okey, ikey);
+                     (int *)vw.T, (int *)vw.outNbr, (int *)vw.inNbr, okey);
   TMPCHK(hipGetLastError());
   const int end_bit = std::min(64, 32 + std::max(1, ceil_log2((long long)V + 1)));
   TMPCHK(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp_bytes, okey, skey, vw.outPos, (int *)vw.outPairPos,
@@ -1091,10 +1122,24 @@ tm_status tm_graph_upload(int32_t device, const tm_host_graph *hg, tm_graph **ou
                                             0, end_bit, s));
   hipLaunchKernelGGL(low_word_kernel, dim3((E + 255) / 256), dim3(256), 0, s, skey, (int *)vw.outPairNbr, E);
   TMPCHK(hipGetLastError());
-  TMPCHK(hipcub::DeviceRadixSort::SortPairs(tmp, tmp_bytes, ikey, skey, vw.inPos, (int *)vw.inPairPos, E, 0,
-                                            end_bit, s));
-  hipLaunchKernelGGL(low_word_kernel, dim3((E + 255) / 256), dim3(256), 0, s, skey, (int *)vw.inPairNbr, E);
-  TMPCHK(hipGetLastError());
+  {
+    // the pair table, at most half full
+    unsigned long long pairs = 0, *d_pairs = okey;  // (okey is not needed any more)
+    TMPCHK(hipMemsetAsync(d_pairs, 0, sizeof(pairs), s));
+    hipLaunchKernelGGL(heads_kernel, dim3((E + 255) / 256), dim3(256), 0, s, skey, E, d_pairs);
+    TMPCHK(hipGetLastError());
+    TMPCHK(hipMemcpyAsync(&pairs, d_pairs, sizeof(pairs), hipMemcpyDeviceToHost, s));
+    TMPCHK(hipStreamSynchronize(s));
+    size_t n = 4;
+    while (n < 2 * (size_t)pairs) n <<= 1;
+    if ((st = dev_alloc(g, &p, 16 * n)) != TM_OK) { free_tmp(); return cleanup(st); }
+    vw.ptab = (const int *)p;
+    vw.pmask = (unsigned)(n - 1);
+    TMPCHK(hipMemsetAsync(p, 0xff, 16 * n, s));
+    hipLaunchKernelGGL(pair_table_kernel, dim3((E + 255) / 256), dim3(256), 0, s, skey, E, (unsigned long long *)p,
+                       vw.pmask);
+    TMPCHK(hipGetLastError());
+  }
   {
     const dim3 gr((E + 255) / 256), bl(256);
     hipLaunchKernelGGL(self_kernel, gr, bl, 0, s, vw.outPos, E, (int *)vw.outSelf);
@@ -1109,8 +1154,8 @@ tm_status tm_graph_upload(int32_t device, const tm_host_graph *hg, tm_graph **ou
                        (int *)vw.tfirst[3], (int *)vw.tfirst[4], (int *)vw.tfirst[5]);
     TMPCHK(hipGetLastError());
     {
-      const int *lists[4] = {vw.outPos, vw.inPos, vw.outPairPos, vw.inPairPos};  // TM_L_* order
-      for (int l = 0; l < 4; l++) {
+      const int *lists[3] = {vw.outPos, vw.inPos, vw.outPairPos};  // TM_L_* order
+      for (int l = 0; l < 3; l++) {
         int *o = (int *)vw.stf + (size_t)l * TM_NTFIRST * E;
         hipLaunchKernelGGL(stf_kernel, gr, bl, 0, s, lists[l], E, vw.tfirst[0], vw.tfirst[1], vw.tfirst[2],
                            vw.tfirst[3], vw.tfirst[4], vw.tfirst[5], o, o + (size_t)E, o + 2 * (size_t)E,

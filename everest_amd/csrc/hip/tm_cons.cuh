@@ -79,9 +79,8 @@ __device__ __forceinline__ void cand_list(const tm_graph_view &g, int j, const i
     *hi = g.inR[y + 1];
   } else {
     const int x = m[CS::a(j)], y = m[CS::b(j)];
-    const int lo0 = g.outR[x], hi0 = g.outR[x + 1];
-    const int s0 = tmk::lower_bound_i(g.outPairNbr, lo0, hi0, y);
-    const int s1 = tmk::upper_bound_i(g.outPairNbr, s0, hi0, y);
+    int s0, s1;
+    tmk::pair_find(g, x, y, &s0, &s1);
     *lo = tmk::upper_bound_i(g.outPairPos, s0, s1, p);
     *hi = s1;
   }

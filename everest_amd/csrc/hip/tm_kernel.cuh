@@ -222,78 +222,60 @@ __device__ __forceinline__ int gallop_ub(const int *__restrict__ a, int lo, int 
   }
 }
 
-// Entries of the pair segment key inside one node's (neighbour, position)-
-// sorted list [lo, hi) whose positions lie in (p, pend).
-__device__ __forceinline__ int pair_count(const int *__restrict__ pnbr, const int *__restrict__ ppos,
-                                          int lo, int hi, int key, int p, int pend, Meter *mt = nullptr) {
-  int s0 = lower_bound_i(pnbr, lo, hi, key, mt);
-  if (mt && s0 < hi) mt->b += 4;
-  if (s0 >= hi || pnbr[s0] != key) return 0;
-  int s1 = gallop_ub(pnbr, s0 + 1, hi, key, mt);
-  int c0 = upper_bound_i(ppos, s0, s1, p, mt);
-  int c1 = gallop_lb(ppos, c0, s1, pend, mt);
-  return c1 - c0;
+// The slots [*s0, *s1) of the pair x -> y in the pair index (none: false),
+// from the pair table: one 16-byte read for most pairs, present or not.  The
+// binary searches in the shorter of out(x) and in(y) that it replaced took
+// two reads for the bounds and one per halving, 15 to 20 dependent ones at a
+// hub (4-cycle on 8M hub edges 38.2 -> 16.6 ms, a fork closing two pairs on 8M
+// edges 17.1 -> 9.3 ms, all 3-edge motifs on 100k edges 9.9 -> 6.2 ms of kernels).
+__device__ __forceinline__ bool pair_find(const tm_graph_view &g, int x, int y, int *s0, int *s1,
+                                          Meter *mt = nullptr) {
+  for (unsigned h = tm_pair_hash(x, y) & g.pmask;; h = (h + 1) & g.pmask) {
+    if (mt) mt->b += 16;
+    const int4 e = ((const int4 *)g.ptab)[h];
+    if (e.x == x && e.y == y) {
+      *s0 = e.z;
+      *s1 = e.w;
+      return true;
+    }
+    if (e.x < 0) {  // (the table is at most half full)
+      *s0 = *s1 = 0;
+      return false;
+    }
+  }
 }
 
-// The last position in (p, pend) of an edge x -> y, or -1 (the pair's
-// positions through the shorter of out(x) and in(y)).
+// The last position in (p, pend) of an edge x -> y, or -1.
 __device__ __forceinline__ int pair_last(const tm_graph_view &g, int x, int y, int p, int pend,
                                          Meter *mt = nullptr) {
-  int lo = g.outR[x], hi = g.outR[x + 1], key = y;
-  const int *pn = g.outPairNbr, *pp = g.outPairPos;
-  const int ilo = g.inR[y], ihi = g.inR[y + 1];
-  if (mt) mt->b += 16;
-  if (ihi - ilo < hi - lo) { lo = ilo; hi = ihi; key = x; pn = g.inPairNbr; pp = g.inPairPos; }
-  const int s0 = lower_bound_i(pn, lo, hi, key, mt);
-  if (mt && s0 < hi) mt->b += 4;
-  if (s0 >= hi || pn[s0] != key) return -1;
-  const int s1 = gallop_ub(pn, s0 + 1, hi, key, mt);
-  const int i = lower_bound_i(pp, s0, s1, pend, mt) - 1;
+  int s0, s1;
+  if (!pair_find(g, x, y, &s0, &s1, mt)) return -1;
+  const int i = lower_bound_i(g.outPairPos, s0, s1, pend, mt) - 1;
   if (mt && i >= s0) mt->b += 4;
-  return (i >= s0 && pp[i] > p) ? pp[i] : -1;
+  return (i >= s0 && g.outPairPos[i] > p) ? g.outPairPos[i] : -1;
 }
 
-// Edges x -> y with positions in (p, pend), searched in the shorter of out(x)
-// and in(y) (the list is chosen first, so the search is in the code once).
+// Edges x -> y with positions in (p, pend).
 __device__ __forceinline__ int edge_count(const tm_graph_view &g, int x, int y, int p, int pend,
                                           Meter *mt = nullptr) {
-  const int olo = g.outR[x], ohi = g.outR[x + 1];
-  const int ilo = g.inR[y], ihi = g.inR[y + 1];
-  if (mt) mt->b += 16;
-  const bool o = ohi - olo <= ihi - ilo;
-  return pair_count(o ? g.outPairNbr : g.inPairNbr, o ? g.outPairPos : g.inPairPos, o ? olo : ilo, o ? ohi : ihi,
-                    o ? y : x, p, pend, mt);
-}
-
-// The slots [*s0, *s1) of the pair x -> y in the pair index of the shorter of
-// out(x) (*dir 0) and in(y) (*dir 1).
-__device__ __forceinline__ void pair_range(const tm_graph_view &g, int x, int y, int *s0, int *s1, int *dir,
-                                           Meter *mt = nullptr) {
-  const int olo = g.outR[x], ohi = g.outR[x + 1];
-  const int ilo = g.inR[y], ihi = g.inR[y + 1];
-  if (mt) mt->b += 16;
-  const bool o = ohi - olo <= ihi - ilo;
-  const int *pn = o ? g.outPairNbr : g.inPairNbr;
-  const int hi = o ? ohi : ihi, key = o ? y : x;
-  *dir = o ? 0 : 1;
-  *s0 = lower_bound_i(pn, o ? olo : ilo, hi, key, mt);
-  *s1 = gallop_ub(pn, *s0, hi, key, mt);
+  int s0, s1;
+  if (!pair_find(g, x, y, &s0, &s1, mt)) return 0;
+  const int c0 = upper_bound_i(g.outPairPos, s0, s1, p, mt);
+  return gallop_lb(g.outPairPos, c0, s1, pend, mt) - c0;
 }
 
 // Candidate list of motif edge j: slots [lo, hi) of `pos` (and `nbr` for new
 // nodes) whose positions are > p, the position matched for edge j-1.
-// dir (CLOSE only): 0 = out-pair index of m[a], 1 = in-pair index of m[b].
 struct CandList {
   const int *pos;
   const int *nbr;
-  int lo, hi, dir;
+  int lo, hi;
 };
 
 template <class SP, int MAXN>
 __device__ __forceinline__ CandList cand_start(const tm_graph_view &g, const tm_motif_dev &md, int j,
                                                const int (&m)[MAXN], int p, Meter *mt = nullptr) {
   CandList L;
-  L.dir = 0;
   const int kind = SP::kind(md, j);
   const int mode = SP::smode(md, j);
   if (kind != TM_K_CLOSE) {
@@ -313,18 +295,14 @@ __device__ __forceinline__ CandList cand_start(const tm_graph_view &g, const tm_
   } else {
     const int x = sel(m, SP::a(md, j)), y = sel(m, SP::b(md, j));
     L.nbr = nullptr;
-    if (mode == TM_S_PAIR_SELF) {
-      // the same pair as edge j-1: continue right after p inside its segment
-      L.pos = g.outPairPos;
+    L.pos = g.outPairPos;
+    int s0;
+    pair_find(g, x, y, &s0, &L.hi, mt);
+    if (mode == TM_S_PAIR_SELF) {  // the same pair as edge j-1: right after p
       L.lo = g.outPairSelf[p] + 1;
-      if (mt) mt->b += 8;
-      L.hi = gallop_ub(g.outPairNbr, L.lo, g.outR[x + 1], y, mt);
+      if (mt) mt->b += 4;
     } else {
-      int s0, s1;
-      pair_range(g, x, y, &s0, &s1, &L.dir, mt);
-      L.pos = L.dir ? g.inPairPos : g.outPairPos;
-      L.lo = upper_bound_i(L.pos, s0, s1, p, mt);
-      L.hi = s1;
+      L.lo = upper_bound_i(L.pos, s0, L.hi, p, mt);
     }
   }
   return L;
@@ -378,11 +356,8 @@ __device__ __forceinline__ unsigned long long leaf_count(const tm_graph_view &g,
 // and y after c; summed over the edges q at y in the window (B = y's list),
 // each counts A's edges to q's other end before it (one pair search).
 
-// lvl word of a frame: level | A's pair direction << 8 | swapped << 9 |
-// B's pair direction << 10 | root index << 16
-constexpr int LV_DIR = 1 << 8;
+// lvl word of a frame: level | swapped << 9 | ... | root index << 16
 constexpr int LV_SWAP = 1 << 9;
-constexpr int LV_BDIR = 1 << 10;
 
 enum { T2_NONE = 0, T2_INDEP = 1, T2_JOIN = 2 };
 
@@ -403,13 +378,12 @@ __device__ __forceinline__ bool tail2_ok(const tm_motif_dev &md) {
 }
 
 // Edge k's candidates (k = M-1) with positions in (pa0, pend), pa0 the
-// position of A's first candidate: [*lo, *hi) in the list of *bdir.
+// position of A's first candidate: [*lo, *hi) of its list.
 template <class SP, int MAXN>
 __device__ __forceinline__ void tail2_range(const tm_graph_view &g, const tm_motif_dev &md, const int (&m)[MAXN],
-                                            int pa0, int pend, int *lo, int *hi, int *bdir, Meter *mt = nullptr) {
+                                            int pa0, int pend, int *lo, int *hi, Meter *mt = nullptr) {
   const int k = SP::M(md) - 1;
   const int kind = SP::kind(md, k);
-  *bdir = 0;
   const int *pos;
   int s0, s1;
   if (tail2_mode<SP>(md) == T2_JOIN || kind != TM_K_CLOSE) {
@@ -424,21 +398,21 @@ __device__ __forceinline__ void tail2_range(const tm_graph_view &g, const tm_mot
     s1 = R[y + 1];
     if (mt) mt->b += 8;
   } else {
-    pair_range(g, sel(m, SP::a(md, k)), sel(m, SP::b(md, k)), &s0, &s1, bdir, mt);
-    pos = *bdir ? g.inPairPos : g.outPairPos;
+    pair_find(g, sel(m, SP::a(md, k)), sel(m, SP::b(md, k)), &s0, &s1, mt);
+    pos = g.outPairPos;
   }
   *lo = upper_bound_i(pos, s0, s1, pa0, mt);
   *hi = gallop_lb(pos, *lo, s1, pend, mt);
 }
 
 // Matches of the last two edges whose last edge is edge k's candidate at
-// `slot` (list direction bdir): edge j's candidates in A [alo, ahi) (pair
-// direction adir) before it, less those whose new node is mapped or equal to
+// `slot`: edge j's candidates in A [alo, ahi) before it, less those whose new
+// node is mapped or equal to
 // the candidate's new node.
 template <class SP, int MAXN>
 __device__ __forceinline__ unsigned long long tail2_item(const tm_graph_view &g, const tm_motif_dev &md,
-                                                         const int (&m)[MAXN], int alo, int ahi, int adir,
-                                                         int slot, int bdir, int zmask = 0, Meter *mt = nullptr) {
+                                                         const int (&m)[MAXN], int alo, int ahi,
+                                                         int slot, int zmask = 0, Meter *mt = nullptr) {
   const int M = SP::M(md);
   const int j = M - 2, k = M - 1;
   const int nm = SP::mapped(md, j);
@@ -455,10 +429,10 @@ __device__ __forceinline__ unsigned long long tail2_item(const tm_graph_view &g,
     if (mt) mt->b += 8;
     if (in_first(m, nm, z)) return 0ull;  // z must be a new node
   } else {
-    qpos = bdir ? g.inPairPos[slot] : g.outPairPos[slot];
+    qpos = g.outPairPos[slot];
     if (mt) mt->b += 4;
   }
-  const int *apos = kj == TM_K_NEW_DST ? g.outPos : (kj == TM_K_NEW_SRC ? g.inPos : (adir ? g.inPairPos : g.outPairPos));
+  const int *apos = kj == TM_K_NEW_DST ? g.outPos : (kj == TM_K_NEW_SRC ? g.inPos : g.outPairPos);
   int r = 0;
   if (!join) {
     r = lower_bound_i(apos, alo, ahi, qpos, mt) - alo;
@@ -668,7 +642,7 @@ __device__ __forceinline__ int pair_tail_edge(const tm_motif_dev &md) {
 // ------------------------------------------------------------------ kernel
 
 // LDS frame stack, structure of arrays, capacity FR frames:
-//   cur, end, p (last matched position), pend, lvl (level | dir << 8 | swap flags),
+//   cur, end, p (last matched position), pend, lvl (level | flags),
 //   m[MAXN][FR] mapping, and in enumeration mode e[MAXE][FR] matched positions.
 // Reference work of one resolved candidate list (the instrumented variant):
 // the reference scans list entries after p until the first one outside the
@@ -1191,6 +1165,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     const int L = Ltop;
     j = L + 1;  // motif edge of the candidates
     const int kind = SP::kind(md, j);
+    const int lst = kind == TM_K_NEW_DST ? TM_L_OUT : (kind == TM_K_NEW_SRC ? TM_L_IN : TM_L_OUTPAIR);
     const int tmn = (j + 1 < M) ? SP::tmode(md, j + 1) : -1;  // pruning rule of edge j + 1
     // further rules: each later edge (k >= j + 2) at a node of this edge
     // needs that node's next edge after this position in the window (not
@@ -1214,9 +1189,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         const int c0 = uni(f_cur[ft]), c1 = uni(f_end[ft]);
         const int tlt = uni(r_tl[(lvt >> 16) & 0xff]);
         if (c1 - c0 < WAVE || (lvt & (LV_SWAP | LV_PAT | 0xff)) != L) break;
-        const int lt = kind == TM_K_NEW_DST ? TM_L_OUT
-                       : (kind == TM_K_NEW_SRC ? TM_L_IN : ((lvt & LV_DIR) ? TM_L_INPAIR : TM_L_OUTPAIR));
-        const int *stl = g.stf + (size_t)(lt * TM_NTFIRST) * (size_t)g.E;
+        const int *stl = g.stf + (size_t)(lst * TM_NTFIRST) * (size_t)g.E;
         int sl = c0;
         while (!full && sl < c1) {
           int x[TM_SWEEP];
@@ -1328,13 +1301,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
       ntop = top - nparts + (last_partial ? 1 : 0);
     }
     st_steps++;
-    int dir = 0, lvw = 0;
+    int lvw = 0;
     unsigned fw = 1;  // the frame's weight (counting)
     if (has) {
       const int lv = f_lvl[myf];
       lvw = lv;
       if (T2) fw = (unsigned)f_w[myf];
-      dir = (lv >> 8) & 1;
       ridx = (lv >> 16) & 0xff;
       pend = r_pend[ridx];
       tl = r_tl[ridx];
@@ -1351,8 +1323,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     const bool swp = T2 && has && (lvw & LV_SWAP);
     if (T2 && swp) {
       cnt += (unsigned long long)fw *
-             tail2_item<SP>(g, md, m, sw_lo[myf & (WAVE - 1)], sw_hi[myf & (WAVE - 1)], dir, slot,
-                            (lvw & LV_BDIR) ? 1 : 0, (lvw >> 24) & 0xff, mt);
+             tail2_item<SP>(g, md, m, sw_lo[myf & (WAVE - 1)], sw_hi[myf & (WAVE - 1)], slot,
+                            (lvw >> 24) & 0xff, mt);
       st_leaves++;
     }
     // a pattern frame (last two edges on one list): the slot adds or removes
@@ -1366,8 +1338,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     int tfn = 0, tx = 0, node = -1;
     // position, neighbour and the next edge's first-candidate time: three
     // loads at the same slot of one list, issued together
-    const int lst = kind == TM_K_NEW_DST ? TM_L_OUT
-                    : (kind == TM_K_NEW_SRC ? TM_L_IN : (dir ? TM_L_INPAIR : TM_L_OUTPAIR));
     if (has && !swp && !patf) {
       // position, neighbour (new node); unless swept, the next edge's time and the further rules' times
       if (mt) meter.b += kind != TM_K_CLOSE ? 8 : 4;
@@ -1386,7 +1356,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         valid = !in_first(m, SP::mapped(md, j), node);
         put(m, SP::a(md, j), node);
       } else {
-        pos = dir ? g.inPairPos[slot] : g.outPairPos[slot];
+        pos = g.outPairPos[slot];
         valid = true;
       }
       if (tx > tl) valid = false;
@@ -1495,7 +1465,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         continue;
       }
     }
-    int cb = 0, ce = 0, cdir = 0, lvl = j, rw = 0, a1lo = 0, a1hi = 0, p0f = pos;
+    int cb = 0, ce = 0, lvl = j, rw = 0, a1lo = 0, a1hi = 0, p0f = pos;
     if (valid) {
       const CandList LL = cand_start<SP>(g, md, j + 1, m, pos, mt);
       cb = LL.lo;
@@ -1504,7 +1474,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         cnt += wi * leaf_count<SP>(g, md, j + 1, m, LL, pos, pend, args.scan_max, skipx, zmk, mt);
         st_leaves++;
       } else {
-        cdir = LL.dir;
         ce = gallop_lb(LL.pos, LL.lo, LL.hi, pend, mt);
       }
       valid = ce > cb;
@@ -1526,7 +1495,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         p0f = g.outPairPos[cb];
         const CandList L2 = cand_start<SP>(g, md, 2, m, p0f, mt);
         cb = L2.lo;
-        cdir = L2.dir;
         ce = gallop_lb(L2.pos, L2.lo, L2.hi, pend, mt);
         valid = ce > cb;
       }
@@ -1542,13 +1510,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         st_leaves++;
         if (pat == TP_SAME) valid = false; else swc = LV_PAT;
       } else if (ce - cb >= args.t2_min && tail2_ok<SP>(md)) {
-        int blo, bhi, bdir;
+        int blo, bhi;
         if (mt) meter.b += 4;
         const int kn = SP::kind(md, j + 1);
-        const int *ap = kn == TM_K_NEW_DST ? g.outPos : (kn == TM_K_NEW_SRC ? g.inPos : (cdir ? g.inPairPos : g.outPairPos));
-        tail2_range<SP>(g, md, m, ap[cb], pend, &blo, &bhi, &bdir, mt);
+        const int *ap = kn == TM_K_NEW_DST ? g.outPos : (kn == TM_K_NEW_SRC ? g.inPos : g.outPairPos);
+        tail2_range<SP>(g, md, m, ap[cb], pend, &blo, &bhi, mt);
         if (2 * (bhi - blo) < ce - cb) {
-          swc = LV_SWAP | (bdir ? LV_BDIR : 0);
+          swc = LV_SWAP;
           t2lo = cb; t2hi = ce;
           cb = blo; ce = bhi;
           valid = ce > cb;
@@ -1563,7 +1531,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
       if (top + n > FR) { if (lane == 0) atomicOr(&sched->error, 1); break; }
       if (valid) {
         const int w = top + __popcll(bm & lt_mask);
-        f_cur[w] = cb; f_end[w] = ce; f_lvl[w] = lvl | (cdir << 8) | swc | rw | (ridx << 16) | (zm << 24);
+        f_cur[w] = cb; f_end[w] = ce; f_lvl[w] = lvl | swc | rw | (ridx << 16) | (zm << 24);
         if (T2 && (swc & (LV_SWAP | LV_R1))) { sw_lo[w & (WAVE - 1)] = t2lo; sw_hi[w & (WAVE - 1)] = t2hi; }
         if (T2) {
           f_w[w] = (int)(unsigned)wi;

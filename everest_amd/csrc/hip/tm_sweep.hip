@@ -151,7 +151,7 @@ __global__ __launch_bounds__(256) void pair_sweep_kernel(tm_graph_view g, const 
   const int *L2R = it.d2 ? g.outR : g.inR;
   const int *L2P = it.d2 ? g.outPos : g.inPos;
   const int *L2N = it.d2 ? g.outNbr : g.inNbr;
-  const int *pp = g.outPairPos, *pn = g.outPairNbr;
+  const int *pp = g.outPairPos;
   constexpr int kScan = 32;
   unsigned long long acc = 0;
   for (long long gi = (long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); gi < groups; gi += wstride) {
@@ -165,8 +165,7 @@ __global__ __launch_bounds__(256) void pair_sweep_kernel(tm_graph_view g, const 
       v = e.v;
       if (u != v) {
         const int k = g.outPairSelf[r];
-        s0 = lower_bound_i(pn, g.outR[u], k, v);
-        s1e = upper_bound_i(pn, k + 1, g.outR[u + 1], v);
+        tmk::pair_find(g, u, v, &s0, &s1e);
         const int clip = pp[lower_bound_i(pp, k, s1e, pend_of(g, (long long)e.t + delta)) - 1];
         int lo = r;
         if (k > s0 && pp[k - 1] >= beg) {

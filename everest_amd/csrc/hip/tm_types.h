@@ -7,6 +7,16 @@
 #define TM_MAXE 8  // most motif edges handled (the reference register stack: 8-bit stackio)
 #define TM_MAXN 8  // most motif nodes handled
 
+// Pair table hash of a graph pair (multiply and fold; any fixed mix would do).
+#ifdef __HIPCC__
+__host__ __device__
+#endif
+static inline unsigned tm_pair_hash(int x, int y) {
+  unsigned h = (unsigned)x * 0x9e3779b1u + (unsigned)y;
+  h = (h ^ (h >> 15)) * 0x85ebca6bu;
+  return h ^ (h >> 13);
+}
+
 // How motif edge j (j >= 1) extends a partial match.
 enum {
   TM_K_NEW_DST = 0,  // src a mapped, dst b new: candidates = out-list of m[a]
@@ -63,7 +73,12 @@ typedef struct {
   const int *outR, *outPos, *outNbr;  // out CSR: offsets, positions (outEdgesV), destinations
   const int *inR, *inPos, *inNbr;     // in CSR: offsets, positions (inEdgesV), sources
   const int *outPairNbr, *outPairPos; // per node, out-list re-sorted by (dst, position)
-  const int *inPairNbr, *inPairPos;   // per node, in-list re-sorted by (src, position)
+  // The pair table: open addressing by tm_pair_hash, linear probing, pmask + 1
+  // entries (a power of two, at least twice the distinct pairs) of 4 ints:
+  // {x, y, s0, s1}, the pair x -> y holding slots [s0, s1) of the pair index;
+  // x = -1: empty
+  const int *ptab;
+  unsigned pmask;
   const int *outSelf;     // slot of position p in out(src of p)
   const int *inSelf;      // slot of position p in in(dst of p)
   const int *outNext;     // first slot of out(dst of p) with position > p
@@ -95,7 +110,7 @@ typedef struct {
 } tm_graph_view;
 
 // Candidate lists, in the order of stf
-enum { TM_L_OUT = 0, TM_L_IN = 1, TM_L_OUTPAIR = 2, TM_L_INPAIR = 3 };
+enum { TM_L_OUT = 0, TM_L_IN = 1, TM_L_OUTPAIR = 2 };
 
 typedef struct {
   tm_motif_dev m;
