@@ -248,6 +248,7 @@ __global__ void reset_kernel(tm_sched *s, unsigned long long *counts, int *stops
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < TM_STRIPES) {
     st_dev(&s->stripe[i].next, 0);
+    st_dev(&s->stripe[i].hungry, 0);
     st_dev(&s->stripe[i].busy, (grid + TM_STRIPES - 1 - i) / TM_STRIPES);  // every wavefront starts out holding (root) work
   }
   if (i == 0) {
@@ -526,8 +527,11 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
     wpe = h >= 6 ? 6 : h == 5 ? 5 : h == 4 ? 4 : 1;
   }
   if (!fn && wpe == 0) {
-    wpe = 5;  // measured best on the 64M-edge set over 15 heavy queries (5: 7.00 s, 6: 7.81 s, 1: 7.68 s);
-              // the autotuner picks 6 per shape where it wins
+    // 4 edges and more: 128 VGPRs, 16 wavefronts per CU (their LDS stack allows
+    // about that many anyway); 3 edges: 96 VGPRs, 20 per CU.  12 queries of 4
+    // to 6 edges: 115 ms with 4, 124 with 5, 130 with 6; 2 of 3 edges: 12.0 ms
+    // with 5, 13.4 with 4
+    wpe = lvls >= 2 ? 4 : 5;
   }
   auto blocks_of = [&](int lds_bytes, int *blocks) -> tm_status {
     if (fn) {
@@ -630,7 +634,8 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
     a.steal_after_ticks = us * g->wall_rate_khz / 1000;
   }
   // two-edge tail: frames of edge M-2 with at least this many window candidates
-  a.t2_min = (tune && tune->tail_swap < 0) ? 0x7fffffff : ((tune && tune->tail_swap > 0) ? tune->tail_swap : 32);
+  // (14 queries: 123.7 ms from 2 on, 125.4 from 8, 132.1 from 32)
+  a.t2_min = (tune && tune->tail_swap < 0) ? 0x7fffffff : ((tune && tune->tail_swap > 0) ? tune->tail_swap : 2);
   sl.last_claim = claim_blocks;
   sl.last_grid = grid;
   sl.last_lds = lds;

@@ -742,7 +742,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
   int top = 0;
   // (a launch has at most 2^30 blocks: blocks of fewer than 1024 roots are only
   // taken while there are few)
-  int claim_next = 0, claim_end = 0;        // blocks of the current claim not yet started
+  int claim_next = 0, claim_end = 0;        // blocks of the current claim not yet started, as indexes
+  int claim_k = 0;                          // into the blocks of this stripe
   int qb0 = 0, qb1 = 0;                     // blocks of the current query
   int ublk = -1;           // first root of the block being dispatched (-1: none)
   unsigned umask = 0;      // this lane's roots of the block still to expand: bit 4 k + i is root
@@ -756,8 +757,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
   const int home_stripe = blockIdx.x & (TM_STRIPES - 1);
   int cstripe = home_stripe;  // the stripe that counts this wavefront's busy credit
   int at_stripe = home_stripe;  // the stripe it claims from
+  // The blocks go to the stripes in turn, a 64th of them at a time: a stripe's
+  // wavefronts (one XCD's) work close to each other in time, where hubs'
+  // windows overlap in its L2 (single blocks in turn: 28% slower for
+  // 0->1, 1->2, 2->3 on 2M hub edges), and a busy period is shared by all.
+  const int nblocks = (int)args.total_blocks, seg = max(1, nblocks / (8 * TM_STRIPES));
   bool scout = false;           // looks at the other stripes and may wait for donations
-  long long task_t0 = 0;   // wall clock when the current task (root group or donated frame) began
+  long long look_t0 = work_t0;  // wall clock when it last looked for idle wavefronts, or took its work
+  bool told = false;       // told the stripes that it waits
   bool is_idle = false;    // gave up its busy credit (sched->busy starts at the grid size)
   bool waiter = false;     // counted in sched->waiters
   int sbn = 0;             // survivors buffered (uniform)
@@ -771,6 +778,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     if (f == 3) return &f_end[w];
     if (T2 && f == 4) return &f_p0[w];
     if (T2 && f == 7 + TM_MAXN) return &f_w[w];
+    if (T2 && f == 8 + TM_MAXN) return &r_alo[(f_lvl[w] >> 16) & 0xff];
+    if (T2 && f == 9 + TM_MAXN) return &r_ahi[(f_lvl[w] >> 16) & 0xff];
+    if (T2 && f == 10 + TM_MAXN) return &sw_lo[w & (WAVE - 1)];
+    if (T2 && f == 11 + TM_MAXN) return &sw_hi[w & (WAVE - 1)];
     if (f == 5) return &r_pend[(f_lvl[w] >> 16) & 0xff];
     if (f == 6) return &r_tl[(f_lvl[w] >> 16) & 0xff];
     if (f >= 7 && f < 7 + MAXN) return &f_m[(f - 7) * FR + w];
@@ -789,7 +800,98 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
       // enumeration cap reached by others: drop the subtrees in flight too
       if (ENUM && top > 0 && uni(ld_rlx(args.queries[qcur].stop))) top = 0;
     }
-    if (top == 0 && sbn == 0 && roots_done) {
+    // ---------------------------------------------- donate to idle wavefronts
+    // a wavefront with work looks every steal_every steps, and at most every
+    // steal_after_ticks, whether its stripe has been told of idle ones
+    bool look = false;
+    if ((top > 0 || claim_next < claim_end) && --steal_cd <= 0) {
+      steal_cd = args.steal_every;
+      const long long now = (long long)wall_clock64();
+      if (now - look_t0 > args.steal_after_ticks) {
+        look_t0 = now;
+        look = uni(ld_rlx(&sched->stripe[home_stripe].hungry)) != 0;
+      }
+    }
+    if (look) {
+      // donate only against unmet demand: tickets drawn minus records reserved
+      int want = 0;
+      if (lane == 0) {
+        const int hd = (int)ld_rlx(&sched->pool_head);
+        const int tl = (int)ld_rlx(&sched->pool_tail);
+        want = min(hd - tl, args.steal_max);
+      }
+      want = uni(__shfl(want, 0));
+      for (int d = 0; d < want; d++) {
+        // half of the claimed root blocks left, else the upper half of the
+        // shallowest frame that is large enough: 2 * steal_min candidates
+        // where each is counted at once, a sixteenth of that where each has a
+        // subtree
+        const int nb = claim_end - claim_next;
+        const int give = claim_next < claim_end ? (top > 0 || ublk >= 0 ? (nb + 1) / 2 : nb / 2) : 0;
+        int b = -1;
+        if (give == 0) {
+          if (top == 0) break;
+          const int leafl = SP::M(args.queries[qcur].m) - (ENUM ? 2 : 3);  // level whose candidates are counted at once
+          bool can = false;
+          if (lane < top) {
+            const int lv = f_lvl[lane] & 0xff;
+            const int mn = lv >= leafl ? args.steal_min : max(1, args.steal_min >> 4);
+            can = f_end[lane] - f_cur[lane] >= 2 * mn;
+          }
+          const unsigned long long cm = __ballot(can);
+          if (cm == 0ull) break;
+          b = __ffsll((long long)cm) - 1;
+        }
+        unsigned t = 0;
+        int ok = 1;
+        if (lane == 0) {
+          add_rlx(&sched->stripe[cstripe].busy, 1);  // the record's credit, before it can be seen
+          t = atomicAdd(&sched->pool_tail, 1u);
+          const unsigned lap = t >> args.pool_shift;
+          if (lap > 0) {
+            // the slot's previous lap must have been copied out by its taker
+            // (a resident wavefront holding that ticket, so this wait ends)
+            const unsigned prev = pool_tag(gen, lap - 1);
+            unsigned w = 0;
+            while (ld_rlx32(args.pool_done + (t & (unsigned)(args.pool_cap - 1))) != prev) {
+              if (ld_rlx(&sched->abort) || ++w > (1u << 24)) { ok = 0; break; }
+              __builtin_amdgcn_s_sleep(8);
+            }
+            if (!ok) {
+              // record t will never be written, so its ticket holder could
+              // only leave through the abort flag: raise it, and every
+              // wavefront (waiting ones included) leaves; the host reports
+              // the error bit as a failed launch
+              atomicOr(&sched->error, 8);
+              atomicOr(&sched->abort, 1);
+            }
+          }
+        }
+        t = (unsigned)uni((int)__shfl((int)t, 0));
+        if (!uni(__shfl(ok, 0))) break;  // abort: leave the donation loop; the main loop sees the flag
+        const int mid = b >= 0 ? uni(f_cur[b] + (f_end[b] - f_cur[b]) / 2) : claim_end - give;
+        const unsigned tag = pool_tag(gen, t >> args.pool_shift);
+        unsigned long long *rec = args.pool + (size_t)(t & (unsigned)(args.pool_cap - 1)) * TM_POOL_FIELDS;
+        if (lane < TM_POOL_FIELDS) {
+          int v = 0;
+          if (lane == 0) v = qcur | (cstripe << 16);
+          else if (lane == 2) v = mid;
+          else if (b < 0) v = lane == 1 ? TM_REC_ROOTS : (lane == 3 ? claim_end : claim_k);
+          else {
+            int *src = frame_field(lane, b);
+            v = src ? *src : 0;
+          }
+          st_rlx(rec + lane, ((unsigned long long)tag << 32) | (unsigned)v);
+        }
+        __syncthreads();
+        if (b < 0) claim_end = uni(mid);
+        else if (lane == 0) f_end[b] = mid;
+        st_don++;
+        __syncthreads();
+      }
+      claim_end = uni(claim_end);
+    }
+    if (top == 0 && sbn == 0 && roots_done && ublk < 0 && claim_next >= claim_end) {
       // ------------------------------------------ idle: take donated work
       // Ticket protocol: an idle wavefront draws ticket t (one atomic on
       // pool_head) and waits for record t.  Donors fill records in order
@@ -826,6 +928,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
           break;
         }
         waiter = true;
+        if (!told && lane < TM_STRIPES) st_rlx32((unsigned *)&sched->stripe[lane].hungry, 1u);
+        told = true;
       }
       unsigned ticket = 0;
       if (lane == 0) ticket = atomicAdd(&sched->pool_head, 1u);
@@ -841,7 +945,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         const bool mine = lane >= TM_POOL_FIELDS || (unsigned)(word >> 32) == tag;
         fv = (int)(unsigned)(word & 0xffffffffull);
         if (__ballot(!mine) == 0ull) { got = true; break; }
-        if ((spin & 3u) == 3u) {
+        // (every waiting wavefront reads the busy counters' 8 lines: seldom, but soon at first)
+        if ((spin & 15u) == 15u || spin == 3u || spin == 7u) {
           int ab = 0;
           const int b = lane < TM_STRIPES ? ld_rlx(&sched->stripe[lane].busy) : 0;
           if (lane == 0) {
@@ -877,15 +982,21 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         cnt = 0;
         qcur = fq;
       }
+      look_t0 = work_t0;
+      if (uni(__shfl(fv, 1)) == TM_REC_ROOTS) {
+        claim_next = uni(__shfl(fv, 2));
+        claim_end = uni(__shfl(fv, 3));
+        claim_k = uni(__shfl(fv, 4));
+        continue;
+      }
       // the taken frame becomes frame 0, its window root entry TM_ROOTS - 1
-      if (lane == 1) f_lvl[0] = (fv & 0xffff) | ((TM_ROOTS - 1) << 16);
+      if (lane == 1) f_lvl[0] = (fv & ~0xff0000) | ((TM_ROOTS - 1) << 16);
       __syncthreads();
       if (lane < TM_POOL_FIELDS && lane != 1) {
         int *dst = frame_field(lane, 0);
         if (dst) *dst = fv;
       }
       top = 1;
-      task_t0 = (long long)wall_clock64();
       __syncthreads();
       continue;
     }
@@ -912,15 +1023,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         if (ublk < 0) {
           if (claim_next >= claim_end) {
             bool got = false;
-            while (!got) {
-              // claim `idx` of stripe k's blocks [k B / S, (k + 1) B / S): the
-              // first of each of its wavefronts by their order, the others by
-              // one atomic.  Rounds of one claim per wavefront share half of
+            while (!got && !roots_done) {
+              // claim `idx` of stripe k's blocks: the first of each of its
+              // wavefronts by their order, the others by one atomic.  Rounds of one claim per wavefront share half of
               // the blocks left, down to single blocks; a caller's fixed size
               // is one round.
               const int k = at_stripe;
-              const int sb = (int)(args.total_blocks * k / TM_STRIPES);
-              const int size = (int)(args.total_blocks * (k + 1) / TM_STRIPES) - sb;
+              const int size = nblocks / (TM_STRIPES * seg) * seg +
+                               min(max(nblocks % (TM_STRIPES * seg) - k * seg, 0), seg);
               const int own = ((int)gridDim.x + TM_STRIPES - 1 - k) / TM_STRIPES;  // the stripe's wavefronts
               const int nw = max(1, own);
               int idx = blockIdx.x / TM_STRIPES;
@@ -942,8 +1052,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
               }
               const long long at = start + (long long)idx * n;
               if (at < size) {
-                claim_next = sb + (int)at;
-                claim_end = sb + (int)min(at + n, (long long)size);
+                claim_k = k;
+                claim_next = (int)at;
+                claim_end = (int)min(at + n, (long long)size);
                 got = true;
                 break;
               }
@@ -960,7 +1071,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
             }
             if (!got) { roots_done = true; break; }
           }
-          const int b = claim_next++;
+          const int b = (claim_next / seg * TM_STRIPES + claim_k) * seg + claim_next % seg;
+          claim_next++;
           if (b < qb0 || b >= qb1) {
             // the block's query: the last q with block_prefix[q] <= b (uniform search)
             int lo = 0, hi = MULTI ? args.nq : 1;
@@ -1099,7 +1211,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
           valid = (pend - r - 1) >= (M - 1);
         }
       }
-      task_t0 = (long long)wall_clock64();
     } else {
     // ------------------------------------------------------ expansion step
     const tm_query_dev &q = args.queries[qcur];
@@ -1557,78 +1668,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
       if (j > 0) st_push += n;
       top += n;
       __syncthreads();
-    }
-    // ---------------------------------------------- donate to idle wavefronts
-    // every steal_every steps; only a wavefront that has held its current
-    // task for steal_after_ticks donates: short tasks never pay for the exchange
-    bool look = false;
-    if (top > 0 && --steal_cd <= 0) {
-      steal_cd = args.steal_every;
-      look = (long long)wall_clock64() - task_t0 > args.steal_after_ticks;
-    }
-    if (look) {
-      // donate only against unmet demand: tickets drawn minus records reserved
-      int want = 0;
-      if (lane == 0) {
-        const int hd = (int)ld_rlx(&sched->pool_head);
-        const int tl = (int)ld_rlx(&sched->pool_tail);
-        want = min(hd - tl, args.steal_max);
-      }
-      want = uni(__shfl(want, 0));
-      for (int d = 0; d < want; d++) {
-        // split the shallowest frame with at least 2 * steal_min candidates left
-        // (a swapped frame keeps its edge M-2 range in this wavefront's side table: not donated)
-        const bool can = lane < top && !(f_lvl[lane] & (LV_SWAP | LV_RW | LV_R1)) &&
-                         (f_end[lane] - f_cur[lane] >= 2 * args.steal_min);
-        const unsigned long long cm = __ballot(can);
-        if (cm == 0ull) break;
-        const int b = __ffsll((long long)cm) - 1;
-        unsigned t = 0;
-        int ok = 1;
-        if (lane == 0) {
-          add_rlx(&sched->stripe[cstripe].busy, 1);  // the record's credit, before it can be seen
-          t = atomicAdd(&sched->pool_tail, 1u);
-          const unsigned lap = t >> args.pool_shift;
-          if (lap > 0) {
-            // the slot's previous lap must have been copied out by its taker
-            // (a resident wavefront holding that ticket, so this wait ends)
-            const unsigned prev = pool_tag(gen, lap - 1);
-            unsigned w = 0;
-            while (ld_rlx32(args.pool_done + (t & (unsigned)(args.pool_cap - 1))) != prev) {
-              if (ld_rlx(&sched->abort) || ++w > (1u << 24)) { ok = 0; break; }
-              __builtin_amdgcn_s_sleep(8);
-            }
-            if (!ok) {
-              // record t will never be written, so its ticket holder could
-              // only leave through the abort flag: raise it, and every
-              // wavefront (waiting ones included) leaves; the host reports
-              // the error bit as a failed launch
-              atomicOr(&sched->error, 8);
-              atomicOr(&sched->abort, 1);
-            }
-          }
-        }
-        t = (unsigned)uni((int)__shfl((int)t, 0));
-        if (!uni(__shfl(ok, 0))) break;  // abort: leave the donation loop; the main loop sees the flag
-        const int cur0 = f_cur[b], end0 = f_end[b];
-        const int mid = cur0 + (end0 - cur0) / 2;
-        const unsigned tag = pool_tag(gen, t >> args.pool_shift);
-        unsigned long long *rec = args.pool + (size_t)(t & (unsigned)(args.pool_cap - 1)) * TM_POOL_FIELDS;
-        if (lane < TM_POOL_FIELDS) {
-          int v = 0;
-          if (lane == 0) v = qcur | (cstripe << 16);
-          else if (lane == 2) v = mid;
-          else {
-            int *src = frame_field(lane, b);
-            v = src ? *src : 0;
-          }
-          st_rlx(rec + lane, ((unsigned long long)tag << 32) | (unsigned)v);
-        }
-        __syncthreads();
-        if (lane == 0) f_end[b] = mid;
-        st_don++;
-        __syncthreads();
-      }
     }
   }
 

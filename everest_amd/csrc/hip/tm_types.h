@@ -130,7 +130,8 @@ typedef struct {
     int next;                 // claims after the wavefronts' first ones
     int pad0[15];
     int busy;                 // wavefronts holding work + records reserved and not yet taken
-    int pad1[15];
+    int hungry;               // set once wavefronts wait for donations
+    int pad1[14];
   } stripe[TM_STRIPES];
   int error;        // bit 0: frame stack overflow, bit 1: empty frame, bit 2: deadline passed,
                     // bit 3: a donated frame never became ready
@@ -159,7 +160,10 @@ typedef struct {
 // goes to slot r mod pool_cap with tag (launch generation, lap r / pool_cap),
 // and its taker stores that tag into pool_done[slot] once the frame is
 // copied out, which lets the slot's next lap be written.
+// A record may also carry root blocks: its level word is TM_REC_ROOTS, cur and
+// end are indexes into the blocks of the stripe in the next field.
 #define TM_POOL_FIELDS 23
+#define TM_REC_ROOTS 0xff
 #define TM_GEN_BITS 18  // launch generations cycle through 1 .. 2^18 - 1
 
 enum {

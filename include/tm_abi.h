@@ -70,11 +70,11 @@ typedef struct tm_tuning {
   int32_t steal_every;   /* busy wavefronts look for idle ones every this many steps */
   int32_t steal_max;     /* frames a busy wavefront donates per look */
   int32_t steal_min;     /* a donated half-frame holds at least this many candidates */
-  int32_t steal_after_us; /* a wavefront donates only after holding one task this long */
+  int32_t steal_after_us; /* a wavefront with work looks for idle ones at most this often */
   int32_t waves_per_simd_hint; /* counting kernel variant: 1 = compiler's register allocation,
                                   4 = capped at 128 VGPRs (16 wavefronts per CU, no spills),
                                   5 = capped at 96 VGPRs (20 per CU), 6 = capped at 80 VGPRs
-                                  (24 per CU); 0 = 5 */
+                                  (24 per CU); 0 = 4 for motifs of 4 edges and more, else 5 */
   int32_t sb_flush;      /* counting: candidates that pass the filters of one level are buffered in
                             LDS and expanded together once this many (1..64) are held; -1 = each
                             step expands its own survivors; 0 = the library's choice */
@@ -83,7 +83,7 @@ typedef struct tm_tuning {
   int32_t tail_swap;     /* counting, two-edge tail: when the last motif edge does not touch the node the
                             second-to-last one brings, a partial match whose second-to-last edge has at
                             least this many candidates in the window is counted over the last edge's
-                            candidates instead, if those are fewer; 0 = library default (32), < 0 = never */
+                            candidates instead, if those are fewer; 0 = library default (2), < 0 = never */
   int32_t batch_mode;    /* tm_batch_count: 0 = one single-query launch per query, back to back on one
                             stream, one synchronization; 1 = one multi-query launch per shape class;
                             2 = every query of the call in one multi-query launch (its stack sized for

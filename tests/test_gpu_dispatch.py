@@ -37,3 +37,34 @@ def test_root_ranges(E):
             print("E", E, "batch", tune, flush=True)
             assert dg.batch_count(qs, tune=abi.tuning(**tune)) == want, tune
     dg.close()
+
+
+# repeated root pair (weights by rank), repeated new pair (weights by slot), two-edge tails summed over the
+# last edge's list, a star's pattern, plain frames
+DONATED = [[(0, 1, 0), (0, 1, 1), (0, 2, 2), (2, 3, 3)], [(0, 1, 0), (0, 2, 1), (0, 2, 2), (3, 2, 3)],
+           [(0, 1, 0), (0, 2, 1), (2, 1, 2)], [(0, 1, 0), (1, 2, 1), (0, 3, 2), (1, 0, 3)],
+           [(0, 1, 0), (0, 2, 1), (0, 3, 2), (0, 4, 3)], [(0, 1, 0), (1, 2, 1), (2, 3, 2), (3, 0, 3)]]
+
+
+@pytest.mark.parametrize("mot", DONATED)
+def test_donated_frames_and_blocks(mot):
+    """A few wavefronts that give away root blocks and frames of every kind at each look, to the last
+    candidate: the count stays the oracle's, and what is given is taken."""
+    from everest_amd import abi
+    rng = np.random.default_rng(5)
+    E = 6000
+    U, V, T = random_graph(rng, E, 60, 40_000)
+    g = prep.preprocess(U, V, T)
+    dg = abi.DeviceGraph.from_dict(g)
+    want = oracle.count(g, mot, 2500, nthreads=4)
+    donated = 0
+    for tune in (dict(waves_per_cu=1, steal_min=1), dict(steal_min=1, claim_blocks=8), dict(steal_min=16, tail_swap=1)):
+        for _ in range(3):
+            print("motif", mot, tune, flush=True)
+            assert dg.count(mot, 2500, tune=abi.tuning(steal_after_us=1, steal_every=1, steal_max=4, **tune)) == want
+            st = dg.last_stats()
+            assert st["donated"] == st["taken"]
+            donated += st["donated"]
+    print("donated", donated)
+    assert donated > 0
+    dg.close()
