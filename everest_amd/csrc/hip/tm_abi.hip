@@ -238,14 +238,17 @@ __device__ __forceinline__ int ld_dev(const int *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// the error bits of the launch just finished, kept for the caller (a batch
-// of single-query launches checks every launch's bits at the end)
-__global__ void error_kernel(const tm_sched *s, int *out) {
-  if (threadIdx.x == 0) *out = ld_dev(&s->error);
-}
-
-__global__ void reset_kernel(tm_sched *s, unsigned long long *counts, int *stops, int n, int grid) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
+// Before a launch: its queries, query table and block prefix from pinned host
+// memory, and the scheduler state, counts and stop flags cleared.  One kernel
+// instead of three copies and a kernel (each copy of a few hundred bytes kept
+// the host for about 10 us).
+__global__ void __launch_bounds__(256) stage_kernel(tm_sched *s, unsigned long long *counts, int *stops, int n, int grid,
+                                                    const int *h_queries, int *queries, const int *h_qtab, int *qtab,
+                                                    const int *h_prefix, int *prefix) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+  for (int k = i; k < n * (int)(sizeof(tm_query_dev) / 4); k += stride) queries[k] = h_queries[k];
+  for (int k = i; k < 4 * n; k += stride) qtab[k] = h_qtab[k];
+  for (int k = i; k < 2 * (n + 1); k += stride) prefix[k] = h_prefix[k];
   if (i < TM_STRIPES) {
     st_dev(&s->stripe[i].next, 0);
     st_dev(&s->stripe[i].hungry, 0);
@@ -257,12 +260,13 @@ __global__ void reset_kernel(tm_sched *s, unsigned long long *counts, int *stops
     st_dev(&s->pool_head, 0u);
     st_dev(&s->pool_tail, 0u);
     st_dev(&s->waiters, 0);
+    st_dev(&s->summed, 0);
     // fresh ring tags for this launch (the host clears the ring before 2^18)
     __hip_atomic_fetch_add(&s->gen, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(&s->t0, (long long)wall_clock64(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   if (i < 16) st_dev(&s->stats[i], 0ull);
-  if (i < n) { st_dev(&counts[i], 0ull); st_dev(&stops[i], 0); }
+  for (int k = i; k < n; k += stride) { st_dev(&counts[k], 0ull); st_dev(&stops[k], 0); }
 }
 
 __global__ void clear_pool_kernel(unsigned long long *pool, size_t nw, unsigned *done, size_t nd, tm_sched *s) {
@@ -272,19 +276,35 @@ __global__ void clear_pool_kernel(unsigned long long *pool, size_t nw, unsigned 
   if (i == 0) __hip_atomic_store(&s->gen, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // next reset: 1
 }
 
-// Sum the per-wavefront counters of a launch into sched->stats (one block).
-__global__ void __launch_bounds__(256) stats_kernel(const unsigned long long *__restrict__ w, int grid, tm_sched *s) {
+// After a launch: the per-wavefront counters summed over several blocks (one
+// block took 60 us for 4,096 wavefronts' 128-byte slots), and by the last of
+// them the sums, the error bits and the counts written to pinned host memory.
+constexpr int kFinishWaves = 64;  // wavefronts' slots per block, at most 64 blocks
+__global__ void __launch_bounds__(256) finish_kernel(const unsigned long long *__restrict__ w, int grid, tm_sched *s,
+                                                     const unsigned long long *counts, int n, unsigned long long *h_counts,
+                                                     int *h_error, unsigned long long *h_stats) {
   __shared__ unsigned long long acc[256];
+  __shared__ int last;
   const int k = threadIdx.x % TM_NSTATS, part = threadIdx.x / TM_NSTATS;  // 16 partial sums per counter
   unsigned long long v = 0;
-  for (int b = part; b < grid; b += 256 / TM_NSTATS) v += w[(size_t)b * TM_NSTATS + k];
+#pragma unroll 4
+  for (int b = blockIdx.x * 16 + part; b < grid; b += gridDim.x * 16) v += w[(size_t)b * TM_NSTATS + k];
   acc[threadIdx.x] = v;
   __syncthreads();
   if (threadIdx.x < TM_NSTATS) {
     unsigned long long t = 0;
     for (int p = 0; p < 256 / TM_NSTATS; p++) t += acc[p * TM_NSTATS + threadIdx.x];
-    s->stats[threadIdx.x] = t;
+    if (t) __hip_atomic_fetch_add(&s->stats[threadIdx.x], t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
+  __syncthreads();
+  if (threadIdx.x == 0)
+    last = __hip_atomic_fetch_add(&s->summed, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
+  __syncthreads();
+  if (!last) return;
+  if (threadIdx.x < TM_NSTATS)
+    h_stats[threadIdx.x] = __hip_atomic_load(&s->stats[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (threadIdx.x == 0) *h_error = ld_dev(&s->error);
+  for (int q = threadIdx.x; q < n; q += blockDim.x) h_counts[q] = counts[q];
 }
 
 int ceil_log2(long long x) {
@@ -541,7 +561,17 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
       *blocks = b;
       return TM_OK;
     }
-    return dispatch<true>(sl, nmap, enumerate, instr, wpe, multi, lds_bytes, blocks, nullptr, 0);
+    for (const auto &o : g->occ)
+      if (o.nmap == nmap && o.enumerate == (int)enumerate && o.instr == instr && o.wpe == wpe &&
+          o.multi == (int)multi && o.lds == lds_bytes) {
+        *blocks = o.blocks;
+        return TM_OK;
+      }
+    tm_status os = dispatch<true>(sl, nmap, enumerate, instr, wpe, multi, lds_bytes, blocks, nullptr, 0);
+    if (os != TM_OK) return os;
+    if (g->occ.size() >= TM_OCC_MAX) g->occ.clear();
+    g->occ.push_back({nmap, (int)enumerate, instr, wpe, (int)multi, lds_bytes, *blocks});
+    return TM_OK;
   };
   int lds = lds_of(sb_flush);
   int blocks = 0;
@@ -591,13 +621,6 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
   // a caller's claim size counts 256 roots; the library's own shrinks with the blocks left
   const int claim_blocks =
       (tune && tune->claim_blocks > 0) ? std::max(1, (int)(((long long)tune->claim_blocks << 8) >> unit_shift)) : 0;
-
-  HIPTRY(hipMemcpyAsync(s.d_queries + q0, s.h_queries.data() + q0, sizeof(tm_query_dev) * nq,
-                        hipMemcpyHostToDevice, sl.stream));
-  HIPTRY(hipMemcpyAsync(s.d_qtab + 4 * (size_t)q0, s.h_qtab.data() + 4 * (size_t)q0, sizeof(int) * 4 * nq,
-                        hipMemcpyHostToDevice, sl.stream));
-  HIPTRY(hipMemcpyAsync(s.d_prefix + q0, s.h_prefix.data() + q0, sizeof(long long) * (nq + 1),
-                        hipMemcpyHostToDevice, sl.stream));
 
   tm_kernel_args a;
   memset(&a, 0, sizeof(a));
@@ -678,14 +701,18 @@ tm_status enqueue(tm_graph *g, Slot &sl, const Plan &pl, bool timing, bool count
   // the generation count belongs to the graph's slot (sl may be a view of it
   // with other staging arrays); a captured launch is counted at each replay
   if (count && (st = count_launch(g, sl.own_ring ? sl : g->slot[sl.index], sl.stream, 1)) != TM_OK) return st;
-  hipLaunchKernelGGL(reset_kernel, dim3((pl.nq + 255) / 256), dim3(256), 0, sl.stream, pl.a.sched, pl.d_counts,
-                     pl.d_stops, pl.nq, pl.grid);
+  const Scratch &sc = sl.s;
+  hipLaunchKernelGGL(stage_kernel, dim3((unsigned)std::min(64, (pl.nq + 3) / 4)), dim3(256), 0, sl.stream, pl.a.sched,
+                     pl.d_counts, pl.d_stops, pl.nq, pl.grid, (const int *)(sc.h_queries + pl.q0),
+                     (int *)const_cast<tm_query_dev *>(pl.a.queries), sc.h_qtab + 4 * (size_t)pl.q0,
+                     const_cast<int *>(pl.a.qtab), (const int *)(sc.h_prefix + pl.q0),
+                     (int *)const_cast<long long *>(pl.a.block_prefix));
   HIPTRY(hipGetLastError());
   if (timing) HIPTRY(hipEventRecord(sl.ev0, sl.stream));
   if (pl.fn) {
     if (pl.fn(1, &pl.a, pl.grid, pl.lds, sl.stream, nullptr, pl.user) != 0)
       return fail(TM_ERR_HIP, "custom kernel launch failed");
-  } else {
+  } else if (pl.a.total_blocks > 0) {  // (every query swept, or no roots: nothing to mine)
     int blocks = 0;
     if ((st = dispatch<false>(sl, pl.nmap, pl.enumerate, pl.instr, pl.wpe, pl.multi, pl.lds, &blocks, &pl.a,
                               pl.grid)) != TM_OK)
@@ -706,7 +733,10 @@ tm_status enqueue(tm_graph *g, Slot &sl, const Plan &pl, bool timing, bool count
     if ((st = pair_enqueue(g->view, pl.a.queries, b, sl.stream)) != TM_OK) return st;
   }
   if (timing) HIPTRY(hipEventRecord(sl.ev1, sl.stream));
-  hipLaunchKernelGGL(stats_kernel, dim3(1), dim3(256), 0, sl.stream, pl.a.wstats, pl.grid, pl.a.sched);
+  const int waves = pl.fn || pl.a.total_blocks > 0 ? pl.grid : 0;
+  hipLaunchKernelGGL(finish_kernel, dim3((unsigned)std::max(1, std::min(64, waves / kFinishWaves))), dim3(256), 0,
+                     sl.stream, pl.a.wstats, waves, pl.a.sched, pl.d_counts, pl.nq, sc.h_counts + pl.q0,
+                     sc.h_errors + pl.q0, sc.h_stats);
   HIPTRY(hipGetLastError());
   return TM_OK;
 }
@@ -732,6 +762,8 @@ tm_status reserve(tm_graph *g, Slot &sl, int nq) {
   int cap = std::max(nq, 256);
   void *p;
   tm_status st;
+  HIPTRY(hipStreamSynchronize(sl.stream));  // (a launch in flight would still use the old pinned side)
+  if ((st = pin_alloc(s, cap)) != TM_OK) return st;
   if ((st = dev_alloc(g, &p, sizeof(tm_query_dev) * cap)) != TM_OK) return st;
   s.d_queries = (tm_query_dev *)p;
   if ((st = dev_alloc(g, &p, sizeof(int) * 4 * cap)) != TM_OK) return st;
@@ -761,9 +793,29 @@ tm_status reserve(tm_graph *g, Slot &sl, int nq) {
     HIPTRY(hipStreamSynchronize(sl.stream));
   }
   s.cap_q = cap;
-  s.h_queries.resize(cap);
-  s.h_qtab.resize(4 * (size_t)cap);
-  s.h_prefix.resize(cap + 1);
+  return TM_OK;
+}
+
+void pin_free(Scratch &s) {
+  if (s.pin) (void)hipHostFree(s.pin);
+  s.pin = nullptr;
+}
+
+tm_status pin_alloc(Scratch &s, int cap) {
+  pin_free(s);
+  auto up = [](size_t x) { return (x + 63) / 64 * 64; };
+  const size_t o_qtab = up(sizeof(tm_query_dev) * cap), o_prefix = o_qtab + up(sizeof(int) * 4 * cap);
+  const size_t o_counts = o_prefix + up(sizeof(long long) * (cap + 1));
+  const size_t o_errors = o_counts + up(sizeof(unsigned long long) * cap);
+  const size_t o_stats = o_errors + up(sizeof(int) * cap);
+  HIPTRY(hipHostMalloc(&s.pin, o_stats + up(sizeof(unsigned long long) * TM_NSTATS)));
+  char *b = (char *)s.pin;
+  s.h_queries = (tm_query_dev *)b;
+  s.h_qtab = (int *)(b + o_qtab);
+  s.h_prefix = (long long *)(b + o_prefix);
+  s.h_counts = (unsigned long long *)(b + o_counts);
+  s.h_errors = (int *)(b + o_errors);
+  s.h_stats = (unsigned long long *)(b + o_stats);
   return TM_OK;
 }
 
@@ -797,13 +849,13 @@ tm_status stage_queries(tm_graph *g, Slot &sl, int q0, int nq, const int *idx, c
   return TM_OK;
 }
 
-// Check a completed launch of the slot: its scheduler state hs (copied back)
-// gives the launch statistics and error bits.
-tm_status collect(tm_graph *g, Slot &sl, const tm_sched &hs) {
+// Check a completed launch of the slot's queries from q0 on: its statistics
+// and error bits, as the finish kernel left them in the pinned side.
+tm_status collect(tm_graph *g, Slot &sl, int q0) {
   // the statistics land in the graph's slot of that index (sl may be a view
   // of it with other device buffers)
   Slot &dst = g->slot[sl.index];
-  memcpy(dst.last_stats, hs.stats, sizeof(hs.stats));
+  memcpy(dst.last_stats, sl.s.h_stats, sizeof(unsigned long long) * TM_NSTATS);
   dst.last_stats[TM_STAT_SWEEP] = (unsigned long long)sl.last_sweep;
   dst.last_stats[TM_STAT_GRID] = (unsigned long long)sl.last_grid;
   dst.last_stats[TM_STAT_CLAIM] = (unsigned long long)sl.last_claim;
@@ -812,20 +864,18 @@ tm_status collect(tm_graph *g, Slot &sl, const tm_sched &hs) {
   float ms = 0.f;
   if (hipEventElapsedTime(&ms, sl.ev0, sl.ev1) == hipSuccess) dst.last_kernel_ms = ms;
   g->last_slot = sl.index;
-  if (hs.error & ~4) return fail(TM_ERR_INTERNAL, "kernel invariant violated (error bits " + std::to_string(hs.error) + ")");
-  if (hs.error & 4) return fail(TM_ERR_TIMEOUT, "query exceeded its time limit; counts discarded");
+  const int error = sl.s.h_errors[q0];
+  if (error & ~4) return fail(TM_ERR_INTERNAL, "kernel invariant violated (error bits " + std::to_string(error) + ")");
+  if (error & 4) return fail(TM_ERR_TIMEOUT, "query exceeded its time limit; counts discarded");
   return TM_OK;
 }
 
 // Wait for the slot's launch of staged queries [q0, q0 + nq); copy their
 // counts out and check the launch's error bits.
 tm_status finish(tm_graph *g, Slot &sl, int q0, int nq, uint64_t *counts) {
-  Scratch &s = sl.s;
-  tm_sched hs;
-  HIPTRY(hipMemcpyAsync(&hs, s.d_sched, sizeof(hs), hipMemcpyDeviceToHost, sl.stream));
-  HIPTRY(hipMemcpyAsync(counts, s.d_counts + q0, sizeof(uint64_t) * nq, hipMemcpyDeviceToHost, sl.stream));
   HIPTRY(hipStreamSynchronize(sl.stream));
-  return collect(g, sl, hs);
+  memcpy(counts, sl.s.h_counts + q0, sizeof(uint64_t) * nq);
+  return collect(g, sl, q0);
 }
 
 // Counts of one motif over consecutive root ranges [cuts[i], cuts[i + 1])
@@ -1205,6 +1255,7 @@ tm_status tm_graph_free(tm_graph *g) {
   if (g->edge_features) (void)hipFree(g->edge_features);
   if (g->vertex_features) (void)hipFree(g->vertex_features);
   for (Slot &sl : g->slot) {
+    pin_free(sl.s);
     if (sl.ev0) (void)hipEventDestroy(sl.ev0);
     if (sl.ev1) (void)hipEventDestroy(sl.ev1);
     if (sl.stream) (void)hipStreamDestroy(sl.stream);
@@ -1438,27 +1489,21 @@ tm_status tm_batch_count(tm_graph *g, int32_t nq, const int32_t *num_edges, cons
       Slot &sq = g->slot[q % ns];
       st = stage_queries(g, sq, q, 1, &q, num_edges, msrc, mdst, TM_MAX_MOTIF_EDGES, deltas, nullptr, nullptr);
       if (st == TM_OK) st = launch(g, sq, q, 1, false, class_tuning(g, key[q], tune), 0, false);
-      if (st == TM_OK) {
-        hipLaunchKernelGGL(error_kernel, dim3(1), dim3(64), 0, sq.stream, sq.s.d_sched, sq.s.d_stops + q);
-        HIPTRY(hipGetLastError());
-      }
     }
-    std::vector<int> err(nq);
-    std::vector<uint64_t> part(nq);
-    std::vector<int> perr(nq);
-    for (int k = 0; k < ns && st == TM_OK; k++) {
+    // every launch is waited for, also when one could not be enqueued: the
+    // pinned staging is theirs until then
+    int bits = 0;
+    for (int k = 0; k < ns; k++) {
       Slot &sk = g->slot[k];
-      st = finish(g, sk, 0, nq, part.data());
-      if (st == TM_OK)
-        HIPTRY(hipMemcpy(perr.data(), sk.s.d_stops, sizeof(int) * nq, hipMemcpyDeviceToHost));
-      for (int q = k; q < nq && st == TM_OK; q += ns) {
-        counts[q] = part[q];
-        err[q] = perr[q];
+      HIPTRY(hipStreamSynchronize(sk.stream));
+      if (st != TM_OK) continue;
+      for (int q = k; q < nq; q += ns) {
+        counts[q] = sk.s.h_counts[q];
+        bits |= sk.s.h_errors[q];
       }
+      (void)collect(g, sk, (nq - 1 - k) / ns * ns + k);  // statistics of the slot's last launch
     }
     if (st != TM_OK) return st;
-    int bits = 0;
-    for (int q = 0; q < nq; q++) bits |= err[q];
     if (bits & ~4) return fail(TM_ERR_INTERNAL, "kernel invariant violated (error bits " + std::to_string(bits) + ")");
     if (bits & 4) return fail(TM_ERR_TIMEOUT, "a query exceeded its time limit; counts discarded");
     return TM_OK;

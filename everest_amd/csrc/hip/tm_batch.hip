@@ -48,8 +48,6 @@ struct tm_batch {
     std::vector<void *> mem;
   };
   std::vector<Group> groups;
-  uint64_t *h_counts = nullptr;  // pinned, staged order
-  tm_sched *h_sched = nullptr;   // pinned, one per group
   hipEvent_t fork = nullptr, join[TM_SLOTS] = {};
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -60,10 +58,10 @@ namespace {
 void release(tm_batch *b) {
   if (b->exec) (void)hipGraphExecDestroy(b->exec);
   if (b->graph) (void)hipGraphDestroy(b->graph);
-  for (auto &gr : b->groups)
+  for (auto &gr : b->groups) {
     for (void *p : gr.mem) (void)hipFree(p);
-  if (b->h_counts) (void)hipHostFree(b->h_counts);
-  if (b->h_sched) (void)hipHostFree(b->h_sched);
+    pin_free(gr.view.s);
+  }
   if (b->fork) (void)hipEventDestroy(b->fork);
   for (hipEvent_t e : b->join)
     if (e) (void)hipEventDestroy(e);
@@ -90,10 +88,8 @@ tm_status group_staging(tm_batch::Group &gr) {
   BTRY(al(&p, sizeof(int) * n));
   s.d_stops = (int *)p;
   s.cap_q = n;
-  s.h_queries.assign(n, tm_query_dev{});
-  s.h_qtab.assign(4 * (size_t)n, 0);
-  s.h_prefix.assign(n + 1, 0);
-  return TM_OK;
+  s.pin = nullptr;  // (the view's own, not the slot's it was copied from)
+  return pin_alloc(s, n);
 }
 
 }  // namespace
@@ -152,9 +148,7 @@ tm_status tm_batch_prepare(tm_graph *g, int32_t nq, const int32_t *num_edges, co
     return st;
   };
   hipError_t he;
-  if ((he = hipHostMalloc((void **)&b->h_counts, sizeof(uint64_t) * nq)) != hipSuccess ||
-      (he = hipHostMalloc((void **)&b->h_sched, sizeof(tm_sched) * b->groups.size())) != hipSuccess ||
-      (he = hipEventCreateWithFlags(&b->fork, hipEventDisableTiming)) != hipSuccess)
+  if ((he = hipEventCreateWithFlags(&b->fork, hipEventDisableTiming)) != hipSuccess)
     return fail_b(set_error(TM_ERR_HIP, std::string("batch host buffers: ") + hipGetErrorString(he)));
   for (int k = 0; k < TM_SLOTS; k++)
     if ((he = hipEventCreateWithFlags(&b->join[k], hipEventDisableTiming)) != hipSuccess)
@@ -168,6 +162,7 @@ tm_status tm_batch_prepare(tm_graph *g, int32_t nq, const int32_t *num_edges, co
     gr.view.ev0 = real.ev0;
     gr.view.ev1 = real.ev1;
     gr.view.s = real.s;  // shared state: scheduler, ring, counter slots
+    gr.view.s.pin = nullptr;
     tm_status st = group_staging(gr);
     if (st == TM_OK)
       st = stage_queries(g, gr.view, 0, gr.n, b->order.data() + gr.first, num_edges, msrc, mdst, TM_MAX_MOTIF_EDGES,
@@ -190,11 +185,6 @@ tm_status tm_batch_prepare(tm_graph *g, int32_t nq, const int32_t *num_edges, co
   for (size_t gi = 0; gi < b->groups.size() && he == hipSuccess && cst == TM_OK; gi++) {
     tm_batch::Group &gr = b->groups[gi];
     cst = enqueue(g, gr.view, gr.pl, false, false);
-    if (cst != TM_OK) break;
-    he = hipMemcpyAsync(b->h_sched + gi, gr.view.s.d_sched, sizeof(tm_sched), hipMemcpyDeviceToHost, gr.view.stream);
-    if (he == hipSuccess)
-      he = hipMemcpyAsync(b->h_counts + gr.first, gr.pl.d_counts, sizeof(uint64_t) * gr.n, hipMemcpyDeviceToHost,
-                          gr.view.stream);
   }
   for (int k = 1; k < used && he == hipSuccess && cst == TM_OK; k++) {
     he = hipEventRecord(b->join[k], g->slot[k].stream);
@@ -229,11 +219,12 @@ tm_status tm_batch_run(tm_batch *b, uint64_t *counts) {
   tm_status st = TM_OK;
   for (size_t gi = 0; gi < b->groups.size(); gi++) {
     tm_batch::Group &gr = b->groups[gi];
-    const tm_status gs = collect(g, g->slot[gr.view.index], b->h_sched[gi]);
+    const tm_status gs = collect(g, gr.view, 0);
     if (st == TM_OK) st = gs;
   }
   if (st != TM_OK) return st;
-  for (int i = 0; i < b->nq; i++) counts[b->order[i]] = b->h_counts[i];
+  for (tm_batch::Group &gr : b->groups)
+    for (int i = 0; i < gr.n; i++) counts[b->order[gr.first + i]] = gr.view.s.h_counts[i];
   return TM_OK;
 }
 

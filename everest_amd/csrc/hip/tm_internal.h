@@ -11,6 +11,7 @@
 #include "tm_types.h"
 
 #define TM_LAUNCH_MAXQ 512  // queries per launch (their table and counts live in LDS)
+#define TM_OCC_MAX 64
 #define TM_SB_FLUSH_DEFAULT 32   // counting: survivors buffered before a full-width expansion
 #define TM_SB_INLINE_DEFAULT 32  // counting: survivors a step expands itself when nothing is buffered
 
@@ -30,10 +31,21 @@ struct Scratch {
   int pool_cap = 0, pool_shift = 0;
   unsigned long long *d_wstats = nullptr; // per-wavefront counters of the last launch
   int wstats_cap = 0;                    // wavefronts they have room for
-  std::vector<tm_query_dev> h_queries;
-  std::vector<int> h_qtab;
-  std::vector<long long> h_prefix;
+  // Host side of the staging and the results: one pinned allocation (pin_alloc)
+  // that the kernels around the mining kernel read and write themselves.
+  void *pin = nullptr;
+  tm_query_dev *h_queries = nullptr;
+  int *h_qtab = nullptr;
+  long long *h_prefix = nullptr;
+  unsigned long long *h_counts = nullptr;  // per query
+  int *h_errors = nullptr;                 // error bits of the launch that starts at this query
+  unsigned long long *h_stats = nullptr;   // TM_NSTATS counters of the last launch
 };
+
+// Allocate (and release) the pinned side for cap queries; a device with no
+// launch in flight on it only.
+tm_status pin_alloc(Scratch &s, int cap);
+void pin_free(Scratch &s);
 
 // One launch lane: a stream with its own scheduler state, donation pool,
 // staging and results, so launches on different slots can run concurrently.
@@ -73,6 +85,12 @@ struct tm_graph {
   tm_tuning class_tune[TM_NCLASSES] = {};  // per shape class (autotuner), used when a call brings none
   bool class_set[TM_NCLASSES] = {};
   std::mutex mtx;            // one API call at a time per graph handle
+  // resident workgroups per CU of the launch shapes seen so far (asking the
+  // runtime takes several us); at most TM_OCC_MAX of them
+  struct Occupancy {
+    int nmap, enumerate, instr, wpe, multi, lds, blocks;
+  };
+  std::vector<Occupancy> occ;
   int *edge_features = nullptr;    // labels (tm_graph_set_features), not read by the kernels
   int *vertex_features = nullptr;
   int num_edge_features = 0, num_vertex_features = 0;
@@ -114,8 +132,9 @@ tm_status launch(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm
 // Count n launches on the slot (each advances the device generation by one),
 // clearing the ring first on `stream` if the generation would wrap.
 tm_status count_launch(tm_graph *g, Slot &sl, hipStream_t stream, int n);
-// After the slot's stream has drained: statistics and error bits of its launch.
-tm_status collect(tm_graph *g, Slot &sl, const tm_sched &hs);
+// After the slot's stream has drained: statistics and error bits of its launch
+// of the queries staged from q0 on (their counts are in s.h_counts).
+tm_status collect(tm_graph *g, Slot &sl, int q0);
 // Synchronous: wait for the slot's launch and copy out its counts.
 tm_status finish(tm_graph *g, Slot &sl, int q0, int nq, uint64_t *counts);
 // The tuning table entry of a motif's shape class (nullptr when none is set).

@@ -125,9 +125,14 @@ tm_status tm_batch_count_noalloc(tm_graph *g, int32_t nq, const int32_t *num_edg
   s.d_pool_done = (unsigned *)(ds->ptr + kOffPoolDone);
   s.pool_shift = kPoolShift;
   s.pool_cap = 1 << kPoolShift;
-  s.h_queries.resize(kMaxQ);
-  s.h_qtab.resize(4 * (size_t)kMaxQ);
-  s.h_prefix.resize(kMaxQ + 1);
+  // the slot's own pinned side (allocated with the graph, for at least kMaxQ queries)
+  if (real.s.cap_q < kMaxQ) return set_error(TM_ERR_INTERNAL, "the slot's staging is smaller than a call");
+  s.h_queries = real.s.h_queries;
+  s.h_qtab = real.s.h_qtab;
+  s.h_prefix = real.s.h_prefix;
+  s.h_counts = real.s.h_counts;
+  s.h_errors = real.s.h_errors;
+  s.h_stats = real.s.h_stats;
   // the queries by shape class, one launch per class, as tm_batch_count
   std::vector<int> key(nq), order(nq);
   for (int q = 0; q < nq; q++) {

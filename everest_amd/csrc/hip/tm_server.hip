@@ -110,8 +110,6 @@ struct Lane {  // one launch slot as the server drives it
   bool enumerate = false;
   std::vector<uint64_t> ids;
   hipEvent_t done = nullptr;
-  tm_sched *h_sched = nullptr;   // pinned
-  uint64_t *h_counts = nullptr;  // pinned, max_batch entries
 };
 
 }  // namespace
@@ -267,10 +265,7 @@ bool launch_next(tm_server *s, int k) {
   }
   if (st == TM_OK) st = launch(s->g, sl, 0, n, enumerate, tune, false, !enumerate && n > 1);
   hipError_t e = hipSuccess;
-  if (st == TM_OK) e = hipMemcpyAsync(ln.h_sched, sl.s.d_sched, sizeof(tm_sched), hipMemcpyDeviceToHost, sl.stream);
-  if (st == TM_OK && e == hipSuccess)
-    e = hipMemcpyAsync(ln.h_counts, sl.s.d_counts, sizeof(uint64_t) * n, hipMemcpyDeviceToHost, sl.stream);
-  if (st == TM_OK && e == hipSuccess) e = hipEventRecord(ln.done, sl.stream);
+  if (st == TM_OK) e = hipEventRecord(ln.done, sl.stream);
   if (st == TM_OK && e != hipSuccess) st = lane_error("server launch", e);
   if (st != TM_OK) {  // the requests fail without running
     for (uint64_t id : pick) {
@@ -297,7 +292,8 @@ bool launch_next(tm_server *s, int k) {
 void complete(tm_server *s, int k) {
   Lane &ln = s->lane[k];
   Slot &sl = s->g->slot[k];
-  const tm_status st = collect(s->g, sl, *ln.h_sched);
+  const tm_status st = collect(s->g, sl, 0);
+  const std::vector<uint64_t> counts(sl.s.h_counts, sl.s.h_counts + ln.ids.size());  // (a cut below reuses them)
   for (size_t i = 0; i < ln.ids.size(); i++) {
     Request &r = *s->reqs[ln.ids[i]];
     if (r.limited && st == TM_ERR_TIMEOUT) {
@@ -310,7 +306,7 @@ void complete(tm_server *s, int k) {
     }
     r.limited = false;
     r.status = st;
-    r.count = ln.h_counts[i];
+    r.count = counts[i];
     if (ln.enumerate) {
       if (st == TM_OK && r.cap > 0 && r.count >= (uint64_t)r.cap) {
         // at the cap: the deterministic rows, as tm_enum returns them (the
@@ -431,14 +427,10 @@ tm_status tm_server_create(tm_graph *g, const tm_server_config *cfg, tm_server *
     s->arena.init(base, s->arena_bytes);
     for (int k = 0; k < s->slots; k++) {
       Lane &ln = s->lane[k];
-      if ((e = hipEventCreateWithFlags(&ln.done, hipEventDisableTiming)) != hipSuccess ||
-          (e = hipHostMalloc((void **)&ln.h_sched, sizeof(tm_sched))) != hipSuccess ||
-          (e = hipHostMalloc((void **)&ln.h_counts, sizeof(uint64_t) * s->max_batch)) != hipSuccess) {
+      if ((e = hipEventCreateWithFlags(&ln.done, hipEventDisableTiming)) != hipSuccess) {
         for (int j = 0; j <= k; j++) {
           Lane &l2 = s->lane[j];
           if (l2.done) (void)hipEventDestroy(l2.done);
-          if (l2.h_sched) (void)hipHostFree(l2.h_sched);
-          if (l2.h_counts) (void)hipHostFree(l2.h_counts);
         }
         (void)hipFree(base);
         return lane_error("server lanes", e);
@@ -567,8 +559,6 @@ tm_status tm_server_destroy(tm_server *s) {
   for (int k = 0; k < s->slots; k++) {
     Lane &ln = s->lane[k];
     if (ln.done) (void)hipEventDestroy(ln.done);
-    if (ln.h_sched) (void)hipHostFree(ln.h_sched);
-    if (ln.h_counts) (void)hipHostFree(ln.h_counts);
   }
   if (s->arena.base) (void)hipFree(s->arena.base);
   delete s;

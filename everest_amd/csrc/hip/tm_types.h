@@ -137,7 +137,9 @@ typedef struct {
                     // bit 3: a donated frame never became ready
   int abort;        // set once the deadline passed: every wavefront stops
   long long t0;     // wall clock at launch (set by the reset kernel)
-  unsigned long long stats[16];  // work counters (see TM_STAT_*)
+  unsigned long long stats[16];  // work counters (see TM_STAT_*), summed after the launch
+  int summed;       // blocks of the finish kernel done with them
+  int pad5[31];
   // each on its own 128-byte line: donors, takers and waiters do not queue
   // behind each other's atomics
   unsigned int pool_head;  // tickets drawn by idle wavefronts
