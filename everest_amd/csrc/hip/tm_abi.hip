@@ -574,7 +574,15 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
   const int nmap = maxN <= 4 ? 4 : 8;
   // cur, end, level word, node map, positions (enumeration), weight and list start (counting)
   const bool counting = !enumerate && instr != 1;
-  const int per_frame = 3 + nmap + (enumerate ? TM_MAXE : 0) + (counting ? 2 : 0);
+  // which side tables the counting kernel needs (a caller's kernel: all)
+  int need = fn && counting ? TM_NEED_P0 | TM_NEED_RW | TM_NEED_TAIL : 0;
+  for (int i = 0; i < nq && counting; i++) {
+    const tm_motif_dev &md = s.h_queries[q0 + i].m;
+    if (tmk::root_pair_ok<tmk::DynSpec>(md)) need |= TM_NEED_RW;
+    if (tmk::pair_tail_edge<tmk::DynSpec>(md) >= 0) need |= TM_NEED_P0 | TM_NEED_TAIL;
+    if (tmk::tail2_mode<tmk::DynSpec>(md) != tmk::T2_NONE) need |= TM_NEED_TAIL;
+  }
+  const int per_frame = 3 + nmap + (enumerate ? TM_MAXE : 0) + (counting ? 1 : 0) + (need & TM_NEED_P0 ? 1 : 0);
   // survivor compaction of the counting kernel: survivors buffered before a
   // full-width expansion (0: expanded in the step that filtered them), and
   // the survivors with which a step expands its own when nothing is buffered
@@ -591,9 +599,9 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
   // ints), the survivor buffer (counting), then the launch's per-query counts
   auto lds_of = [&](int flush) {
     const int sb = flush > 0 ? (4 + nmap) * tmk::WAVE : 0;  // position, root, weight (2), node map
-    const int t2 = counting ? 2 * tmk::WAVE : 0;             // two-edge tail side table
-    const int roots = (counting ? 4 : 2) * tmk::TM_ROOTS;    // window, and the root-pair list (counting)
-    const int swept = 2 * tmk::WAVE;                         // long frames' candidates
+    const int t2 = need & TM_NEED_TAIL ? 2 * tmk::WAVE : 0;  // two-edge tail side table
+    const int roots = (need & TM_NEED_RW ? 4 : 2) * tmk::TM_ROOTS;  // window, and the root-pair list
+    const int swept = tmk::WAVE + tmk::WAVE / 4;             // long frames' candidates: slots, frames as bytes
     return (frames * per_frame + roots + sb + t2 + swept) * (int)sizeof(int) + nq * (int)sizeof(unsigned long long);
   };
   int wpe = 0;  // register cap of the counting kernel: 1 (none), 4 (128 VGPRs), 5 (96) or 6 (80)
@@ -602,11 +610,13 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
     wpe = h >= 6 ? 6 : h == 5 ? 5 : h == 4 ? 4 : 1;
   }
   if (!fn && wpe == 0) {
-    // 4 edges and more: 128 VGPRs, 16 wavefronts per CU (their LDS stack allows
-    // about that many anyway); 3 edges: 96 VGPRs, 20 per CU.  12 queries of 4
-    // to 6 edges: 115 ms with 4, 124 with 5, 130 with 6; 2 of 3 edges: 12.0 ms
-    // with 5, 13.4 with 4
-    wpe = lvls >= 2 ? 4 : 5;
+    // 3 and 4 edges: 96 VGPRs, 20 wavefronts per CU, which their stacks leave
+    // room for (4-cycle on 8M hub edges 12.2 ms, 13.7 with 128 VGPRs and 16
+    // wavefronts; 12 queries of the sort 7% less); the pair rewrites (a
+    // query of 4 edges 23.1 against 21.5 ms) and deeper stacks: 128 VGPRs
+    // (5-cycle on 3.1M 27.2 ms, 29.2 with 96; 80 VGPRs lose everywhere but at
+    // 3 edges, by 4%)
+    wpe = lvls >= 3 || (need & (TM_NEED_P0 | TM_NEED_RW)) ? 4 : 5;
   }
   auto blocks_of = [&](int lds_bytes, int *blocks) -> tm_status {
     if (fn) {
@@ -693,6 +703,7 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
   a.frames = frames;
   a.sb_flush = sb_flush;
   a.sb_inline = sb_inline;
+  a.need = need;
   a.scan_max = (tune && tune->scan_max > 0) ? tune->scan_max : 16;
   a.limit_ticks = 0;
   if (tune && tune->time_limit_ms > 0) a.limit_ticks = (long long)tune->time_limit_ms * (g->wall_rate_khz);
@@ -1563,14 +1574,15 @@ tm_status tm_batch_count(tm_graph *g, int32_t nq, const int32_t *num_edges, cons
   std::vector<uint64_t> out(nq);
   Slot &sl = g->slot[0];
   if (mode <= 0) {
-    // one single-query launch per query, in call order, alternating between
-    // two slots (each its own stream, scheduler state and ring), so the tail
-    // of one launch overlaps the start of the next; one synchronization per
-    // slot for the call.  The single-query kernel runs 6-11% faster per
+    // one single-query launch per query, in call order, over the four slots in
+    // turn (each its own stream, scheduler state and ring), so the tails of
+    // launches overlap others' starts (256 queries on 8M edges 92.2 ms with
+    // two slots, 84.9 with four; 36 on 100k edges 4.15, 3.70); one
+    // synchronization per slot for the call.  The single-query kernel runs 6-11% faster per
     // query than the multi-query one (a query index known at compile time),
     // and on a work-dominated set the launches of light queries are a few
     // percent of the time anyway.
-    const int ns = nq > 1 ? 2 : 1;
+    const int ns = std::min(nq, TM_SLOTS);
     tm_status st = TM_OK;
     for (int k = 0; k < ns && st == TM_OK; k++) st = reserve(g, g->slot[k], nq);
     for (int q = 0; q < nq && st == TM_OK; q++) {

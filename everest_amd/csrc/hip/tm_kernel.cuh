@@ -162,12 +162,12 @@ __device__ __forceinline__ unsigned pool_tag(int gen, unsigned lap) {
 // returns compile-time constants for one motif, so the compiler folds the
 // per-edge branches away.
 struct DynSpec {
-  static __device__ __forceinline__ int M(const tm_motif_dev &md) { return md.M; }
-  static __device__ __forceinline__ int kind(const tm_motif_dev &md, int j) { return md.kind[j]; }
-  static __device__ __forceinline__ int a(const tm_motif_dev &md, int j) { return md.a[j]; }
-  static __device__ __forceinline__ int b(const tm_motif_dev &md, int j) { return md.b[j]; }
-  static __device__ __forceinline__ int mapped(const tm_motif_dev &md, int j) { return md.mapped[j]; }
-  static __device__ __forceinline__ int smode(const tm_motif_dev &md, int j) { return md.smode[j]; }
+  static __host__ __device__ __forceinline__ int M(const tm_motif_dev &md) { return md.M; }
+  static __host__ __device__ __forceinline__ int kind(const tm_motif_dev &md, int j) { return md.kind[j]; }
+  static __host__ __device__ __forceinline__ int a(const tm_motif_dev &md, int j) { return md.a[j]; }
+  static __host__ __device__ __forceinline__ int b(const tm_motif_dev &md, int j) { return md.b[j]; }
+  static __host__ __device__ __forceinline__ int mapped(const tm_motif_dev &md, int j) { return md.mapped[j]; }
+  static __host__ __device__ __forceinline__ int smode(const tm_motif_dev &md, int j) { return md.smode[j]; }
   static __device__ __forceinline__ int tmode(const tm_motif_dev &md, int j) { return md.tmode[j]; }
   static __device__ __forceinline__ int xmask(const tm_motif_dev &md, int j) { return md.xmask[j]; }
 };
@@ -362,7 +362,7 @@ constexpr int LV_SWAP = 1 << 9;
 enum { T2_NONE = 0, T2_INDEP = 1, T2_JOIN = 2 };
 
 template <class SP>
-__device__ __forceinline__ int tail2_mode(const tm_motif_dev &md) {
+__host__ __device__ __forceinline__ int tail2_mode(const tm_motif_dev &md) {
   const int M = SP::M(md);
   if (M < 3) return T2_NONE;
   if (SP::kind(md, M - 2) == TM_K_CLOSE) return T2_INDEP;
@@ -622,13 +622,13 @@ constexpr int LV_RW = 1 << 12;   // level-1 frame of the root-pair rewrite: weig
 constexpr int LV_R1 = 1 << 13;   // frame of the pair-tail rewrite: weight = slot - first slot + 1
 
 template <class SP>
-__device__ __forceinline__ bool root_pair_ok(const tm_motif_dev &md) {
+__host__ __device__ __forceinline__ bool root_pair_ok(const tm_motif_dev &md) {
   return SP::M(md) >= 4 && SP::kind(md, 1) == TM_K_CLOSE && SP::smode(md, 1) == TM_S_PAIR_SELF;
 }
 
 // the edge j (= M-3) whose pair edge M-2 repeats, when j brings a node; else -1
 template <class SP>
-__device__ __forceinline__ int pair_tail_edge(const tm_motif_dev &md) {
+__host__ __device__ __forceinline__ int pair_tail_edge(const tm_motif_dev &md) {
   const int M = SP::M(md);
   if (M < 4) return -1;
   const int j = M - 3;
@@ -694,17 +694,21 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
   int *f_e = f_m + MAXN * FR;
   // (counting) the frame's weight and the position its candidate list starts after
   int *f_w = f_e + (ENUM ? MAXE * FR : 0);
+  // (kept only where a query of the launch needs them: the wavefronts a CU
+  // holds go by this memory)
+  const bool P0 = T2 && (args.need & TM_NEED_P0) != 0, RW = T2 && (args.need & TM_NEED_RW) != 0;
+  const bool T2B = T2 && (args.need & TM_NEED_TAIL) != 0;
   int *f_p0 = f_w + (T2 ? FR : 0);
-  int *r_pend = f_p0 + (T2 ? FR : 0);
+  int *r_pend = f_p0 + (P0 ? FR : 0);
   int *r_tl = r_pend + TM_ROOTS;
   // (counting) the root's pair list [r_alo, r_ahi) of the root-pair rewrite
   int *r_alo = r_tl + TM_ROOTS;
-  int *r_ahi = r_alo + (T2 ? TM_ROOTS : 0);
+  int *r_ahi = r_alo + (RW ? TM_ROOTS : 0);
   // survivor buffer (counting, when args.sb_flush > 0): candidates of one
   // level that passed the injectivity and pruning tests, waiting to be
   // expanded up to 64 at a time, with their weights
   const bool COMPACT = !ENUM && INSTR != 1 && args.sb_flush > 0;
-  int *sb_pos = r_ahi + (T2 ? TM_ROOTS : 0);
+  int *sb_pos = r_ahi + (RW ? TM_ROOTS : 0);
   int *sb_ridx = sb_pos + (COMPACT ? WAVE : 0);
   int *sb_wl = sb_ridx + (COMPACT ? WAVE : 0);  // weight, low and high words
   int *sb_wh = sb_wl + (COMPACT ? WAVE : 0);
@@ -713,11 +717,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
   // swapped frame, at the frame's stack index mod 64 (the frames of the
   // deepest level are pushed in one step, at most 64 of them)
   int *sw_lo = sb_m + (COMPACT ? MAXN * WAVE : 0);
-  int *sw_hi = sw_lo + (T2 ? WAVE : 0);
+  int *sw_hi = sw_lo + (T2B ? WAVE : 0);
   // candidates of long frames that passed their rules: slot and frame
-  int *sl_slot = sw_hi + (T2 ? WAVE : 0);
-  int *sl_frame = sl_slot + WAVE;
-  // per-query counts of this wavefront, flushed once at the end
+  int *sl_slot = sw_hi + (T2B ? WAVE : 0);
+  unsigned char *sl_frame = (unsigned char *)(sl_slot + WAVE);  // frames below the top
+  // per-query counts of this wavefront, flushed once at the end (every table
+  // before them is an even number of ints)
   unsigned long long *q_cnt = (unsigned long long *)(sl_frame + WAVE);
   for (int q = lane; q < args.nq; q += WAVE) q_cnt[q] = 0;
   __syncthreads();
@@ -776,12 +781,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     if (f == 1) return &f_lvl[w];
     if (f == 2) return &f_cur[w];
     if (f == 3) return &f_end[w];
-    if (T2 && f == 4) return &f_p0[w];
+    if (P0 && f == 4) return &f_p0[w];
     if (T2 && f == 7 + TM_MAXN) return &f_w[w];
-    if (T2 && f == 8 + TM_MAXN) return &r_alo[(f_lvl[w] >> 16) & 0xff];
-    if (T2 && f == 9 + TM_MAXN) return &r_ahi[(f_lvl[w] >> 16) & 0xff];
-    if (T2 && f == 10 + TM_MAXN) return &sw_lo[w & (WAVE - 1)];
-    if (T2 && f == 11 + TM_MAXN) return &sw_hi[w & (WAVE - 1)];
+    if (RW && f == 8 + TM_MAXN) return &r_alo[(f_lvl[w] >> 16) & 0xff];
+    if (RW && f == 9 + TM_MAXN) return &r_ahi[(f_lvl[w] >> 16) & 0xff];
+    if (T2B && f == 10 + TM_MAXN) return &sw_lo[w & (WAVE - 1)];
+    if (T2B && f == 11 + TM_MAXN) return &sw_hi[w & (WAVE - 1)];
     if (f == 5) return &r_pend[(f_lvl[w] >> 16) & 0xff];
     if (f == 6) return &r_tl[(f_lvl[w] >> 16) & 0xff];
     if (f >= 7 && f < 7 + MAXN) return &f_m[(f - 7) * FR + w];
@@ -1289,7 +1294,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     // frames as it takes to collect a wavefront's worth of candidates that
     // pass; those go on below as if dealt.  The general deal costs 4.3 us of
     // dependent LDS traffic per 64 candidates: that query 348 ms, 68 ms so.
+    // (at most 64 frames give a candidate, but others may give none: frames are
+    // noted by their distance below the top, within a byte)
     int nl = 0;
+    const int top0 = top;
     if (INSTR != 1 && (tmn >= 0 || xm != 0)) {
       const int r0 = tmn >= 0 ? tmn : __ffs(xm) - 1;
       const unsigned rules = xm & ~(1u << r0);
@@ -1299,7 +1307,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         const int lvt = uni(f_lvl[ft]);
         const int c0 = uni(f_cur[ft]), c1 = uni(f_end[ft]);
         const int tlt = uni(r_tl[(lvt >> 16) & 0xff]);
-        if (c1 - c0 < WAVE || (lvt & (LV_SWAP | LV_PAT | 0xff)) != L) break;
+        if (c1 - c0 < WAVE || (lvt & (LV_SWAP | LV_PAT | 0xff)) != L || top0 - ft > 255) break;
         const int *stl = g.stf + (size_t)(lst * TM_NTFIRST) * (size_t)g.E;
         int sl = c0;
         while (!full && sl < c1) {
@@ -1343,7 +1351,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
             if ((om[k] >> lane) & 1) {
               const int w = nl + __popcll(om[k] & lt_mask);
               sl_slot[w] = sl + lane;
-              sl_frame[w] = ft;
+              sl_frame[w] = (unsigned char)(top0 - ft);
             }
             nl += n;
             sl = min(sl + WAVE, c1);
@@ -1368,7 +1376,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     if (nl > 0) {
       if (has) {
         slot = sl_slot[lane];
-        myf = sl_frame[lane];
+        myf = top0 - sl_frame[lane];
       }
     } else {
       // ---- deal the next candidate slots of the topmost frames of one level
@@ -1646,14 +1654,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         if (T2 && (swc & (LV_SWAP | LV_R1))) { sw_lo[w & (WAVE - 1)] = t2lo; sw_hi[w & (WAVE - 1)] = t2hi; }
         if (T2) {
           f_w[w] = (int)(unsigned)wi;
-          f_p0[w] = p0f;
+          if (P0) f_p0[w] = p0f;
         }
 #pragma unroll
         for (int i = 0; i < MAXN; i++) f_m[i * FR + w] = m[i];
         if (j == 0) {  // the window of this lane's root (no frame of an older root is left)
           r_pend[lane] = pend;
           r_tl[lane] = tl;
-          if (T2) {
+          if (RW) {
             r_alo[lane] = a1lo;
             r_ahi[lane] = a1hi;
           }

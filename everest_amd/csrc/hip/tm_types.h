@@ -186,6 +186,13 @@ enum {
   TM_STAT_LDS = 14,    //   LDS bytes per wavefront,
   TM_STAT_WPE = 15     //   register-cap variant (1: none, 6: 80 VGPRs, 0: caller's kernel)
 };
+// Side tables a counting launch keeps per wavefront only when one of its queries
+// uses them: the position a frame's list starts after (pair tail), the root's
+// pair list (root-pair rewrite), edge M-2's range of a frame (pair tail,
+// two-edge tail).
+#define TM_NEED_P0 1
+#define TM_NEED_RW 2
+#define TM_NEED_TAIL 4
 #define TM_NSTATS 16  // per-wavefront counter slot (one 128-byte line)
 #define TM_STAT_SWEEP 16      // host only: queries of the launch counted by the window-sweep kernel
 #define TM_NSTATS_HOST 17
@@ -207,6 +214,7 @@ typedef struct {
   int frames;                 // LDS frame capacity per wavefront
   int scan_max;               // last-edge ranges up to this size are scanned
   int sb_flush;               // counting: survivors buffered before a full-width expansion (0: none buffered)
+  int need;                   // counting: TM_NEED_* side tables of the launch
   int sb_inline;              // counting: with nothing buffered, a step with this many survivors expands them itself
   long long limit_ticks;      // wall-clock budget of the launch (0 = none)
   tm_sched *sched;
