@@ -206,6 +206,22 @@ __global__ void rgap_kernel(const tm_edge *__restrict__ Eg, int E, const int *t0
   }
 }
 
+// Per rule, the root gaps by their number of bits (none: not counted).
+__global__ void __launch_bounds__(256) gap_hist_kernel(const unsigned *__restrict__ rgap, int epad, int E,
+                                                       unsigned *__restrict__ hist) {
+  __shared__ unsigned h[TM_NTFIRST * 33];
+  for (int i = threadIdx.x; i < TM_NTFIRST * 33; i += blockDim.x) h[i] = 0;
+  __syncthreads();
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < E; i += (long long)gridDim.x * blockDim.x)
+    for (int k = 0; k < TM_NTFIRST; k++) {
+      const unsigned gap = rgap[(size_t)k * epad + i];
+      if (gap != 0xffffffffu) atomicAdd(&h[k * 33 + 32 - __clz((int)gap)], 1u);
+    }
+  __syncthreads();
+  for (int i = threadIdx.x; i < TM_NTFIRST * 33; i += blockDim.x)
+    if (h[i]) atomicAdd(&hist[i], h[i]);
+}
+
 // Previous edge of the same pair, per slot of the out- and in-lists: the
 // entry before the edge's own slot in its source's out-pair index.
 __global__ void sprev_kernel(const tm_edge *__restrict__ Eg, const int *__restrict__ outPos,
@@ -512,6 +528,42 @@ static bool pair_pays(const tm_graph *g, const PairItem &it, int delta) {
   return d2 * frac >= PAIR_SLOTS * (double)g->E;
 }
 
+// Edge-1 order: a launch whose blocks are of edge 1's positions, each expanded
+// with the range of roots it extends.  Root by root, every slot of edge 1's list
+// in the window is tested against its pruning rules; here the roots from
+// which they hold are found by one search, so the work goes by the pairs that
+// pass.  It takes a motif whose edge 1 brings a node and has a rule (M = 3: no
+// two-edge tail), over most of the graph's roots.  It pays when edge 1's rules
+// are the rarer ones: the share of edges whose rarest rule's next edge comes
+// within delta, for edge 1 against the root.  Of 60 queries on three
+// power-law graphs those at a quarter or less took 0.1 to 0.9 of the time (0->1,
+// 0->2, 2->3 at 4.7 days on 64M edges 66 -> 8.3 ms; 0->1, 0->2, 0->2, 3->2 at 4.2
+// days on 8M 21.5 -> 7.8); those nearer to each other up to 1.3 times the
+// time, and a rarer root up to 70 times.
+static const double EDGE1_SHARE = 0.25;
+static bool edge1_shape(const tm_motif_dev &md) {
+  if (md.M < 3 || md.kind[1] == TM_K_CLOSE || (md.tmode[2] < 0 && md.xmask[1] == 0)) return false;
+  return md.M > 3 || (tmk::tail2_mode<tmk::DynSpec>(md) == tmk::T2_NONE && tmk::tail_pattern<tmk::DynSpec>(md) == tmk::TP_NONE);
+}
+// the share of edges whose gaps under rule `next` and the rules of `mask` are at
+// most delta, by the rarest: counts by bits, and of the last power of two the
+// part that delta reaches into
+static double rule_share(const tm_graph *g, int next, int mask, int delta) {
+  int bits = 0;
+  while (bits < 31 && (delta >> bits) != 0) bits++;
+  double share = 1.0;
+  for (int k = 0; k < TM_NTFIRST; k++) {
+    if (next != k && !((mask >> k) & 1)) continue;
+    const double lo = bits > 0 ? g->gap_cum[k][bits - 1] : 0.0, hi = g->gap_cum[k][bits];
+    const double part = bits > 0 ? (double)delta / (double)(1u << (bits - 1)) - 1.0 : 1.0;
+    share = std::min(share, (lo + (hi - lo) * std::min(1.0, part)) / (double)g->E);
+  }
+  return share;
+}
+static bool edge1_pays(const tm_graph *g, const tm_motif_dev &md, int delta) {
+  return rule_share(g, md.tmode[2], md.xmask[1], delta) <= EDGE1_SHARE * rule_share(g, md.tmode[1], md.xmask[0], delta);
+}
+
 // Kernel variants (tm_variants.h): node map of 4 or 8, count / enumerate /
 // instrumented count; counting also comes with register caps of 96 and 80
 // VGPRs, and in a single-query and a multi-query (batch) form.
@@ -553,10 +605,19 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
       }
     }
   }
+  // edge-1 order (one query per launch; most of the graph's roots): the blocks
+  // are of positions up to the last edge
+  bool edge1 = false;
+  if (nq == 1 && !swept[0] && !enumerate && instr != 1 && !fn && !multi && !(tune && tune->sweep < 0)) {
+    const tm_query_dev &qd = s.h_queries[q0];
+    edge1 = edge1_shape(qd.m) && qd.root_end > qd.root_beg &&
+            ((tune && tune->sweep > 0) ||
+             (2ll * (qd.root_end - qd.root_beg) >= g->E && edge1_pays(g, qd.m, qd.delta)));
+  }
   auto range_of = [&](int i, int *b, int *e) {
     const tm_query_dev &qd = s.h_queries[q0 + i];
     *b = qd.root_beg;
-    *e = swept[i] ? qd.root_beg : qd.root_end;
+    *e = swept[i] ? qd.root_beg : (edge1 ? g->E : qd.root_end);
   };
   int maxM = 2, maxN = 2;
   long long span = 0;  // roots over all queries (aligned down to 4 per query)
@@ -676,6 +737,10 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
     // start rule of edge 1 and, outside the instrumented kernel (which
     // follows the reference's search tree), the root's second rule
     qt[3] = qd.m.tmode[1] | (instr == 1 ? 0 : qd.m.xmask[0] << TM_QT_XRULE_SHIFT);
+    if (edge1) {  // edge 1's rules: the next edge's, the further ones
+      const int x = qd.m.xmask[1], r = qd.m.tmode[2] >= 0 ? qd.m.tmode[2] : __builtin_ctz((unsigned)x);
+      qt[3] = r | ((x & ~(1 << r)) << TM_QT_XRULE_SHIFT);
+    }
     s.h_prefix[q0 + i] = total_blocks;
     if (re > rb) {
       total_blocks += ((long long)re - (rb & ~3) + (1 << unit_shift) - 1) >> unit_shift;
@@ -704,6 +769,7 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
   a.sb_flush = sb_flush;
   a.sb_inline = sb_inline;
   a.need = need;
+  a.edge1 = edge1 ? 1 : 0;
   a.scan_max = (tune && tune->scan_max > 0) ? tune->scan_max : 16;
   a.limit_ticks = 0;
   if (tune && tune->time_limit_ms > 0) a.limit_ticks = (long long)tune->time_limit_ms * (g->wall_rate_khz);
@@ -1232,7 +1298,7 @@ tm_status tm_graph_upload(int32_t device, const tm_host_graph *hg, tm_graph **ou
                                             E, 0, end_bit, s));
   {
     const size_t kb = up(sizeof(unsigned long long) * (size_t)E);
-    TMPCHK(hipMalloc(&okey, 2 * kb + tmp_bytes));
+    TMPCHK(hipMalloc(&okey, 2 * kb + std::max(tmp_bytes, (size_t)1024)));
     skey = (unsigned long long *)((char *)okey + kb);
     tmp = (char *)okey + 2 * kb;
   }
@@ -1335,7 +1401,20 @@ tm_status tm_graph_upload(int32_t device, const tm_host_graph *hg, tm_graph **ou
   hipLaunchKernelGGL(bucket_kernel, dim3((unsigned)((nb + 1 + 255) / 256)), dim3(256), 0, s, vw.T, E, tmin,
                      bshift, nb, (int *)vw.bucket);
   TMPCHK(hipGetLastError());
-  TMPCHK(hipStreamSynchronize(s));
+  {
+    unsigned hist[TM_NTFIRST * 33];
+    unsigned *d_hist = (unsigned *)okey;
+    TMPCHK(hipMemsetAsync(d_hist, 0, sizeof(hist), s));
+    hipLaunchKernelGGL(gap_hist_kernel, dim3((unsigned)std::min(1024, (E + 255) / 256)), dim3(256), 0, s, vw.rgap, vw.epad,
+                       E, d_hist);
+    TMPCHK(hipGetLastError());
+    TMPCHK(hipMemcpyAsync(hist, d_hist, sizeof(hist), hipMemcpyDeviceToHost, s));
+    TMPCHK(hipStreamSynchronize(s));
+    for (int k = 0; k < TM_NTFIRST; k++) {
+      double sum = 0;
+      for (int b = 0; b < 33; b++) g->gap_cum[k][b] = sum += hist[k * 33 + b];
+    }
+  }
 #undef TMPCHK
   free_tmp();
   // the view itself in device memory, for the kernels to read the graph through

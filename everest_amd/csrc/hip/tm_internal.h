@@ -74,6 +74,7 @@ struct tm_graph {
   int E = 0, V = 0;
   double deg2[3] = {};  // sums over nodes of out*out, in*in and out*in degrees
   double tspan = 0;     // last edge time minus first
+  double gap_cum[TM_NTFIRST][33] = {};  // per rule: edges whose gap to its next edge has at most so many bits
   int num_cus = 0;
   long long wall_rate_khz = 100000;  // wall_clock64 ticks per millisecond
   std::vector<void *> allocs;

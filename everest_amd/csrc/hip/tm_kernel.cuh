@@ -264,6 +264,17 @@ __device__ __forceinline__ int edge_count(const tm_graph_view &g, int x, int y, 
   return gallop_lb(g.outPairPos, c0, s1, pend, mt) - c0;
 }
 
+// first index in [lo, hi) with a[i] >= x, probing down from hi
+__device__ __forceinline__ int gallop_lb_down(const int *__restrict__ a, int lo, int hi, int x, Meter *mt = nullptr) {
+  for (int step = 1; hi > lo; step <<= 1) {
+    const int at = max(lo, hi - step);
+    if (mt) mt->b += 4;
+    if (a[at] < x) return lower_bound_i(a, at + 1, hi, x, mt);
+    hi = at;
+  }
+  return lo;
+}
+
 // Candidate list of motif edge j: slots [lo, hi) of `pos` (and `nbr` for new
 // nodes) whose positions are > p, the position matched for edge j-1.
 struct CandList {
@@ -357,6 +368,7 @@ __device__ __forceinline__ unsigned long long leaf_count(const tm_graph_view &g,
 // each counts A's edges to q's other end before it (one pair search).
 
 // lvl word of a frame: level | swapped << 9 | ... | root index << 16
+constexpr int LV_EDGE1 = 1 << 8;  // frame of edge 1's position: its slots are roots (edge-1 order)
 constexpr int LV_SWAP = 1 << 9;
 
 enum { T2_NONE = 0, T2_INDEP = 1, T2_JOIN = 2 };
@@ -473,7 +485,7 @@ enum { TP_NONE = 0, TP_STAR = 1, TP_PAIR = 2, TP_SAME = 3 };
 constexpr int LV_PAT = 1 << 11;  // frame of edge M-2 summed by its pattern
 
 template <class SP>
-__device__ __forceinline__ int tail_pattern(const tm_motif_dev &md) {
+__host__ __device__ __forceinline__ int tail_pattern(const tm_motif_dev &md) {
   const int M = SP::M(md);
   if (M < 3) return TP_NONE;
   const int j = M - 2, k = M - 1;
@@ -698,6 +710,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
   // holds go by this memory)
   const bool P0 = T2 && (args.need & TM_NEED_P0) != 0, RW = T2 && (args.need & TM_NEED_RW) != 0;
   const bool T2B = T2 && (args.need & TM_NEED_TAIL) != 0;
+  const bool EDGE1 = T2 && !MULTI && args.edge1 != 0;  // the launch's blocks are of edge 1's positions
   int *f_p0 = f_w + (T2 ? FR : 0);
   int *r_pend = f_p0 + (P0 ? FR : 0);
   int *r_tl = r_pend + TM_ROOTS;
@@ -1010,6 +1023,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     // buffered survivors; the expansion itself is in the code once.
     int j = 0, pos = 0, ridx = 0, pend = 0, tl = 0, zmk = 0, skipx = -1;
     bool valid = false;
+    // (uniform) the lanes hold roots at rp0, rt0 whose windows are not set yet,
+    // in edge-1 order together with edge 1's position
+    bool setup = false, trans = false;
+    int rp0 = 0, rt0 = 0;
     unsigned long long wi = 1;
     int m[MAXN];
     int e[ENUM ? MAXE : 1];
@@ -1183,37 +1200,64 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         u = ed.u; v = ed.v; t = ed.t;
         gvalid = u != v;
       }
+      if (EDGE1) {
+        // edge-1 order: the lane's edge is a candidate of motif edge 1, and its
+        // frame holds the roots it extends: those of the list's node before
+        // it from which every rule's next edge is in the window, a range of
+        // the node's root list (ends by one rank read and one search)
+        const bool out = SP::kind(md, 1) == TM_K_NEW_DST;
+        const int an = out ? SP::a(md, 1) : SP::b(md, 1);  // the list's motif node, 0 or 1
+        const int x = out ? u : v, w = out ? v : u;
+        int lo = 0, hi = 0;
+        if (inq) {
+          int tt = t;
+          for (unsigned rr = (unsigned)cxmask | (1u << crule); rr != 0; rr &= rr - 1) {
+            const int k = __ffs(rr) - 1;
+            if (mt) meter.b += 4;
+#pragma unroll
+            for (int i = 0; i < TM_NTFIRST; i++)
+              if (i == k) tt = max(tt, g.tfirst[i][r]);
+          }
+          int from = max(cbeg, pend_of(g, (long long)tt - cdelta - 1, mt));
+          if (pair_tail_edge<SP>(md) == 1) {  // only the first edge of its pair after the root expands
+            if (mt) meter.b += 8;
+            from = max(from, out ? g.sprev[g.outSelf[r]] : g.sprev[(size_t)g.E + g.inSelf[r]]);
+          }
+          if (mt) meter.b += 8;
+          hi = an == 0 ? (out ? g.outSelf[r] : g.outNext[r]) : (out ? g.inNext[r] : g.inSelf[r]);
+          lo = gallop_lb_down(an == 0 ? g.outPos : g.inPos, an == 0 ? g.outR[x] : g.inR[x], hi, from, mt);
+        }
+        const bool ok = lo < hi;
+        const unsigned long long bm = __ballot(ok);
+        const int n = __popcll(bm);
+        if (n > FR) { if (lane == 0) atomicOr(&sched->error, 1); break; }
+        if (ok) {
+          const int at = __popcll(bm & lt_mask);
+          f_cur[at] = lo; f_end[at] = hi; f_lvl[at] = LV_EDGE1 | (lane << 16);
+          if (T2) f_w[at] = 1;
+          if (P0) f_p0[at] = 0;
+          f_m[an * FR + at] = x;
+          f_m[(1 - an) * FR + at] = r;  // (the other node is the root's: not known yet)
+          f_m[2 * FR + at] = w;
+#pragma unroll
+          for (int i = 3; i < MAXN; i++) f_m[i * FR + at] = 0;
+        }
+        top = n;
+        __syncthreads();
+        continue;
+      }
       valid = pass;
       pos = r;
       ridx = lane;
       m[0] = u; m[1] = v;
-      const long long tll = (long long)t + q.delta;
-      tl = tll > 0x7fffffffll ? 0x7fffffff : (int)tll;
+      rp0 = r;
+      rt0 = t;
+      setup = true;
       if constexpr (INSTR == 1) {
         if (gvalid) {
-          const int pe = pend_of(g, tll);
+          const int pe = pend_of(g, (long long)t + q.delta);
           (SP::kind(md, 1) == TM_K_CLOSE ? rx2 : rx1) += 1;
           rp += ref_probes<SP>(g, md, 1, m, r, pe);
-        }
-      }
-      if (valid) {
-        pend = pend_of(g, tll, mt);
-        if (INSTR != 1) valid = (pend - r - 1) >= (M - 1);
-      }
-      // (counting) the last motif edge closes the root's own two nodes: every
-      // edge of a match lies at or before that pair's last edge in the
-      // window, so the root's window ends there (positions and pruning time)
-      if (T2 && valid && M >= 3 && SP::kind(md, M - 1) == TM_K_CLOSE && SP::a(md, M - 1) < 2 &&
-          SP::b(md, M - 1) < 2) {
-        const int x = SP::a(md, M - 1) == 0 ? u : v, y = SP::b(md, M - 1) == 0 ? u : v;
-        const int pl = pair_last(g, x, y, r, pend, mt);
-        if (pl < 0) {
-          valid = false;
-        } else {
-          pend = pl + 1;
-          if (mt) meter.b += 4;
-          tl = g.T[pl];
-          valid = (pend - r - 1) >= (M - 1);
         }
       }
     } else {
@@ -1298,7 +1342,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     // noted by their distance below the top, within a byte)
     int nl = 0;
     const int top0 = top;
-    if (INSTR != 1 && (tmn >= 0 || xm != 0)) {
+    trans = EDGE1 && L == 0;
+    if (INSTR != 1 && !trans && (tmn >= 0 || xm != 0)) {
       const int r0 = tmn >= 0 ? tmn : __ffs(xm) - 1;
       const unsigned rules = xm & ~(1u << r0);
       bool full = false, moved = false;
@@ -1457,7 +1502,24 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     int tfn = 0, tx = 0, node = -1;
     // position, neighbour and the next edge's first-candidate time: three
     // loads at the same slot of one list, issued together
-    if (has && !swp && !patf) {
+    if (trans) {
+      if (has) {
+        // the slot is a root of the list's node: with edge 1's position a candidate
+        const int an = kind == TM_K_NEW_DST ? SP::a(md, 1) : SP::b(md, 1);
+        const int x = sel(m, an), other = an == 0 ? g.outNbr[slot] : g.inNbr[slot];
+        rp0 = an == 0 ? g.outPos[slot] : g.inPos[slot];
+        rt0 = g.T[rp0];
+        pos = sel(m, 1 - an);
+        if (mt) meter.b += 12 + 4 * __popc((unsigned)SP::xmask(md, 0));
+        tx = -0x7fffffff - 1;
+        for (unsigned rr = (unsigned)SP::xmask(md, 0); rr != 0; rr &= rr - 1)
+          tx = max(tx, g.stf[(size_t)((an == 0 ? TM_L_OUT : TM_L_IN) * TM_NTFIRST + __ffs(rr) - 1) * (size_t)g.E + slot]);
+        valid = other != x && other != m[2] && rp0 < q.root_end && (long long)tx <= (long long)rt0 + q.delta;
+        put(m, 1 - an, other);
+        ridx = lane;
+      }
+      setup = true;
+    } else if (has && !swp && !patf) {
       // position, neighbour (new node); unless swept, the next edge's time and the further rules' times
       if (mt) meter.b += kind != TM_K_CLOSE ? 8 : 4;
       if (mt && nl == 0) meter.b += 4 * ((tmn >= 0 ? 1 : 0) + __popc(xm));
@@ -1498,7 +1560,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     // follows; otherwise (nothing buffered, and sb_inline survivors or the
     // level's last candidates in hand) they are expanded in this step
     bool buffer = false;
-    if (COMPACT) {
+    if (COMPACT && !trans) {
       const bool surv = valid && (tmn < 0 || tfn <= tl);
       const unsigned long long bm = __ballot(surv);
       const int ns = __popcll(bm);
@@ -1529,9 +1591,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         rp += ref_probes<SP>(g, md, j + 1, m, pos, pend);
       }
     }
-    valid = valid && (tmn < 0 || tfn <= tl);
+    valid = valid && (trans || tmn < 0 || tfn <= tl);
     zmk = (lvw >> 24) & 0xff;
-    if (T2 && valid && j == M - 2) {
+    if (T2 && trans) {
+      zmk = 0;
+    } else if (T2 && valid && j == M - 2) {
       const int cr = tail_crule<SP>(md);
       if (cr >= 0) {
         if (mt) meter.b += 4;
@@ -1539,6 +1603,45 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
       }
     }
     }  // deal and filter
+    }
+    if (setup) {
+      // ------------------------------------------ the windows of the lanes' roots
+      const tm_query_dev &q = args.queries[qcur];
+      const tm_motif_dev &md = q.m;
+      const int M = SP::M(md);
+      const long long tll = (long long)rt0 + q.delta;
+      tl = tll > 0x7fffffffll ? 0x7fffffff : (int)tll;
+      if (valid) {
+        pend = pend_of(g, tll, mt);
+        if (INSTR != 1) valid = (pend - rp0 - 1) >= (M - 1);
+      }
+      // (counting) the last motif edge closes the root's own two nodes: every
+      // edge of a match lies at or before that pair's last edge in the
+      // window, so the root's window ends there (positions and pruning time)
+      if (T2 && valid && M >= 3 && SP::kind(md, M - 1) == TM_K_CLOSE && SP::a(md, M - 1) < 2 &&
+          SP::b(md, M - 1) < 2) {
+        const int x = SP::a(md, M - 1) == 0 ? m[0] : m[1], y = SP::b(md, M - 1) == 0 ? m[0] : m[1];
+        const int pl = pair_last(g, x, y, rp0, pend, mt);
+        if (pl < 0) {
+          valid = false;
+        } else {
+          pend = pl + 1;
+          if (mt) meter.b += 4;
+          tl = g.T[pl];
+          valid = (pend - rp0 - 1) >= (M - 1);
+        }
+      }
+      if (T2 && trans) {
+        valid = valid && pos < pend;
+        if (valid && j == M - 2) {
+          const int cr = tail_crule<SP>(md);
+          if (cr >= 0) {
+            if (mt) meter.b += 4;
+            const int tn = (cr & 0xff) == TM_T_PAIR_SELF ? g.tfirst[TM_T_PAIR_SELF][pos] : g.tfirst[TM_T_RECIP][pos];
+            if (tn > tl) skipx = sel(m, cr >> 8);
+          }
+        }
+      }
     }
     // ---------------------------------------------- expand the matches at edge j
     // One copy of these searches serves the roots, the dealt candidates and
@@ -1658,7 +1761,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         }
 #pragma unroll
         for (int i = 0; i < MAXN; i++) f_m[i * FR + w] = m[i];
-        if (j == 0) {  // the window of this lane's root (no frame of an older root is left)
+        if (setup) {  // the window of this lane's root (no frame of an older root is left)
           r_pend[lane] = pend;
           r_tl[lane] = tl;
           if (RW) {

@@ -214,6 +214,7 @@ typedef struct {
   int frames;                 // LDS frame capacity per wavefront
   int scan_max;               // last-edge ranges up to this size are scanned
   int sb_flush;               // counting: survivors buffered before a full-width expansion (0: none buffered)
+  int edge1;                  // counting: the launch's blocks are of edge 1's positions (edge-1 order)
   int need;                   // counting: TM_NEED_* side tables of the launch
   int sb_inline;              // counting: with nothing buffered, a step with this many survivors expands them itself
   long long limit_ticks;      // wall-clock budget of the launch (0 = none)

@@ -97,7 +97,10 @@ typedef struct tm_tuning {
                             The same choice for 4-edge motifs whose last edge repeats the root's pair
                             (edge 1 a new node on a root node's list, edge 2 a new node on edge 1's new
                             node's list): counted by the root-pair sweep kernel, which expands each
-                            pair's edge-1 slots once for all of the pair's roots */
+                            pair's edge-1 slots once for all of the pair's roots; and for single-query
+                            launches of motifs whose edge 1 brings a node: edge by edge 1's
+                            positions instead of root by root (0: when its pruning rules are
+                            the rarer ones over most of the graph's roots) */
 } tm_tuning;
 
 /* Library version (TM_ABI_VERSION) and last error of the calling thread. */
