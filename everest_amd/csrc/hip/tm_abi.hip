@@ -723,8 +723,14 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
   // graph's roots reach every wavefront and a large one's are read 1024 at a
   // time (100k edges, the 36 3-edge motifs: 86.4 ms with 256-root blocks in
   // claims of 4, which 98 wavefronts took, 7.9 ms with 16-root blocks).
-  int unit_shift = 4;
-  while (unit_shift < 10 && (span >> (unit_shift + 1)) >= 4ll * grid) unit_shift++;
+  // A small range (a few roots of an enumeration's cut, each of thousands of
+  // matches) goes down to 4 roots, with idle wavefronts beside it that take
+  // what its own give away early: the rows of 26 roots,
+  // 20,000 of them, 820 us with two wavefronts of 16 roots, 315 so (cap of
+  // 20,000 rows on 2M hub edges 2.2 -> 1.3 ms).
+  int unit_shift = 2;
+  while (unit_shift < 10 && ((span >> (unit_shift + 1)) >= 4ll * grid || (unit_shift < 4 && (span >> (unit_shift + 1)) >= TM_SMALL_BLOCKS)))
+    unit_shift++;
   long long total_blocks = 0;
   for (int i = 0; i < nq; i++) {
     const tm_query_dev &qd = s.h_queries[q0 + i];
@@ -747,7 +753,8 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
     }
   }
   s.h_prefix[q0 + nq] = total_blocks;
-  if (total_blocks < grid) grid = (int)std::max<long long>(1, total_blocks);
+  const bool small = total_blocks > 0 && total_blocks < TM_SMALL_BLOCKS;
+  if (total_blocks < grid) grid = (int)std::max<long long>(1, small ? std::min(grid, TM_SMALL_BLOCKS) : total_blocks);
   // a caller's claim size counts 256 roots; the library's own shrinks with the blocks left
   const int claim_blocks =
       (tune && tune->claim_blocks > 0) ? std::max(1, (int)(((long long)tune->claim_blocks << 8) >> unit_shift)) : 0;
@@ -785,7 +792,7 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
   a.scouts = a.idle_cap / TM_STRIPES;
   a.steal_min = (tune && tune->steal_min > 0) ? tune->steal_min : 64;
   {
-    const long long us = (tune && tune->steal_after_us > 0) ? tune->steal_after_us : 1000;
+    const long long us = (tune && tune->steal_after_us > 0) ? tune->steal_after_us : (small ? 20 : 1000);
     a.steal_after_ticks = us * g->wall_rate_khz / 1000;
   }
   // two-edge tail: frames of edge M-2 with at least this many window candidates
@@ -1034,13 +1041,39 @@ static tm_status count_ranges(tm_graph *g, Slot &sl, int M, const int32_t *src, 
   return st;
 }
 
+// Device memory for enumeration rows: the slot keeps one buffer of up to
+// TM_ROWS_KEEP bytes between calls (making and freeing one took 0.2 ms, three
+// times per enumeration that reaches its cap); larger ones are a call's own.
+static tm_status rows_get(tm_graph *g, Slot &sl, size_t bytes, int32_t **out) {
+  if (bytes > sl.rows_bytes && bytes <= TM_ROWS_KEEP) {
+    // (dev_alloc's memory goes with the graph: a quarter at a time keeps what is outgrown small)
+    size_t want = std::max<size_t>(1 << 16, sl.rows_bytes * 4);
+    while (want < bytes) want *= 4;
+    void *p = nullptr;
+    tm_status st = dev_alloc(g, &p, std::min<size_t>(want, TM_ROWS_KEEP));
+    if (st != TM_OK) return st;
+    sl.rows = (int32_t *)p;
+    sl.rows_bytes = std::min<size_t>(want, TM_ROWS_KEEP);
+  }
+  if (bytes <= sl.rows_bytes) {
+    *out = sl.rows;
+    return TM_OK;
+  }
+  HIPTRY(hipMalloc(out, bytes));
+  return TM_OK;
+}
+static void rows_put(Slot &sl, int32_t *rows) {
+  if (rows && rows != sl.rows) (void)hipFree(rows);
+}
+
 // Every row of the roots [b, e) (fewer than `room` of them) into host rows.
 static tm_status enum_all(tm_graph *g, Slot &sl, int M, const int32_t *src, const int32_t *dst, int32_t delta,
                           int32_t b, int32_t e, int64_t room, std::vector<int32_t> *rows, tm_launch_fn fn,
                           void *user) {
   int32_t *d_rows = nullptr;
-  HIPTRY(hipMalloc(&d_rows, sizeof(int32_t) * (size_t)std::max<int64_t>(room, 1) * M));
-  tm_status st = stage_queries(g, sl, 0, 1, nullptr, &M, src, dst, M, &delta, &b, &e);
+  tm_status st = rows_get(g, sl, sizeof(int32_t) * (size_t)std::max<int64_t>(room, 1) * M, &d_rows);
+  if (st != TM_OK) return st;
+  st = stage_queries(g, sl, 0, 1, nullptr, &M, src, dst, M, &delta, &b, &e);
   uint64_t c = 0;
   if (st == TM_OK) {
     sl.s.h_queries[0].rows = d_rows;
@@ -1056,7 +1089,7 @@ static tm_status enum_all(tm_graph *g, Slot &sl, int M, const int32_t *src, cons
       if (he != hipSuccess) st = fail(TM_ERR_HIP, hipGetErrorString(he));
     }
   }
-  (void)hipFree(d_rows);
+  rows_put(sl, d_rows);
   return st;
 }
 
@@ -1763,10 +1796,10 @@ static tm_status enum_impl(tm_graph *g, int32_t num_edges, const int32_t *msrc, 
   const int32_t rbeg = s.h_queries[0].root_beg, rend = s.h_queries[0].root_end;
   int32_t *d_rows = nullptr;
   const size_t row_bytes = sizeof(int32_t) * (size_t)std::max<int64_t>(cap, 1) * num_edges;
-  HIPTRY(hipMalloc(&d_rows, row_bytes));
+  if ((st = rows_get(g, sl, row_bytes, &d_rows)) != TM_OK) return st;
   s.h_queries[0].rows = d_rows;
   s.h_queries[0].cap = cap;
-  if ((st = launch(g, sl, 0, 1, true, tune, false, false, fn, user)) != TM_OK) { (void)hipFree(d_rows); return st; }
+  if ((st = launch(g, sl, 0, 1, true, tune, false, false, fn, user)) != TM_OK) { rows_put(sl, d_rows); return st; }
   st = finish(g, sl, 0, 1, count);
   if (st == TM_OK && *count < (uint64_t)cap) {
     // below the cap no root was held back: every match is written
@@ -1777,7 +1810,7 @@ static tm_status enum_impl(tm_graph *g, int32_t num_edges, const int32_t *msrc, 
     if (rows_written) *rows_written = (int64_t)*count;
   } else if (st == TM_OK) {
     // at the cap: replace the schedule-dependent subset by the deterministic one
-    (void)hipFree(d_rows);
+    rows_put(sl, d_rows);
     d_rows = nullptr;
     int64_t nw = 0;
     // the cut counts with the caller's kernel only when it counts (else the
@@ -1786,7 +1819,7 @@ static tm_status enum_impl(tm_graph *g, int32_t num_edges, const int32_t *msrc, 
                   cut_with_fn ? fn : nullptr, cut_with_fn ? user : nullptr);
     if (rows_written) *rows_written = st == TM_OK ? nw : 0;
   }
-  if (d_rows) (void)hipFree(d_rows);
+  rows_put(sl, d_rows);
   return st;
 }
 

@@ -12,6 +12,8 @@
 
 #define TM_LAUNCH_MAXQ 512  // queries per launch (their table and counts live in LDS)
 #define TM_OCC_MAX 64
+#define TM_ROWS_KEEP ((size_t)16 << 20)  // bytes of enumeration rows a slot keeps at most
+#define TM_SMALL_BLOCKS 256  // a launch of fewer root blocks has idle wavefronts beside them
 #define TM_SB_FLUSH_DEFAULT 32   // counting: survivors buffered before a full-width expansion
 #define TM_SB_INLINE_DEFAULT 32  // counting: survivors a step expands itself when nothing is buffered
 
@@ -58,6 +60,8 @@ struct Slot {
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;  // around the mining kernel
   Scratch s;
+  int32_t *rows = nullptr;                  // enumeration rows kept between calls (rows_get)
+  size_t rows_bytes = 0;
   float last_kernel_ms = 0.f;
   int last_claim = 0, last_grid = 0, last_lds = 0, last_wpe = 0, last_sweep = 0;
   unsigned long long last_stats[TM_NSTATS_HOST] = {};
