@@ -356,6 +356,8 @@ void dispatcher(tm_server *s, std::mutex *ready_mu, std::condition_variable *rea
   }
   ready_cv->notify_all();
   std::unique_lock<std::mutex> lk(s->mu);
+  constexpr double kSpinMs = 0.3;
+  Clock::time_point moved = Clock::now();  // when a launch last began or ended
   for (;;) {
     bool progress = false;
     int busy = 0;
@@ -380,8 +382,16 @@ void dispatcher(tm_server *s, std::mutex *ready_mu, std::condition_variable *rea
         if (s->lane[k].busy) busy++;
       }
     if (s->stop && s->waiting.empty() && busy == 0) break;
+    if (progress) moved = Clock::now();
     if (!progress) {
-      if (busy)
+      if (busy && ms_between(moved, Clock::now()) < kSpinMs) {
+        // a light launch ends within this time: look again at once (a timed
+        // wait of 50 us comes back after 100 and more, longer than most
+        // launches take), with the lock free for submitters in between
+        lk.unlock();
+        std::this_thread::yield();
+        lk.lock();
+      } else if (busy)
         s->cv_work.wait_for(lk, std::chrono::microseconds(50));  // poll the running launches
       else
         s->cv_work.wait(lk);  // idle until a request or the stop arrives
