@@ -135,48 +135,133 @@ __global__ __launch_bounds__(256) void sweep_kernel(tm_graph_view g, const tm_qu
 // v or w.  A wavefront takes 64 consecutive roots, one per lane, and deals
 // the union of their pieces over its lanes (a scan of the piece lengths,
 // each slot's root found by a binary search over the lanes), so a hub's
-// long piece is shared by all 64 lanes.  Runs to completion, like the
-// window sweep.
-__global__ __launch_bounds__(256) void pair_sweep_kernel(tm_graph_view g, const tm_query_dev *queries,
-                                                         tmh::PairBatch b) {
+// long piece is shared by all 64 lanes.  Of the slots so dealt some 40% add
+// anything, and those take from one step to hundreds: they are collected in
+// LDS and summed 64 at a time, so that the sums run with all lanes at work.
+// A slot's edge-2 slots are read in order up to kScan of them, four loads in
+// flight; past that every p_j's rank is found from the last one's, the
+// pairs with u, v and w looked up once.  Blocks are single wavefronts with
+// few groups each: sums differ by orders of magnitude between groups, and a block
+// of four kept three wavefronts waiting (8M power-law edges, 0->1 0->2 3->2
+// 0->1, window 5.5 days: 13.3 ms -> 11.4 with single wavefronts -> 5.9 with
+// the collected sums, cursors and loads; now 19 GB of cache lines missed in
+// L2 at 3.2 TB/s, nearly all of them single random reads).  kScan of 12, 32 and
+// 96 measure 5.87, 5.87 and 6.11 ms.  Runs to completion, like the window sweep.
+constexpr int kScan = 32;
+
+struct PairWork {  // L1 slots that count, one per index
+  int a[128], w[128], u[128], v[128], A[128], j[128], lo[128], s1[128], l2[128];
+};
+
+// One such slot per lane: node w at position a, its edge-2 list from slot l2,
+// the pair u -> v with slots up to s1, its roots before a ending at slot A,
+// the first of them whose window covers a at slot lo, and j the first pair
+// edge after w's first edge-2 slot (j < s1, and root A - 1 reaches it).
+__device__ __forceinline__ unsigned long long pair_slot_sum(const tm_graph_view &g, bool d2, int delta, int a, int w,
+                                                            int u, int v, int A, int j, int lo, int s1, int l2) {
+  const int *L2R = d2 ? g.outR : g.inR;
+  const int *L2P = d2 ? g.outPos : g.inPos;
+  const int *L2N = d2 ? g.outNbr : g.inNbr;
+  const int *pp = g.outPairPos;
+  const int hi = L2R[w + 1], scan = min(hi, l2 + kScan);
+  const long long tlim = (long long)g.T[pp[A - 1]] + delta;  // past it no root before a reaches
+  unsigned long long acc = 0;
+  int pj = pp[j], cur = l2;
+  long long tj = g.T[pj], n2 = 0;
+  {  // the first root that reaches p_j: lo or later, at most A - 1
+    int h = A - 1;
+    while (lo < h) {
+      const int mid = (lo + h) >> 1;
+      if ((long long)g.T[pp[mid]] < tj - delta) lo = mid + 1;
+      else h = mid;
+    }
+  }
+  bool more = true;
+  while (true) {
+    // four slots in one step: their loads are under way together
+    bool all = cur + 4 <= scan;
+    if (all) {
+      const int p0 = L2P[cur], p1 = L2P[cur + 1], p2 = L2P[cur + 2], p3 = L2P[cur + 3];
+      const int y0 = L2N[cur], y1 = L2N[cur + 1], y2 = L2N[cur + 2], y3 = L2N[cur + 3];
+      const bool b0 = p0 < pj, b1 = p1 < pj, b2 = p2 < pj, b3 = p3 < pj;
+      n2 += (int)(b0 && y0 != u && y0 != v && y0 != w) + (int)(b1 && y1 != u && y1 != v && y1 != w) +
+            (int)(b2 && y2 != u && y2 != v && y2 != w) + (int)(b3 && y3 != u && y3 != v && y3 != w);
+      cur += (int)b0 + (int)b1 + (int)b2 + (int)b3;
+      all = b3;
+    } else {
+      while (cur < scan && L2P[cur] < pj) {
+        const int y = L2N[cur++];
+        n2 += (int)(y != u && y != v && y != w);
+      }
+      if (cur == scan && scan < hi) break;  // a long list: counted by ranks from here
+    }
+    if (all) continue;
+    acc += (unsigned long long)(A - lo) * (unsigned long long)n2;
+    if (++j == s1 || (tj = g.T[pj = pp[j]]) > tlim) {
+      more = false;
+      break;
+    }
+    while ((long long)g.T[pp[lo]] < tj - delta) lo++;  // (root A - 1 reaches p_j)
+  }
+  if (!more) return acc;
+  // edge-2 slots in (a, p_j) less those to u, v and w, each rank found from the last one's
+  int x0 = 0, x1 = 0, y0 = 0, y1 = 0, z0 = 0, z1 = 0;
+  if (tmk::pair_find(g, d2 ? w : u, d2 ? u : w, &x0, &x1)) x0 = upper_bound_i(pp, x0, x1, a);
+  if (tmk::pair_find(g, d2 ? w : v, d2 ? v : w, &y0, &y1)) y0 = upper_bound_i(pp, y0, y1, a);
+  if (!g.no_self_loops && tmk::pair_find(g, w, w, &z0, &z1)) z0 = upper_bound_i(pp, z0, z1, a);
+  int x = x0, y = y0, z = z0;
+  while (true) {
+    cur = tmk::gallop_lb(L2P, cur, hi, pj);
+    x = tmk::gallop_lb(pp, x, x1, pj);
+    y = tmk::gallop_lb(pp, y, y1, pj);
+    z = tmk::gallop_lb(pp, z, z1, pj);
+    acc += (unsigned long long)(A - lo) * (unsigned long long)((cur - l2) - (x - x0) - (y - y0) - (z - z0));
+    if (++j == s1 || (tj = g.T[pj = pp[j]]) > tlim) return acc;
+    while ((long long)g.T[pp[lo]] < tj - delta) lo++;
+  }
+}
+
+__global__ __launch_bounds__(64) void pair_sweep_kernel(tm_graph_view g, const tm_query_dev *queries,
+                                                        tmh::PairBatch b) {
+  __shared__ PairWork work;
   const tmh::PairItem it = b.item[blockIdx.y];
   const tm_query_dev &qd = queries[it.q];
   const int beg = qd.root_beg, end = qd.root_end, delta = qd.delta;
-  const int lane = threadIdx.x & 63;
+  const int lane = threadIdx.x;
   const long long groups = ((long long)end - beg + 63) / 64;
-  const long long wstride = (long long)gridDim.x * (blockDim.x >> 6);
   const int *L1R = it.d1 ? g.outR : g.inR;
   const int *L1P = it.d1 ? g.outPos : g.inPos;
   const int *L1N = it.d1 ? g.outNbr : g.inNbr;
   const int *L2R = it.d2 ? g.outR : g.inR;
   const int *L2P = it.d2 ? g.outPos : g.inPos;
-  const int *L2N = it.d2 ? g.outNbr : g.inNbr;
   const int *pp = g.outPairPos;
-  constexpr int kScan = 32;
   unsigned long long acc = 0;
-  for (long long gi = (long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); gi < groups; gi += wstride) {
-    // this lane's root: its pair run [s0, s1e), its roots from slot rb, its L1 piece [i0, i0 + n)
+  int held = 0;  // slots in `work`, below 64 between rounds
+  for (long long gi = blockIdx.x; gi < groups; gi += gridDim.x) {
+    // this lane's root: its pair's slots from its own, k, up to s1e, its L1 piece [i0, i0 + n)
     const long long rr = beg + gi * 64 + lane;
-    int n = 0, u = 0, v = 0, s0 = 0, s1e = 0, rb = 0, i0 = 0;
+    int n = 0, u = 0, v = 0, k = 0, s1e = 0, i0 = 0;
     if (rr < end) {
       const int r = (int)rr;
       const tm_edge e = g.Eg[r];
       u = e.u;
       v = e.v;
       if (u != v) {
-        const int k = g.outPairSelf[r];
+        int s0 = 0;
+        k = g.outPairSelf[r];
         tmk::pair_find(g, u, v, &s0, &s1e);
-        const int clip = pp[lower_bound_i(pp, k, s1e, pend_of(g, (long long)e.t + delta)) - 1];
-        int lo = r;
-        if (k > s0 && pp[k - 1] >= beg) {
-          const int pr = pp[k - 1];
-          lo = max(lo, pp[lower_bound_i(pp, k - 1, s1e, pend_of(g, (long long)g.T[pr] + delta)) - 1]);
-        }
-        if (clip > lo) {
-          const int x = it.s1 == 0 ? u : v;
-          i0 = upper_bound_i(L1P, L1R[x], L1R[x + 1], lo);
-          n = lower_bound_i(L1P, i0, L1R[x + 1], clip) - i0;
-          rb = lower_bound_i(pp, s0, s1e, beg);
+        if (s1e - s0 > 1) {
+          const int clip = pp[lower_bound_i(pp, k, s1e, pend_of(g, (long long)e.t + delta)) - 1];
+          int lo = r;
+          if (k > s0 && pp[k - 1] >= beg) {
+            const int pr = pp[k - 1];
+            lo = max(lo, pp[lower_bound_i(pp, k - 1, s1e, pend_of(g, (long long)g.T[pr] + delta)) - 1]);
+          }
+          if (clip > lo) {
+            const int x = it.s1 == 0 ? u : v;
+            i0 = upper_bound_i(L1P, L1R[x], L1R[x + 1], lo);
+            n = lower_bound_i(L1P, i0, L1R[x + 1], clip) - i0;
+          }
         }
       }
     }
@@ -200,65 +285,53 @@ __global__ __launch_bounds__(256) void pair_sweep_kernel(tm_graph_view g, const 
       const long long oincl = __shfl(incl, own, 64);
       const int on = __shfl(n, own, 64), oi0 = __shfl(i0, own, 64);
       const int ou = __shfl(u, own, 64), ov = __shfl(v, own, 64);
-      const int os0 = __shfl(s0, own, 64), os1 = __shfl(s1e, own, 64), orb = __shfl(rb, own, 64);
-      if (item >= total) continue;
-      const int slot = oi0 + (int)(item - (oincl - on));
-      const int a = L1P[slot], w = L1N[slot];
-      if (w == ou || w == ov) continue;
-      // w's edge-2 list after a, from the upload's rank arrays (a lies in
-      // in(w) when edge 1 enters w, in out(w) when it leaves w)
-      const int l2lo = it.d1 ? (it.d2 ? g.outNext[a] : g.inSelf[a] + 1) : (it.d2 ? g.outSelf[a] + 1 : g.inNext[a]);
-      const int l2hi = L2R[w + 1];
-      if (l2lo >= l2hi) continue;
-      const int first2 = L2P[l2lo];  // no j with p_j <= first2 adds anything
-      const int A = lower_bound_i(pp, orb, os1, min(a, end));
-      const long long tlim = (long long)g.T[pp[A - 1]] + delta;  // p_j beyond it: no root before a reaches it
-      // edge-2 slots of w after a are scanned once for all j (their other
-      // ends checked directly) while the scan stays short; past kScan slots
-      // each j's count is a rank minus the pair counts of u, v and w
-      int cur = l2lo;
-      long long valid = 0;
-      bool scan = true;
-      int loj = -1;
-      // the first pair edge after a: A itself when a < end (a is no pair edge and a > r >= beg)
-      for (int j = a < end ? A : upper_bound_i(pp, os0, os1, a); j < os1; j++) {
-        const int pj = pp[j];
-        const long long tpj = g.T[pj];
-        if (tpj > tlim) break;
-        if (pj <= first2) continue;
-        const long long tj = tpj - delta;  // roots from the first with time >= tj
-        if (loj < 0) {
-          int lo2 = orb, hi2 = A;
-          while (lo2 < hi2) {
-            const int mid = (lo2 + hi2) >> 1;
-            if ((long long)g.T[pp[mid]] < tj) lo2 = mid + 1;
-            else hi2 = mid;
-          }
-          loj = lo2;
-        } else {
-          while (loj < A && (long long)g.T[pp[loj]] < tj) loj++;
+      const int ok = __shfl(k, own, 64), os1 = __shfl(s1e, own, 64);
+      bool in = item < total;
+      int a = 0, w = 0, l2 = 0, A = 0, j = 0;
+      if (in) {
+        const int slot = oi0 + (int)(item - (oincl - on));
+        a = L1P[slot];
+        w = L1N[slot];
+        in = w != ou && w != ov;
+      }
+      if (in) {
+        // w's edge-2 list after a, from the upload's rank arrays (a lies in
+        // in(w) when edge 1 enters w, in out(w) when it leaves w)
+        l2 = it.d1 ? (it.d2 ? g.outNext[a] : g.inSelf[a] + 1) : (it.d2 ? g.outSelf[a] + 1 : g.inNext[a]);
+        A = tmk::gallop_lb(pp, ok + 1, os1, min(a, end));
+        // no pair edge before w's first edge-2 slot adds anything.  Whether l2 is
+        // w's at all is asked last: most are ruled out without that read
+        const int first2 = L2P[min(l2, g.E - 1)];
+        j = tmk::gallop_lb(pp, A, os1, first2);
+        in = j < os1 && (long long)g.T[pp[j]] <= (long long)g.T[pp[A - 1]] + delta &&
+             l2 < L2R[w + 1];
+      }
+      const unsigned long long m = __ballot(in);
+      if (in) {
+        const int at = held + __popcll(m & ((1ull << lane) - 1));
+        work.a[at] = a, work.w[at] = w, work.u[at] = ou, work.v[at] = ov, work.A[at] = A;
+        work.j[at] = j, work.lo[at] = ok, work.s1[at] = os1, work.l2[at] = l2;
+      }
+      held += __popcll(m);
+      __syncthreads();
+      if (held >= 64) {
+        acc += pair_slot_sum(g, it.d2, delta, work.a[lane], work.w[lane], work.u[lane], work.v[lane], work.A[lane],
+                             work.j[lane], work.lo[lane], work.s1[lane], work.l2[lane]);
+        held -= 64;
+        __syncthreads();
+        if (lane < held) {
+          const int f = lane + 64;
+          work.a[lane] = work.a[f], work.w[lane] = work.w[f], work.u[lane] = work.u[f], work.v[lane] = work.v[f];
+          work.A[lane] = work.A[f], work.j[lane] = work.j[f], work.lo[lane] = work.lo[f];
+          work.s1[lane] = work.s1[f], work.l2[lane] = work.l2[f];
         }
-        if (loj >= A) break;
-        long long n2;
-        if (scan) {
-          while (cur < l2hi && cur - l2lo < kScan && L2P[cur] < pj) {
-            const int y = L2N[cur++];
-            valid += (y != ou) & (y != ov) & (y != w);
-          }
-          scan = !(cur < l2hi && L2P[cur] < pj);  // every slot before pj scanned
-        }
-        if (scan) {
-          n2 = valid;
-        } else {
-          n2 = lower_bound_i(L2P, l2lo, l2hi, pj) - l2lo;
-          if (it.d2) n2 -= edge_count(g, w, ou, a, pj) + edge_count(g, w, ov, a, pj);
-          else n2 -= edge_count(g, ou, w, a, pj) + edge_count(g, ov, w, a, pj);
-          if (!g.no_self_loops) n2 -= edge_count(g, w, w, a, pj);
-        }
-        acc += (unsigned long long)(A - loj) * (unsigned long long)n2;
+        __syncthreads();
       }
     }
   }
+  if (lane < held)
+    acc += pair_slot_sum(g, it.d2, delta, work.a[lane], work.w[lane], work.u[lane], work.v[lane], work.A[lane],
+                         work.j[lane], work.lo[lane], work.s1[lane], work.l2[lane]);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
   if (lane == 0 && acc) atomicAdd(qd.count, acc);
@@ -287,10 +360,10 @@ int pair_shape(const tm_motif_dev &md, PairItem *it) {
 
 tm_status pair_enqueue(const tm_graph_view &g, const tm_query_dev *d_queries, const PairBatch &b, hipStream_t stream) {
   if (b.n <= 0) return TM_OK;
-  // one wavefront per 64 roots, at most 4096 blocks of 4 wavefronts per query
-  const long long per = ((long long)g.E + 255) / 256;
-  const unsigned gx = (unsigned)std::max<long long>(1, std::min<long long>(per, 4096));
-  hipLaunchKernelGGL(pair_sweep_kernel, dim3(gx, (unsigned)b.n), dim3(256), 0, stream, g, d_queries, b);
+  // one wavefront per 64 roots, at most 32768 (four times what is resident) per query
+  const long long per = ((long long)g.E + 63) / 64;
+  const unsigned gx = (unsigned)std::max<long long>(1, std::min<long long>(per, 32768));
+  hipLaunchKernelGGL(pair_sweep_kernel, dim3(gx, (unsigned)b.n), dim3(64), 0, stream, g, d_queries, b);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_error(TM_ERR_HIP, std::string("pair-sweep launch: ") + hipGetErrorString(e));
   return TM_OK;
