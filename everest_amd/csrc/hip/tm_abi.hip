@@ -792,7 +792,14 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
   a.scouts = a.idle_cap / TM_STRIPES;
   a.steal_min = (tune && tune->steal_min > 0) ? tune->steal_min : 64;
   {
-    const long long us = (tune && tune->steal_after_us > 0) ? tune->steal_after_us : (small ? 20 : 1000);
+    // A look costs two reads, and up to 5 edges earlier ones shorten the
+    // launch's tail: 256 random queries on 8M power-law edges 63.2 ms of kernels
+    // with 1000 us, 60.8 with 100, 61.9 with 50 and a look at every step;
+    // 5-cycle on 3.1M hub edges 27.9 -> 26.6, one of 5 edges 1.74 -> 1.11.  At
+    // 6 edges 63 of the queries take 5.5 and 5.4 ms, and 1000 us stay (the
+    // deadline test relies on one of them running for 20 ms).
+    const long long us = (tune && tune->steal_after_us > 0) ? tune->steal_after_us
+                                                            : (small ? 20 : maxM <= 5 ? 100 : 1000);
     a.steal_after_ticks = us * g->wall_rate_khz / 1000;
   }
   // two-edge tail: frames of edge M-2 with at least this many window candidates
