@@ -26,12 +26,12 @@ from . import abi
 
 # (field, values): the first value, 0, is the library default
 AXES = [
-    ("waves_per_simd_hint", [0, 6, 4, 1]),  # register cap: 0 = 5 (96 VGPRs), 6 = 80, 4 = 128, 1 = none
-    ("tail_swap", [0, 2, 4, 8, -1]),        # two-edge tail threshold (0 = 32, -1 = off)
+    ("waves_per_simd_hint", [0, 6, 4, 1]),  # register cap: 0 = 5 (96 VGPRs) or 4, 6 = 80, 4 = 128, 1 = none
+    ("tail_swap", [0, 4, 8, 32, -1]),       # two-edge tail threshold (0 = 2, -1 = off)
     ("sb_flush", [0, -1, 48, 64]),          # survivor compaction (0 = 32 where it costs no occupancy)
     ("sb_inline", [0, 16, 48]),             # survivors a step expands itself with none buffered (0 = 32)
     ("scan_max", [0, 8, 32]),               # last-edge ranges scanned up to this size (0 = 16)
-    ("claim_blocks", [0, 1, 2, 8, 32]),     # 256-root blocks per claim (0 = ~8 claims per wavefront)
+    ("claim_blocks", [0, 1, 2, 8, 32]),     # 256-root blocks per claim (0 = half of what is left, shared out)
     ("waves_per_cu", [0, 16, 24]),          # resident wavefronts per CU (0 = occupancy-limited, <= 32)
     ("steal_after_us", [0, 250, 4000]),     # donation trigger (0 = 100 us, 6 edges 1000)
     ("steal_min", [0, 16, 256]),            # smallest donated half-frame (0 = 64 candidates)

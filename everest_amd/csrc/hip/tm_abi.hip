@@ -621,6 +621,7 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
   };
   int maxM = 2, maxN = 2;
   long long span = 0;  // roots over all queries (aligned down to 4 per query)
+  double passing = 0;  // those of them that their rules let through, about
   for (int i = 0; i < nq; i++) {
     const tm_query_dev &qd = s.h_queries[q0 + i];
     if (qd.m.tmode[1] < 0 || qd.m.tmode[1] >= TM_NTFIRST) return fail(TM_ERR_INTERNAL, "edge 1 has no start rule");
@@ -628,7 +629,11 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
     maxN = std::max(maxN, qd.m.n);
     int rb, re;
     range_of(i, &rb, &re);
-    if (re > rb) span += re - (rb & ~3);
+    if (re > rb) {
+      span += re - (rb & ~3);
+      passing += (re - rb) * (edge1 ? rule_share(g, qd.m.tmode[2], qd.m.xmask[1], qd.delta)
+                                    : rule_share(g, qd.m.tmode[1], qd.m.xmask[0], qd.delta));
+    }
   }
   const int lvls = enumerate ? std::max(1, maxM - 1) : std::max(1, maxM - 2);
   const int frames = 64 * lvls;
@@ -714,6 +719,19 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
       blocks = b0;
     }
   }
+  if (!fn && counting && lvls <= 2 && !(tune && tune->waves_per_simd_hint > 0) && passing >= 256.0 * g->num_cus) {
+    // 3 and 4 edges with roots enough to fill the chip: 80 VGPRs where the stacks
+    // leave room for more than 20 wavefronts per CU (0->1, 0->2, 2->3 on 64M
+    // edges 7.97 -> 7.29 ms, 0->1, 2->1, 0->3, 3->0 there 5.38 -> 4.96, 0->1, 0->2,
+    // 0->2 on 8M 2.00 -> 1.87; one in eight a few percent slower).  A launch
+    // with few only has more wavefronts to start (.069 -> .077 ms).
+    const int w5 = wpe;
+    int b6 = 0;
+    wpe = 6;
+    if ((st = blocks_of(lds, &b6)) != TM_OK) return st;
+    if (b6 > 20) blocks = b6;
+    else wpe = w5;
+  }
   int wpc = (tune && tune->waves_per_cu > 0) ? tune->waves_per_cu : 32;
   if (blocks > 0) wpc = std::min(wpc, blocks);
   if (wpc < 1) wpc = 1;
@@ -731,6 +749,15 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
   int unit_shift = 2;
   while (unit_shift < 10 && ((span >> (unit_shift + 1)) >= 4ll * grid || (unit_shift < 4 && (span >> (unit_shift + 1)) >= TM_SMALL_BLOCKS)))
     unit_shift++;
+  // Up to 5 edges, blocks of half to an eighth of that while 48 or more roots of
+  // one pass: an expansion is nearly as full, and the launch's tail shorter
+  // (cycles of 4 and 5 edges 12.1 -> 11.3 and 21.9 -> 20.3 ms; where 33 or fewer
+  // passed it took 2 to 20% more: 256 random queries 57.9 -> 61.3).  6 edges keep
+  // the larger ones (the deadline test relies on one of them running for
+  // 20 ms; 25 -> 20).
+  while (maxM <= 5 && unit_shift > 5 && passing * (double)(1 << unit_shift) >= 48.0 * span &&
+         (span >> unit_shift) <= 16ll * grid)
+    unit_shift--;
   long long total_blocks = 0;
   for (int i = 0; i < nq; i++) {
     const tm_query_dev &qd = s.h_queries[q0 + i];
@@ -755,9 +782,15 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
   s.h_prefix[q0 + nq] = total_blocks;
   const bool small = total_blocks > 0 && total_blocks < TM_SMALL_BLOCKS;
   if (total_blocks < grid) grid = (int)std::max<long long>(1, small ? std::min(grid, TM_SMALL_BLOCKS) : total_blocks);
-  // a caller's claim size counts 256 roots; the library's own shrinks with the blocks left
-  const int claim_blocks =
-      (tune && tune->claim_blocks > 0) ? std::max(1, (int)(((long long)tune->claim_blocks << 8) >> unit_shift)) : 0;
+  // A caller's claim size counts 256 roots.  The library's own is one block
+  // where two roots or more per wavefront pass: the wavefronts of a stripe then
+  // work on neighbouring blocks, whose windows overlap in its L2, and none is
+  // left with a long run of them (5-cycle on 3.1M hub edges 26.6 -> 21.9 ms; 0->1,
+  // 0->2, 2->3 on 64M edges 9.96 -> 7.97).  With fewer the claims themselves
+  // are the cost, and shrink with the blocks left (64M edges .10 ms, .16 with single blocks).
+  const int claim_blocks = (tune && tune->claim_blocks > 0)
+                               ? std::max(1, (int)(((long long)tune->claim_blocks << 8) >> unit_shift))
+                               : passing >= 2.0 * grid ? 1 : 0;
 
   tm_kernel_args a;
   memset(&a, 0, sizeof(a));

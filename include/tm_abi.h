@@ -61,7 +61,8 @@ typedef struct tm_host_graph {
 /* Launch parameters; zero fields take the library defaults (occupancy-limited
  * waves up to 32 per CU, scan_max 16, no time
  * limit, steal_every 16, steal_max 4, steal_min 64, steal_after_us 100 (6 edges 1000),
- * claim_blocks: claims that shrink with the roots left). */
+ * claim_blocks: single blocks of roots, or claims that shrink with the roots
+ * left where few of them pass the start rules). */
 typedef struct tm_tuning {
   int32_t waves_per_cu;  /* resident wavefronts per CU in the persistent grid */
   int32_t claim_blocks;  /* roots per claim of the root schedule, in units of 256 */
@@ -75,7 +76,8 @@ typedef struct tm_tuning {
                                   4 = capped at 128 VGPRs (16 wavefronts per CU, no spills),
                                   5 = capped at 96 VGPRs (20 per CU), 6 = capped at 80 VGPRs
                                   (24 per CU); 0 = 5 for motifs of 3 and 4 edges without
-                                  a repeated pair, else 4 */
+                                  a repeated pair, else 4, and 6 for 3 and 4 edges where many
+                                  roots pass and the stacks leave room */
   int32_t sb_flush;      /* counting: candidates that pass the filters of one level are buffered in
                             LDS and expanded together once this many (1..64) are held; -1 = each
                             step expands its own survivors; 0 = the library's choice */

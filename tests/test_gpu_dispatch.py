@@ -39,6 +39,26 @@ def test_root_ranges(E):
     dg.close()
 
 
+@pytest.mark.parametrize("E", [4097, 40_003, 270_001])
+def test_passing_roots(E):
+    """Single-block claims, smaller blocks and more wavefronts go by how many roots the start rules let through:
+    windows from the shortest to the whole graph, on a quarter wavefront per SIMD and on the full grid."""
+    from everest_amd import abi
+    rng = np.random.default_rng(E)
+    U, V, T = random_graph(rng, E, max(4, E // 12), 4 * E)
+    g = prep.preprocess(U, V, T)
+    dg = abi.DeviceGraph.from_dict(g)
+    for mot in ([(0, 1, 0), (1, 2, 1), (2, 3, 2)], [(0, 1, 0), (0, 2, 1), (3, 2, 2), (3, 1, 3)],
+                [(0, 1, 0), (0, 2, 1), (0, 2, 2), (3, 2, 3)]):
+        for delta in (4, E // 50, E // 2, 4 * E):
+            for beg, end in ((0, -1), (5, E // 2 + 3)):
+                want = oracle.count(g, mot, delta, beg, end, nthreads=4)
+                for tune in (dict(), dict(waves_per_cu=1), dict(sweep=-1), dict(claim_blocks=1, waves_per_simd_hint=6)):
+                    print("E", E, "motif", mot, "delta", delta, "roots", beg, end, tune, flush=True)
+                    assert dg.count(mot, delta, beg, end, tune=abi.tuning(**tune)) == want, (mot, delta, beg, tune)
+    dg.close()
+
+
 # repeated root pair (weights by rank), repeated new pair (weights by slot), two-edge tails summed over the
 # last edge's list, a star's pattern, plain frames
 DONATED = [[(0, 1, 0), (0, 1, 1), (0, 2, 2), (2, 3, 3)], [(0, 1, 0), (0, 2, 1), (0, 2, 2), (3, 2, 3)],
