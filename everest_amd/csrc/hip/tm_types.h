@@ -182,7 +182,7 @@ enum {
   TM_STAT_CAPEXIT = 10,// wavefronts that left because enough were waiting
   TM_STAT_WORK = 11,   // wall-clock ticks wavefronts held work (summed)
   TM_STAT_GRID = 12,   // launch shape, filled in by the host: wavefronts,
-  TM_STAT_CLAIM = 13,  //   256-root blocks per claim,
+  TM_STAT_CLAIM = 13,  //   blocks per claim (0: shrinking claims),
   TM_STAT_LDS = 14,    //   LDS bytes per wavefront,
   TM_STAT_WPE = 15     //   register-cap variant (1: none, 6: 80 VGPRs, 0: caller's kernel)
 };

@@ -87,8 +87,8 @@ typedef struct tm_tuning {
                             second-to-last one brings, a partial match whose second-to-last edge has at
                             least this many candidates in the window is counted over the last edge's
                             candidates instead, if those are fewer; 0 = library default (2), < 0 = never */
-  int32_t batch_mode;    /* tm_batch_count: 0 = one single-query launch per query, back to back on one
-                            stream, one synchronization; 1 = one multi-query launch per shape class;
+  int32_t batch_mode;    /* tm_batch_count: 0 = one single-query launch per query, over the graph's
+                            launch slots in turn, one synchronization per slot; 1 = one multi-query launch per shape class;
                             2 = every query of the call in one multi-query launch (its stack sized for
                             the deepest motif) */
   int32_t sweep;         /* counting, 3-edge motifs whose last two edges take candidates from one list of a
