@@ -502,14 +502,16 @@ tm_status build_motif(int M, const int32_t *src, const int32_t *dst, tm_motif_de
 // The window sweep costs a fixed O(E log E) per query; the mining kernel
 // costs about the windows' slots summed over the roots.  Their mean is
 // estimated as sum_x deg_root(x) * deg_window(x) * min(1, delta / time span)
-// / E over the anchor nodes x; measured on a 64M-edge power-law graph the
-// two cost the same near 8 slots per root (mean windows of 0.02 to 3 slots:
-// mining 1-30 ms, sweep 15-60 ms; 22 to 350 slots: mining 0.1-3.3 s).
+// / E over the anchor nodes x.  Measured at estimates 1 to 8: the two cost the
+// same at 2 to 3 slots per root on 8M edges (power law and hubs: sweep 0.9 to
+// 1.0 ms, mining 0.4 to 0.6 at 1 slot and 1.5 to 2.2 at 6; with the root's other
+// list 1.5 ms and 5 slots), at 4 (stars) to 6 (pairs) on 64M power-law edges (sweep
+// 9.0 to 9.8 ms, mining 3.0 to 3.5 at 1 and 9.6 to 13.4 at 6).
 static bool sweep_pays(const tm_graph *g, const SweepItem &it, int delta) {
   const bool root_out = it.anchor == 0, win_out = it.out != 0;
   const double d2 = root_out == win_out ? g->deg2[root_out ? 0 : 1] : g->deg2[2];
   const double frac = g->tspan > 0 ? std::min(1.0, (double)delta / g->tspan) : 1.0;
-  return d2 * frac >= 8.0 * (double)g->E;
+  return d2 * frac >= 6.0 * (double)g->E;
 }
 
 // The root-pair sweep replaces the expansion of every root's edge-1 slots up

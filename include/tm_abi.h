@@ -95,7 +95,7 @@ typedef struct tm_tuning {
                             root node (a star of two new nodes, or a new node's pair twice): > 0 = counted by
                             the window-sweep kernel (O(E log E) per query whatever delta), < 0 = by the
                             mining kernel like every other motif, 0 = the sweep when the roots' windows
-                            are estimated (node degrees x delta / time span) at 8 or more slots on average.
+                            are estimated (node degrees x delta / time span) at 6 or more slots on average.
                             The same choice for 4-edge motifs whose last edge repeats the root's pair
                             (edge 1 a new node on a root node's list, edge 2 a new node on edge 1's new
                             node's list): counted by the root-pair sweep kernel, which expands each
