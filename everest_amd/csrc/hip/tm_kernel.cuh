@@ -892,7 +892,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
         unsigned long long *rec = args.pool + (size_t)(t & (unsigned)(args.pool_cap - 1)) * TM_POOL_FIELDS;
         if (lane < TM_POOL_FIELDS) {
           int v = 0;
-          if (lane == 0) v = qcur | (cstripe << 16);
+          // (root blocks name no query, their taker reads it from its first one: this
+          // wavefront may not have begun one yet)
+          if (lane == 0) v = (b >= 0 ? qcur : 0) | (cstripe << 16);
           else if (lane == 2) v = mid;
           else if (b < 0) v = lane == 1 ? TM_REC_ROOTS : (lane == 3 ? claim_end : claim_k);
           else {
@@ -1110,7 +1112,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
             crule = qt.w & ((1 << TM_QT_XRULE_SHIFT) - 1);
             cxmask = qt.w >> TM_QT_XRULE_SHIFT;
           }
-          if (ENUM && ld_rlx(args.queries[cq].stop)) { roots_done = true; break; }  // enumeration cap reached
+          if (ENUM && ld_rlx(args.queries[cq].stop)) {  // enumeration cap reached: nothing is kept, or left to give away
+            claim_next = claim_end;
+            roots_done = true;
+            break;
+          }
           const int units = 1 << args.unit_shift;
           ublk = (cbeg & ~3) + (b - qb0) * units;
           // this lane's roots of the block inside the query's range
