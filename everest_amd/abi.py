@@ -196,12 +196,12 @@ class DeviceGraph:
         return dict(device_bytes=b.value, num_edges=e.value, num_vertices=v.value, device=d.value)
 
     def last_stats(self):
-        st = np.zeros(17, dtype=np.uint64)
-        check(lib().tm_last_stats(self.handle, _p(st), 17))
+        st = np.zeros(18, dtype=np.uint64)
+        check(lib().tm_last_stats(self.handle, _p(st), 18))
         return dict(steps=int(st[0]), items=int(st[1]), roots=int(st[2]), leaves=int(st[3]), pushes=int(st[4]),
                     donated=int(st[8]), taken=int(st[9]), capexit=int(st[10]), work_ticks=int(st[11]),
                     grid=int(st[12]), claim_blocks=int(st[13]), lds=int(st[14]), wpe=int(st[15]),
-                    sweep=int(st[16]))
+                    sweep=int(st[16]), ring=int(st[17]))
 
     def last_kernel_ms(self):
         ms = ctypes.c_double()

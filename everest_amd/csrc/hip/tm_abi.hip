@@ -819,10 +819,13 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
   a.wstats = s.d_wstats;
   a.pool = s.d_pool;
   a.pool_done = s.d_pool_done;
-  a.pool_cap = s.pool_cap;
-  a.pool_shift = s.pool_shift;
+  // the ring: as many slots as records can be ahead of the tickets (steal_max
+  // per wavefront, which what is allocated bounds), so that a long launch goes
+  // round it several times
+  a.steal_max = std::min((tune && tune->steal_max > 0) ? tune->steal_max : TM_STEAL_MAX, s.pool_cap / grid);
+  a.pool_shift = std::min(s.pool_shift, ceil_log2((long long)grid * a.steal_max));
+  a.pool_cap = 1 << a.pool_shift;
   a.steal_every = (tune && tune->steal_every > 0) ? tune->steal_every : 16;
-  a.steal_max = (tune && tune->steal_max > 0) ? tune->steal_max : 4;
   a.idle_cap = std::max(64, g->num_cus / 2);
   a.scouts = a.idle_cap / TM_STRIPES;
   a.steal_min = (tune && tune->steal_min > 0) ? tune->steal_min : 64;
@@ -844,6 +847,7 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
   sl.last_grid = grid;
   sl.last_lds = lds;
   sl.last_wpe = fn ? 0 : wpe;
+  sl.last_ring = a.pool_cap;
   sl.last_sweep = (int)(pl->sweep.size() + pl->pair.size());
   pl->a = a;
   pl->d_counts = s.d_counts + q0;
@@ -958,9 +962,9 @@ tm_status reserve(tm_graph *g, Slot &sl, int nq) {
   s.d_counts = (unsigned long long *)(b + nqd + nqt + npf);
   s.d_stops = (int *)(b + nqd + nqt + npf + nct);
   if (!s.d_sched) {
-    s.pool_shift = 18;
-    s.pool_cap = 1 << s.pool_shift;
     s.wstats_cap = g->num_cus * 32;  // the most resident one-wave workgroups
+    s.pool_shift = ceil_log2((long long)s.wstats_cap * TM_STEAL_MAX);  // (plan())
+    s.pool_cap = 1 << s.pool_shift;
     const size_t nsc = up(sizeof(tm_sched)), nws = up(sizeof(unsigned long long) * TM_NSTATS * (size_t)s.wstats_cap);
     const size_t ndn = up(sizeof(unsigned) * (size_t)s.pool_cap);
     const size_t npl = sizeof(unsigned long long) * TM_POOL_FIELDS * (size_t)s.pool_cap;
@@ -1042,6 +1046,7 @@ tm_status collect(tm_graph *g, Slot &sl, int q0) {
   dst.last_stats[TM_STAT_CLAIM] = (unsigned long long)sl.last_claim;
   dst.last_stats[TM_STAT_LDS] = (unsigned long long)sl.last_lds;
   dst.last_stats[TM_STAT_WPE] = (unsigned long long)sl.last_wpe;
+  dst.last_stats[TM_STAT_RING] = (unsigned long long)sl.last_ring;
   float ms = 0.f;
   if (hipEventElapsedTime(&ms, sl.ev0, sl.ev1) == hipSuccess) dst.last_kernel_ms = ms;
   g->last_slot = sl.index;

@@ -14,6 +14,7 @@
 #define TM_OCC_MAX 64
 #define TM_ROWS_KEEP ((size_t)16 << 20)  // bytes of enumeration rows a slot keeps at most
 #define TM_SMALL_BLOCKS 256  // a launch of fewer root blocks has idle wavefronts beside them
+#define TM_STEAL_MAX 4  // records a wavefront with work gives away per look
 #define TM_SB_FLUSH_DEFAULT 32   // counting: survivors buffered before a full-width expansion
 #define TM_SB_INLINE_DEFAULT 32  // counting: survivors a step expands itself when nothing is buffered
 
@@ -63,7 +64,7 @@ struct Slot {
   int32_t *rows = nullptr;                  // enumeration rows kept between calls (rows_get)
   size_t rows_bytes = 0;
   float last_kernel_ms = 0.f;
-  int last_claim = 0, last_grid = 0, last_lds = 0, last_wpe = 0, last_sweep = 0;
+  int last_claim = 0, last_grid = 0, last_lds = 0, last_wpe = 0, last_sweep = 0, last_ring = 0;
   unsigned long long last_stats[TM_NSTATS_HOST] = {};
 };
 

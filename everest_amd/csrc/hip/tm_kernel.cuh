@@ -831,7 +831,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
       }
     }
     if (look) {
-      // donate only against unmet demand: tickets drawn minus records reserved
+      // donate only against unmet demand: tickets drawn minus records reserved.
+      // A wavefront is steal_max records ahead of the tickets at most, and the
+      // ring holds that many for each, so a slot's previous lap always has its
+      // ticket drawn
       int want = 0;
       if (lane == 0) {
         const int hd = (int)ld_rlx(&sched->pool_head);

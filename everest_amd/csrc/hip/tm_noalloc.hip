@@ -26,6 +26,7 @@ namespace {
 constexpr int kMaxQ = TM_NOALLOC_MAXQ;
 constexpr int kMaxWaves = 256 * 32;  // per-wavefront counter slots: 256 CUs x 32 wavefronts
 constexpr int kPoolShift = 15;       // donation ring of 2^15 records
+static_assert((1 << kPoolShift) >= kMaxWaves * TM_STEAL_MAX, "a wavefront's records of one look each");
 constexpr size_t kAlign = 256;
 
 constexpr size_t up(size_t x) { return (x + kAlign - 1) / kAlign * kAlign; }

@@ -158,7 +158,8 @@ typedef struct {
 // stripe of the record's busy credit), each stored as a 64-bit word
 // (tag << 32 | value) with device-scope atomic stores, so a taker knows the
 // record is complete when every word carries the tag it expects: no fences,
-// no cache invalidation.  Records live in a ring of pool_cap slots; record r
+// no cache invalidation.  Records live in a ring of pool_cap slots (at least
+// steal_max per wavefront, so that the taker of a slot's previous lap is there); record r
 // goes to slot r mod pool_cap with tag (launch generation, lap r / pool_cap),
 // and its taker stores that tag into pool_done[slot] once the frame is
 // copied out, which lets the slot's next lap be written.
@@ -195,7 +196,8 @@ enum {
 #define TM_NEED_TAIL 4
 #define TM_NSTATS 16  // per-wavefront counter slot (one 128-byte line)
 #define TM_STAT_SWEEP 16      // host only: queries of the launch counted by the window-sweep kernel
-#define TM_NSTATS_HOST 17
+#define TM_STAT_RING 17       // host only: donation ring slots of the launch
+#define TM_NSTATS_HOST 18
 
 typedef struct {
   tm_graph_view g;

@@ -196,7 +196,8 @@ tm_status tm_device_free(tm_graph *g, void *device_ptr);
  * work, summed, and the launch shape: [12]
  * wavefronts in the grid, [13] blocks per claim, [14] LDS bytes per
  * wavefront, [15] register-cap variant, [16] queries of the launch counted
- * by the window-sweep or root-pair sweep kernels (their work is not in [0..11]).  Up to 17
+ * by the window-sweep or root-pair sweep kernels (their work is not in [0..11]),
+ * [17] slots of the donation ring ([8] beyond them: it was used again).  Up to 18
  * entries.
  * No reference counterpart (instrumentation).
  */
@@ -344,7 +345,7 @@ tm_status tm_batch_count(tm_graph *g, int32_t nq, const int32_t *num_edges,
  * results as tm_batch_count, for at most TM_NOALLOC_MAXQ queries per call
  * (TM_ERR_ARG beyond).  Every device buffer of its launches (scheduler
  * state, query tables, counts, per-wavefront counters, a donation ring of
- * 2^15 records) lives in one static device array of
+ * up to 2^15 records) lives in one static device array of
  * TM_NOALLOC_SCRATCH_BYTES, one copy per GPU the library runs on, held
  * until the process ends; the call makes no hipMalloc / hipFree.  Calls on
  * one GPU share that array: this library's calls take turns (one lock per

@@ -1,6 +1,7 @@
 """CPU model of the mining kernel's scheduling protocol: striped root claims,
-busy credits per stripe, and donated records of both kinds (frames and root
-blocks), for counting and for listings that reach their cap.  Any number of
+busy credits per stripe, donated records of both kinds (frames and root
+blocks) in a ring of steal_max slots per wavefront, for counting and for
+listings that reach their cap.  Any number of
 wavefronts step in any order; a launch must end, every credit must be given
 back, every record must be taken, and a counting launch must expand every
 root block exactly once."""
@@ -11,7 +12,7 @@ STRIPES = 8
 
 
 class Launch:
-    def __init__(self, rng, grid, work, claim_blocks, cap=None, idle_cap=4, scouts=2, steal_max=4, steal_min=1,
+    def __init__(self, rng, grid, work, claim_blocks, cap=None, idle_cap=4, scouts=2, steal_max=2, steal_min=1,
                  drop_claim=True, root_query=0):
         """work[b]: candidates of root block b (0: no root of it passes).  drop_claim and root_query: what a
         wavefront that sees the stop flag does with its claim (True: drops it), and the query word of a record of
@@ -26,7 +27,10 @@ class Launch:
         self.busy = [len(range(k, grid, STRIPES)) for k in range(STRIPES)]
         self.hungry = [False] * STRIPES
         self.head = self.tail = self.waiters = 0
-        self.ring, self.taken = {}, 0
+        self.slots = 1 << (grid * steal_max - 1).bit_length()
+        self.ring, self.done, self.taken = {}, {}, 0   # slot -> (record number, record), slot -> record number copied out
+        self.kinds = {"frame": 0, "roots": 0}
+        self.ahead = 0                # most records ahead of the tickets
         self.rows, self.stop = 0, False
         self.done_blocks = [0] * self.nblocks
         self.items = 0
@@ -59,13 +63,16 @@ class Wave:
         self.claim_next = self.claim_end = 0
         self.home = self.cstripe = self.at = self.claim_k = b % STRIPES
         self.first, self.roots_done, self.scout, self.idle, self.waiter, self.told = True, False, False, False, False, False
-        self.ticket = None
+        self.ticket, self.giving = None, None
 
     def give(self):
+        """The donation loop; each yield is a point where others run."""
         L = self.L
-        for _ in range(L.steal_max):
-            if L.head - L.tail <= 0:
-                return
+        head = L.head
+        yield
+        want = min(head - L.tail, L.steal_max)
+        yield
+        for _ in range(want):
             nb = self.claim_end - self.claim_next
             g = ((nb + 1) // 2 if self.frames or self.ublk else nb // 2) if nb > 0 else 0
             b = -1
@@ -74,6 +81,12 @@ class Wave:
                 if b < 0:
                     return
             L.busy[self.cstripe] += 1
+            yield
+            t = L.tail
+            L.tail += 1
+            L.ahead = max(L.ahead, L.tail - L.head)
+            while t >= L.slots and L.done.get(t % L.slots) != t - L.slots:
+                yield  # its slot's previous lap is not copied out yet
             if b >= 0:
                 n = self.frames[b] - self.frames[b] // 2
                 self.frames[b] -= n
@@ -84,8 +97,8 @@ class Wave:
                 word = word - (1 << 32) if word >> 31 else word
                 rec = (word & 0xffff, word >> 16, "roots", self.claim_end - g, self.claim_end, self.claim_k)
                 self.claim_end -= g
-            L.ring[L.tail] = rec
-            L.tail += 1
+            L.kinds[rec[2]] += 1
+            L.ring[t % L.slots] = (t, rec)
 
     def dispatch(self):
         """Until a block with passing roots is in hand, or none is left."""
@@ -131,11 +144,18 @@ class Wave:
     def step(self):
         """One turn of the kernel's main loop; True: the wavefront has left."""
         L = self.L
-        if self.ticket is None:
+        if self.giving is not None:
+            try:
+                next(self.giving)
+                return False
+            except StopIteration:
+                self.giving = None
+        elif self.ticket is None:
             if L.cap is not None and self.frames and L.stop and L.rng.random() < 0.1:
                 self.frames = []
             if (self.frames or self.claim_next < self.claim_end) and L.hungry[self.home]:
-                self.give()
+                self.giving = self.give()
+                return False
         if not self.frames and self.roots_done and self.claim_next >= self.claim_end:
             return self.wait()
         if not self.frames:
@@ -172,12 +192,13 @@ class Wave:
             self.ticket = L.head
             L.head += 1
             return False
-        rec = L.ring.get(self.ticket)
-        if rec is None:
+        t, rec = L.ring.get(self.ticket % L.slots, (None, None))
+        if t != self.ticket:
             if not any(L.busy):
                 L.waiters -= 1
                 return True
             return False
+        L.done[self.ticket % L.slots] = self.ticket
         self.ticket, self.waiter, self.idle = None, False, False
         L.waiters -= 1
         L.taken += 1
@@ -200,26 +221,30 @@ def random_launch(rng, listing, **kw):
     work[lo:lo + busy_part] = rng.integers(0, 60, busy_part)
     cap = int(rng.integers(1, max(2, int(work.sum())))) if listing else None
     return Launch(rng, int(rng.integers(1, 40)), work.tolist(), int(rng.integers(1, 33)), cap,
-                  idle_cap=int(rng.integers(1, 8)), scouts=int(rng.integers(1, 4)), **kw)
+                  idle_cap=int(rng.integers(1, 8)), scouts=int(rng.integers(1, 4)),
+                  steal_max=int(rng.integers(1, 3)), **kw)
 
 
 def settle(L):
     L.run()
     assert L.busy == [0] * STRIPES and L.waiters == 0
-    assert L.taken == L.tail == len(L.ring)
+    assert L.taken == L.tail == sum(L.kinds.values())
+    assert L.ahead <= L.grid * L.steal_max  # records never run further ahead of the tickets than the ring is long
 
 
 def test_counting_expands_every_block_once():
     rng = np.random.default_rng(3)
-    kinds = {"frame": 0, "roots": 0}
+    kinds, laps = {"frame": 0, "roots": 0}, 0
     for _ in range(300):
         L = random_launch(rng, False)
         settle(L)
         assert L.done_blocks == [1] * L.nblocks
         assert L.items == sum(L.work)
-        for r in L.ring.values():
-            kinds[r[2]] += 1
+        for k, n in L.kinds.items():
+            kinds[k] += n
+        laps = max(laps, L.tail // L.slots)
     assert min(kinds.values()) > 100, kinds
+    assert laps > 2, laps
 
 
 def test_listing_at_its_cap_ends_with_every_credit_back():
