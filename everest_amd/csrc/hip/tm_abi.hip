@@ -28,6 +28,9 @@ thread_local std::string g_last_error;
 
 tm_status fail(tm_status s, const std::string &msg) {
   g_last_error = msg;
+  // the runtime keeps an error until it is asked for: told here, it must not
+  // come up again after the next call's first launch
+  if (s == TM_ERR_HIP || s == TM_ERR_NOMEM) (void)hipGetLastError();
   return s;
 }
 
