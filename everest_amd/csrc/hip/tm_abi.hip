@@ -934,7 +934,11 @@ tm_status launch(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm
   Plan pl;
   tm_status st = plan(g, sl, q0, nq, enumerate, tune, instr, multi, fn, user, &pl);
   if (st != TM_OK) return st;
-  return enqueue(g, sl, pl, true, true);
+  st = enqueue(g, sl, pl, true, true);
+  // part of it may run: its first kernel reads the pinned staging and its
+  // second may write rows, which are the next call's once this one returns
+  if (st != TM_OK) (void)hipStreamSynchronize(sl.stream);
+  return st;
 }
 
 // Create the slot's stream and reserve its staging space for nq queries

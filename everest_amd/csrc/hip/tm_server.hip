@@ -266,7 +266,10 @@ bool launch_next(tm_server *s, int k) {
   if (st == TM_OK) st = launch(s->g, sl, 0, n, enumerate, tune, false, !enumerate && n > 1);
   hipError_t e = hipSuccess;
   if (st == TM_OK) e = hipEventRecord(ln.done, sl.stream);
-  if (st == TM_OK && e != hipSuccess) st = lane_error("server launch", e);
+  if (st == TM_OK && e != hipSuccess) {
+    st = lane_error("server launch", e);
+    (void)hipStreamSynchronize(sl.stream);  // (its staging and rows are the next launch's)
+  }
   if (st != TM_OK) {  // the requests fail without running
     for (uint64_t id : pick) {
       Request &r = *s->reqs[id];

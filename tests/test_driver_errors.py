@@ -17,3 +17,59 @@ fake.fake_limit(1 << 40)
 %s
 g.close()
 """ % (call, call))
+
+
+CALLS = {
+    "count": "g.count(MOT, 100)",
+    "work": "g.count_work(MOT, 100)",
+    "bytes": "g.count_bytes(MOT, 100)",
+    "enum": "g.enum(MOT, 100, 50)",
+    "batch": "g.batch_count([(MOT, 100)] * 3)",
+    "batch by class": "g.batch_count([(MOT, 100)] * 3, tune=abi.tuning(batch_mode=1))",
+    "noalloc": "g.batch_count_noalloc([(MOT, 100)] * 3)",
+}
+
+
+SWEPT = [c for c in CALLS if c not in ("work", "bytes", "enum")]
+
+
+@pytest.mark.parametrize("call,kernel", [(c, k) for c in CALLS for k in ("mine_kernel", "finish_kernel")] +
+                         [(c, "sweep_kernel") for c in SWEPT])
+def test_a_launch_that_fails_midway_is_waited_for(call, kernel):
+    """Its first kernel reads pinned staging that the next call rewrites."""
+    if kernel == "sweep_kernel":
+        body = CALLS[call].replace("MOT, 100", "[(0, 1, 0), (0, 2, 1), (0, 3, 2)], 100")
+        body = body.replace("batch_mode=1", "batch_mode=1, sweep=1")
+        if "tune" not in body:
+            body = body[:-1] + ", tune=abi.tuning(sweep=1))"
+    else:
+        body = CALLS[call]
+    run("""
+g = graph()
+fake.fake_fail_kernel(b"%s", 0)
+fails(lambda: %s)
+assert b"launch fails" in fake.fake_trace()
+assert pend() == 0, pend()
+%s
+g.close()
+""" % (kernel, body, body))
+
+
+@pytest.mark.parametrize("how", ["fake.fake_fail_kernel(b'mine_kernel', 0)", "fake.fake_fail_record(%d)"])
+@pytest.mark.parametrize("cap", [-1, 50])
+def test_a_served_launch_that_fails_midway_is_waited_for(how, cap):
+    """Before its staging and its place in the row arena go to the next request."""
+    if "record" in how:
+        how = how % 3  # the launch's two timing events pass, its end does not
+    run("""
+g = graph()
+s = abi.Server(g, slots=1)
+%s
+r = s.wait(s.submit(MOT, 100, %d), 5000)
+assert r["status"] != 0, r
+assert pend() == 0, pend()
+r = s.wait(s.submit(MOT, 100, %d), 5000)
+assert r["status"] == 0, r
+s.close()
+g.close()
+""" % (how, cap, cap))
