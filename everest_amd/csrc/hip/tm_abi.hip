@@ -1756,12 +1756,13 @@ tm_status tm_batch_count(tm_graph *g, int32_t nq, const int32_t *num_edges, cons
       st = stage_queries(g, sq, q, 1, &q, num_edges, msrc, mdst, TM_MAX_MOTIF_EDGES, deltas, nullptr, nullptr);
       if (st == TM_OK) st = launch(g, sq, q, 1, false, class_tuning(g, key[q], tune), 0, false);
     }
-    // every launch is waited for, also when one could not be enqueued: the
-    // pinned staging is theirs until then
+    // every launch is waited for, also when one could not be enqueued or
+    // another slot's wait failed: the pinned staging is theirs until then
     int bits = 0;
     for (int k = 0; k < ns; k++) {
       Slot &sk = g->slot[k];
-      HIPTRY(hipStreamSynchronize(sk.stream));
+      const hipError_t he = sk.stream ? hipStreamSynchronize(sk.stream) : hipSuccess;
+      if (he != hipSuccess && st == TM_OK) st = fail(TM_ERR_HIP, std::string("batch wait: ") + hipGetErrorString(he));
       if (st != TM_OK) continue;
       for (int q = k; q < nq; q += ns) {
         counts[q] = sk.s.h_counts[q];

@@ -73,3 +73,18 @@ assert r["status"] == 0, r
 s.close()
 g.close()
 """ % (how, cap, cap))
+
+
+@pytest.mark.parametrize("slot", [1, 2, 4])
+def test_a_batch_waits_for_every_slot(slot):
+    """Also when the wait for one of them fails."""
+    run("""
+g = graph()
+qs = [(MOT, 100)] * 9
+fake.fake_fail_sync(%d)
+fails(lambda: g.batch_count(qs), 3)
+assert b"sync fails" in fake.fake_trace()
+assert pend() == 0, pend()
+assert len(g.batch_count(qs)) == 9
+g.close()
+""" % slot)
