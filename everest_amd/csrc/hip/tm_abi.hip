@@ -994,14 +994,16 @@ void pin_free(Scratch &s) {
 }
 
 tm_status pin_alloc(Scratch &s, int cap) {
-  pin_free(s);
   auto up = [](size_t x) { return (x + 63) / 64 * 64; };
   const size_t o_qtab = up(sizeof(tm_query_dev) * cap), o_prefix = o_qtab + up(sizeof(int) * 4 * cap);
   const size_t o_counts = o_prefix + up(sizeof(long long) * (cap + 1));
   const size_t o_errors = o_counts + up(sizeof(unsigned long long) * cap);
   const size_t o_stats = o_errors + up(sizeof(int) * cap);
-  HIPTRY(hipHostMalloc(&s.pin, o_stats + up(sizeof(unsigned long long) * TM_NSTATS)));
-  char *b = (char *)s.pin;
+  void *pin = nullptr;
+  HIPTRY(hipHostMalloc(&pin, o_stats + up(sizeof(unsigned long long) * TM_NSTATS)));
+  pin_free(s);  // (only now: without the new one the slot keeps what its cap_q and pointers describe)
+  s.pin = pin;
+  char *b = (char *)pin;
   s.h_queries = (tm_query_dev *)b;
   s.h_qtab = (int *)(b + o_qtab);
   s.h_prefix = (long long *)(b + o_prefix);

@@ -88,3 +88,21 @@ assert pend() == 0, pend()
 assert len(g.batch_count(qs)) == 9
 g.close()
 """ % slot)
+
+
+def test_pinned_staging_survives_a_failed_growth():
+    """A batch larger than the slots' staging, refused for pinned memory, leaves the old staging in use."""
+    run("""
+g = graph()
+qs = [(MOT, 100)] * 400
+for _ in range(2):
+    fake.fake_fail_host(1)
+    fails(lambda: g.batch_count(qs), 4)
+    fake.fake_fail_host(0)
+    assert g.count(MOT, 100) == 0
+    assert len(g.batch_count(qs[:200])) == 200
+    assert len(g.batch_count_noalloc(qs[:200])) == 200
+assert len(g.batch_count(qs)) == 400
+g.close()
+assert fake.fake_used() == 0
+""")
