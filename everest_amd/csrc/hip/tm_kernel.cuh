@@ -30,6 +30,7 @@ constexpr int WAVE = 64;
 constexpr int TM_ROW = 4 * WAVE;    // roots of one 16-byte load per lane
 constexpr int TM_ROWS = 4;          // most rows of a dispatch block (1024 roots)
 constexpr int TM_SWEEP = 8;         // 64-slot chunks of a long frame whose rule times are read together
+constexpr int TM_SWEEP_STEP = 16384;  // slots after which a step of such reads ends
 constexpr int TM_ROOTS = WAVE + 1;  // window table entries: one per lane's root, one for a taken frame
 
 // ------------------------------------------------------------------ helpers
@@ -1356,6 +1357,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
       const int r0 = tmn >= 0 ? tmn : __ffs(xm) - 1;
       const unsigned rules = xm & ~(1u << r0);
       bool full = false, moved = false;
+      int left = TM_SWEEP_STEP;
       while (!full && top > 0) {
         const int ft = top - 1;
         const int lvt = uni(f_lvl[ft]);
@@ -1409,6 +1411,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
             }
             nl += n;
             sl = min(sl + WAVE, c1);
+          }
+          left -= TM_SWEEP * WAVE;
+          if (left <= 0) {
+            // enough for one step (some 0.2 ms) where hardly any slot passes: the
+            // deadline, the other flags and idle wavefronts are looked at now
+            full = true;
+            iter |= 63u;
+            steal_cd = 0;
           }
         }
         st_items += (unsigned long long)(sl - c0);
