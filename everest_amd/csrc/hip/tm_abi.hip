@@ -616,7 +616,7 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
   if (nq == 1 && !swept[0] && !enumerate && instr != 1 && !fn && !multi && !(tune && tune->sweep < 0)) {
     const tm_query_dev &qd = s.h_queries[q0];
     edge1 = edge1_shape(qd.m) && qd.root_end > qd.root_beg &&
-            ((tune && tune->sweep > 0) ||
+            ((tune && tune->sweep > 1) ||  // (1 is about the sweep kernels: here it would cost up to 70 times the time)
              (2ll * (qd.root_end - qd.root_beg) >= g->E && edge1_pays(g, qd.m, qd.delta)));
   }
   auto range_of = [&](int i, int *b, int *e) {

@@ -99,10 +99,10 @@ typedef struct tm_tuning {
                             The same choice for 4-edge motifs whose last edge repeats the root's pair
                             (edge 1 a new node on a root node's list, edge 2 a new node on edge 1's new
                             node's list): counted by the root-pair sweep kernel, which expands each
-                            pair's edge-1 slots once for all of the pair's roots; and for single-query
-                            launches of motifs whose edge 1 brings a node: edge by edge 1's
-                            positions instead of root by root (0: when its pruning rules are
-                            the rarer ones over most of the graph's roots) */
+                            pair's edge-1 slots once for all of the pair's roots.  Single-query
+                            launches of other motifs whose edge 1 brings a node can go by edge 1's
+                            positions instead of root by root: 0 and 1 = when its pruning rules are
+                            the rarer ones over most of the graph's roots, 2 or more = always, < 0 = never */
 } tm_tuning;
 
 /* Library version (TM_ABI_VERSION) and last error of the calling thread. */
@@ -189,7 +189,8 @@ tm_status tm_device_free(tm_graph *g, void *device_ptr);
 
 /*
  * Work counters of the graph's last launch: [0] wavefront steps, [1] candidate
- * items examined, [2] roots dispatched, [3] last-edge range computations,
+ * items examined, [2] roots dispatched (positions of edge 1 where the launch
+ * goes by those: tm_tuning.sweep), [3] last-edge range computations,
  * [4] frames pushed, [5..7] reference work of an instrumented run (X1, X2, P),
  * [8] frames donated between wavefronts, [9] donated frames taken, [10]
  * wavefronts that left early, [11] wall-clock ticks (100 MHz) wavefronts held
