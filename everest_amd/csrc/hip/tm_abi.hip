@@ -751,8 +751,14 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
   // what its own give away early: the rows of 26 roots,
   // 20,000 of them, 820 us with two wavefronts of 16 roots, 315 so (cap of
   // 20,000 rows on 2M hub edges 2.2 -> 1.3 ms).
-  int unit_shift = 2;
-  while (unit_shift < 10 && ((span >> (unit_shift + 1)) >= 4ll * grid || (unit_shift < 4 && (span >> (unit_shift + 1)) >= TM_SMALL_BLOCKS)))
+  // Where the caller gives a claim's size, in units of 256 roots, blocks divide it
+  // (as far as their number stays within 32 bits).
+  int unit_shift = 2, most = 10;
+  if (tune && tune->claim_blocks > 0) {
+    most = std::min(most, 8 + __builtin_ctz((unsigned)tune->claim_blocks));
+    while (most < 10 && (span >> most) >= 1ll << 29) most++;
+  }
+  while (unit_shift < most && ((span >> (unit_shift + 1)) >= 4ll * grid || (unit_shift < 4 && (span >> (unit_shift + 1)) >= TM_SMALL_BLOCKS)))
     unit_shift++;
   // Up to 5 edges, blocks of half to an eighth of that while 48 or more roots of
   // one pass: an expansion is nearly as full, and the launch's tail shorter

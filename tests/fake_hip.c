@@ -10,6 +10,7 @@
 #include <stdlib.h>
 #include <string.h>
 #include <sys/mman.h>
+#include "tm_types.h"
 
 #define MAXK 4096
 #define MAXS 64
@@ -24,6 +25,7 @@ static char fail_kernel[64];
 static int fail_kernel_after, fail_host, fail_record, fail_sync, fail_stream;
 static unsigned long long head_pairs;
 static char trace[1 << 16];
+static tm_kernel_args mined;       /* of the last mining launch */
 
 void fake_fail_kernel(const char *part, int after) { snprintf(fail_kernel, sizeof fail_kernel, "%s", part); fail_kernel_after = after; }
 void fake_fail_host(int on) { fail_host = on; }
@@ -31,6 +33,8 @@ void fake_fail_record(int on) { fail_record = on; }
 void fake_fail_sync(int stream) { fail_sync = 1; fail_stream = stream; }
 void fake_limit(size_t bytes) { limit = bytes; }
 void fake_pairs(unsigned long long n) { head_pairs = n; }
+int fake_unit_shift(void) { return mined.unit_shift; }
+int fake_claim_blocks(void) { return mined.claim_blocks; }
 size_t fake_used(void) { return used; }
 size_t fake_peak(int reset) { size_t p = peak; if (reset) peak = used; return p; }
 int fake_pending(void) { int n = 0; for (int i = 0; i < MAXS; i++) n += pending[i]; return n; }
@@ -124,6 +128,7 @@ hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **a, size_t s, hi
   if (fail_kernel[0] && strstr(n, fail_kernel) && fail_kernel_after-- <= 0) { fail_kernel[0] = 0; note("launch fails"); return ret(hipErrorLaunchFailure); }
   note(n);
   pending[sid(t)]++;
+  if (strstr(n, "mine_kernel")) mined = *(tm_kernel_args *)a[0];
   if (strstr(n, "heads_kernel")) **(unsigned long long **)a[2] = head_pairs;
   return hipSuccess;
 }

@@ -47,6 +47,7 @@ def library():
     if _so is None:
         _so = os.path.join(tempfile.mkdtemp(prefix="fakehip"), "libfakehip.so")
         subprocess.check_call(["gcc", "-O1", "-shared", "-fPIC", "-w", "-I/opt/rocm/include",
+                               "-I" + os.path.join(ROOT, "everest_amd", "csrc", "hip"),
                                os.path.join(TESTS, "fake_hip.c"), "-o", _so])
     return _so
 

@@ -106,3 +106,19 @@ assert len(g.batch_count(qs)) == 400
 g.close()
 assert fake.fake_used() == 0
 """)
+
+
+def test_a_callers_claim_size_counts_256_roots():
+    """Whatever the size of a dispatch block."""
+    run("""
+for E in (900, 300_000, 1_100_000):
+    g = graph(E, E // 8)
+    for waves in (0, 1):
+        for claim in (1, 2, 3, 4, 6, 8, 31, 32):
+            g.count(MOT, 100, tune=abi.tuning(claim_blocks=claim, waves_per_cu=waves))
+            got = fake.fake_claim_blocks() << fake.fake_unit_shift()
+            assert got == 256 * claim, (E, waves, claim, got)
+    g.count(MOT, 100, tune=abi.tuning(waves_per_cu=1))
+    assert E < 1_000_000 or fake.fake_unit_shift() == 10
+    g.close()
+""")
