@@ -1112,10 +1112,10 @@ static tm_status rows_get(tm_graph *g, Slot &sl, size_t bytes, int32_t **out) {
     size_t want = std::max<size_t>(1 << 16, sl.rows_bytes * 4);
     while (want < bytes) want *= 4;
     void *p = nullptr;
-    tm_status st = dev_alloc(g, &p, std::min<size_t>(want, TM_ROWS_KEEP));
-    if (st != TM_OK) return st;
-    sl.rows = (int32_t *)p;
-    sl.rows_bytes = std::min<size_t>(want, TM_ROWS_KEEP);
+    if (dev_alloc(g, &p, std::min<size_t>(want, TM_ROWS_KEEP)) == TM_OK) {
+      sl.rows = (int32_t *)p;
+      sl.rows_bytes = std::min<size_t>(want, TM_ROWS_KEEP);
+    }  // (else the call's own size may still fit)
   }
   if (bytes <= sl.rows_bytes) {
     *out = sl.rows;

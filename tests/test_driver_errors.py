@@ -122,3 +122,20 @@ for E in (900, 300_000, 1_100_000):
     assert E < 1_000_000 or fake.fake_unit_shift() == 10
     g.close()
 """)
+
+
+def test_a_listing_that_fits_is_not_refused_for_the_kept_buffer():
+    """The buffer a slot keeps is rounded up; where that does not fit, the listing's own size is taken."""
+    run("""
+g = graph()
+g.enum(MOT, 100, 100)
+for cap in (10_000, 500_000, 1_000_000):
+    room = 12 * cap + 4096
+    fake.fake_limit(fake.fake_used() + room)
+    held = fake.fake_used()
+    for _ in range(3):
+        assert g.enum(MOT, 100, cap)[0] == 0
+    assert fake.fake_used() == held
+    fails(lambda: g.enum(MOT, 100, 2 * cap), 4)
+g.close()
+""")
