@@ -110,7 +110,7 @@ unsigned nblocks(long long n) { return (unsigned)((n + 255) / 256); }
 
 // device buffers of one call, freed on every path: pieces of blocks of at
 // least `block` bytes (an allocation each, 25 per CSR build, took 0.1 ms to
-// make and 0.2 ms to free)
+// make and 0.2 ms to free), or an allocation each with block = 1
 struct Bufs {
   std::vector<void *> p;
   size_t block;
@@ -184,17 +184,21 @@ tm_status start(int32_t device, Stream &st) {
   return TM_OK;
 }
 
-}  // namespace
+// A call's work with its buffers in blocks, and where those do not fit (they
+// hold up to twice what is used) once more with an allocation each.
+template <class F>
+tm_status with_buffers(size_t block, F work) {
+  tm_status s;
+  {
+    Bufs b(block);
+    s = work(b);
+  }
+  if (s != TM_ERR_NOMEM) return s;
+  Bufs b(1);
+  return work(b);
+}
 
-extern "C" {
-
-tm_status tm_time_order(int32_t device, int64_t n, const int32_t *T, int32_t *order) {
-  if (n < 0 || (n > 0 && (!T || !order))) return tmh::set_error(TM_ERR_ARG, "bad argument");
-  if (n > 0x7fffffffll) return tmh::set_error(TM_ERR_ARG, "edge list too long for int32 positions");
-  Stream st;
-  BST(start(device, st));
-  if (n == 0) return TM_OK;
-  Bufs b((size_t)n * 32);
+tm_status time_order(Bufs &b, Stream &st, int64_t n, const int32_t *T, int32_t *order) {
   int *dT, *v0, *v1;
   unsigned *k0, *k1;
   BST(b.get(&dT, n));
@@ -212,22 +216,10 @@ tm_status tm_time_order(int32_t device, int64_t n, const int32_t *T, int32_t *or
   return TM_OK;
 }
 
-tm_status tm_csr_build(int32_t device, int64_t n, const int32_t *U, const int32_t *V, const int32_t *T, int32_t *Eg,
-                       int32_t *outEdgesV, int32_t *inEdgesV, int32_t *outEdgesR, int32_t *inEdgesR,
-                       int32_t *vertexIds, int32_t *numVertices) {
-  if (n < 0 || !numVertices || !outEdgesR || !inEdgesR ||
-      (n > 0 && (!U || !V || !T || !Eg || !outEdgesV || !inEdgesV || !vertexIds)))
-    return tmh::set_error(TM_ERR_ARG, "bad argument");
-  if (n > 0x3fffffffll) return tmh::set_error(TM_ERR_ARG, "edge list too long for int32 endpoint slots");
-  Stream st;
-  BST(start(device, st));
-  if (n == 0) {
-    *numVertices = 0;
-    outEdgesR[0] = inEdgesR[0] = 0;
-    return TM_OK;
-  }
+tm_status csr_build(Bufs &b, Stream &st, int64_t n, const int32_t *U, const int32_t *V, const int32_t *T, int32_t *Eg,
+                    int32_t *outEdgesV, int32_t *inEdgesV, int32_t *outEdgesR, int32_t *inEdgesR, int32_t *vertexIds,
+                    int32_t *numVertices) {
   const long long m = 2 * n;
-  Bufs b((size_t)n * 160);
   int *dU, *dV, *dT, *slot0, *slot1, *head, *grp, *rawk, *order, *gidx, *rank, *raw, *Un, *Vn, *dEg, *pos, *P, *R;
   unsigned *key0, *key1, *first, *first1;
   BST(b.get(&dU, n));
@@ -298,6 +290,38 @@ tm_status tm_csr_build(int32_t device, int64_t n, const int32_t *U, const int32_
   }
   *numVertices = nv;
   return TM_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+tm_status tm_time_order(int32_t device, int64_t n, const int32_t *T, int32_t *order) {
+  if (n < 0 || (n > 0 && (!T || !order))) return tmh::set_error(TM_ERR_ARG, "bad argument");
+  if (n > 0x7fffffffll) return tmh::set_error(TM_ERR_ARG, "edge list too long for int32 positions");
+  Stream st;
+  BST(start(device, st));
+  if (n == 0) return TM_OK;
+  return with_buffers((size_t)n * 32, [&](Bufs &b) { return time_order(b, st, n, T, order); });
+}
+
+tm_status tm_csr_build(int32_t device, int64_t n, const int32_t *U, const int32_t *V, const int32_t *T, int32_t *Eg,
+                       int32_t *outEdgesV, int32_t *inEdgesV, int32_t *outEdgesR, int32_t *inEdgesR,
+                       int32_t *vertexIds, int32_t *numVertices) {
+  if (n < 0 || !numVertices || !outEdgesR || !inEdgesR ||
+      (n > 0 && (!U || !V || !T || !Eg || !outEdgesV || !inEdgesV || !vertexIds)))
+    return tmh::set_error(TM_ERR_ARG, "bad argument");
+  if (n > 0x3fffffffll) return tmh::set_error(TM_ERR_ARG, "edge list too long for int32 endpoint slots");
+  Stream st;
+  BST(start(device, st));
+  if (n == 0) {
+    *numVertices = 0;
+    outEdgesR[0] = inEdgesR[0] = 0;
+    return TM_OK;
+  }
+  return with_buffers((size_t)n * 160, [&](Bufs &b) {
+    return csr_build(b, st, n, U, V, T, Eg, outEdgesV, inEdgesV, outEdgesR, inEdgesR, vertexIds, numVertices);
+  });
 }
 
 }  // extern "C"

@@ -24,6 +24,7 @@ static size_t used, peak, limit = (size_t)-1;
 static char fail_kernel[64];
 static int fail_kernel_after, fail_host, fail_record, fail_sync, fail_stream;
 static unsigned long long head_pairs;
+static int word_on, word;           /* what a 4-byte copy to the host brings */
 static char trace[1 << 16];
 static tm_kernel_args mined;       /* of the last mining launch */
 
@@ -32,6 +33,7 @@ void fake_fail_host(int on) { fail_host = on; }
 void fake_fail_record(int on) { fail_record = on; }
 void fake_fail_sync(int stream) { fail_sync = 1; fail_stream = stream; }
 void fake_limit(size_t bytes) { limit = bytes; }
+void fake_word(int v) { word_on = 1; word = v; }
 void fake_pairs(unsigned long long n) { head_pairs = n; }
 int fake_unit_shift(void) { return mined.unit_shift; }
 int fake_claim_blocks(void) { return mined.claim_blocks; }
@@ -73,7 +75,11 @@ hipError_t hipFree(void *p) { return drop(p); }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned f) { (void)f; return fail_host ? ret(hipErrorOutOfMemory) : take(p, n, 1); }
 hipError_t hipHostFree(void *p) { return drop(p); }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind k) { (void)k; memmove(d, s, n); return hipSuccess; }
-hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t t) { (void)k; memmove(d, s, n); pending[sid(t)]++; return hipSuccess; }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t t) {
+  if (word_on && n == 4 && k == hipMemcpyDeviceToHost) *(int *)d = word; else memmove(d, s, n);
+  pending[sid(t)]++;
+  return hipSuccess;
+}
 hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t t) { memset(d, v, n); pending[sid(t)]++; return hipSuccess; }
 hipError_t hipStreamCreate(hipStream_t *s) { *s = (hipStream_t)(size_t)(1 + nstream++); return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t s) { (void)s; return hipSuccess; }

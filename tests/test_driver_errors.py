@@ -139,3 +139,37 @@ for cap in (10_000, 500_000, 1_000_000):
     fails(lambda: g.enum(MOT, 100, 2 * cap), 4)
 g.close()
 """)
+
+
+@pytest.mark.parametrize("nv", [1000, 1_400_000, 2_000_000])
+def test_a_build_that_fits_is_not_refused_for_its_blocks(nv):
+    """The build's buffers come in blocks of up to twice what is used; where those do not fit it takes each by
+    itself, so the memory it needs is the sum of what it uses."""
+    run("""
+n, nv = 1_000_000, %d
+x = np.zeros(n, np.int32)
+fake.fake_word(nv)
+def build():
+    return abi.csr_build(x, x, x)["V"]
+def order():
+    return abi.time_order(x).size
+def need(call):  # the least memory the call runs in
+    lo, hi = 0, 512 * n
+    while hi - lo > 4096:
+        mid = (lo + hi) // 2
+        fake.fake_limit(mid)
+        try:
+            call()
+            hi = mid
+        except abi.TMError:
+            lo = mid
+    return hi
+for call, words in ((build, 3 + 6 * 2 + 2 + 3 + 2 + 8 * nv / n), (order, 5)):
+    got = need(call)
+    print(got / n, words * 4)
+    assert words * 4 * n <= got <= words * 4 * n + 52 * n, (got / n, words * 4)  # (and the sorts' own)
+    for more in (0, 1, 5, 20, 60, 160, 400):  # nothing between is refused
+        fake.fake_limit(got + more * n)
+        call()
+    assert fake.fake_used() == 0
+""" % nv)
