@@ -254,7 +254,7 @@ __global__ void __launch_bounds__(256) heads_kernel(const unsigned long long *__
 // The pair table's entries: the first slot of each run claims a place by its
 // key and writes the run's slots.
 __global__ void pair_table_kernel(const unsigned long long *__restrict__ k, int n, unsigned long long *tab,
-                                  unsigned mask) {
+                                  unsigned size) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n || (i > 0 && k[i] == k[i - 1])) return;
   const unsigned long long key = k[i];
@@ -271,7 +271,7 @@ __global__ void pair_table_kernel(const unsigned long long *__restrict__ k, int 
   }
   const int x = (int)(unsigned)(key >> 32), y = (int)(unsigned)key;
   const unsigned long long word = ((unsigned long long)(unsigned)y << 32) | (unsigned)x;  // {x, y} in memory
-  for (unsigned h = tm_pair_hash(x, y) & mask;; h = (h + 1) & mask)
+  for (unsigned h = tm_pair_place(x, y, size);; h = h + 1 < size ? h + 1 : 0)
     if (atomicCAS(tab + 2 * (size_t)h, ~0ull, word) == ~0ull) {
       tab[2 * (size_t)h + 1] = ((unsigned long long)(unsigned)hi << 32) | (unsigned)i;
       return;
@@ -1440,7 +1440,10 @@ tm_status tm_graph_upload(int32_t device, const tm_host_graph *hg, tm_graph **ou
   hipLaunchKernelGGL(low_word_kernel, dim3((E + 255) / 256), dim3(256), 0, s, skey, (int *)vw.outPairNbr, E);
   TMPCHK(hipGetLastError());
   {
-    // the pair table, at most half full
+    // the pair table, at most half full: the next power of two (about 0.4 full; a
+    // 5-cycle on 3.1M hub edges takes 1% more at 0.5) where that is an eighth of
+    // the free memory at most, else no more than two entries per edge: a graph
+    // that fills the memory gets 8 words an edge, not up to 16
     unsigned long long pairs = 0, *d_pairs = okey;  // (okey is not needed any more)
     TMPCHK(hipMemsetAsync(d_pairs, 0, sizeof(pairs), s));
     hipLaunchKernelGGL(heads_kernel, dim3((E + 255) / 256), dim3(256), 0, s, skey, E, d_pairs);
@@ -1449,12 +1452,15 @@ tm_status tm_graph_upload(int32_t device, const tm_host_graph *hg, tm_graph **ou
     TMPCHK(hipStreamSynchronize(s));
     size_t n = 4;
     while (n < 2 * (size_t)pairs) n <<= 1;
+    size_t room = 0, all = 0;
+    if (hipMemGetInfo(&room, &all) != hipSuccess) room = 0;
+    if (16 * n > room / 8) n = std::min(n, std::max<size_t>(4, 2 * (size_t)E));
     if ((st = dev_alloc(g, &p, 16 * n)) != TM_OK) { free_tmp(); return cleanup(st); }
     vw.ptab = (const int *)p;
-    vw.pmask = (unsigned)(n - 1);
+    vw.psize = (unsigned)n;
     TMPCHK(hipMemsetAsync(p, 0xff, 16 * n, s));
     hipLaunchKernelGGL(pair_table_kernel, dim3((E + 255) / 256), dim3(256), 0, s, skey, E, (unsigned long long *)p,
-                       vw.pmask);
+                       vw.psize);
     TMPCHK(hipGetLastError());
   }
   {

@@ -231,7 +231,7 @@ __device__ __forceinline__ int gallop_ub(const int *__restrict__ a, int lo, int 
 // edges 17.1 -> 9.3 ms, all 3-edge motifs on 100k edges 9.9 -> 6.2 ms of kernels).
 __device__ __forceinline__ bool pair_find(const tm_graph_view &g, int x, int y, int *s0, int *s1,
                                           Meter *mt = nullptr) {
-  for (unsigned h = tm_pair_hash(x, y) & g.pmask;; h = (h + 1) & g.pmask) {
+  for (unsigned h = tm_pair_place(x, y, g.psize);; h = h + 1 < g.psize ? h + 1 : 0) {
     if (mt) mt->b += 16;
     const int4 e = ((const int4 *)g.ptab)[h];
     if (e.x == x && e.y == y) {

@@ -7,7 +7,8 @@
 #define TM_MAXE 8  // most motif edges handled (the reference register stack: 8-bit stackio)
 #define TM_MAXN 8  // most motif nodes handled
 
-// Pair table hash of a graph pair (multiply and fold; any fixed mix would do).
+// Pair table hash of a graph pair (multiply and fold; any fixed mix would do),
+// and the place it has in a table of n entries (any n: its share of the range).
 #ifdef __HIPCC__
 __host__ __device__
 #endif
@@ -15,6 +16,12 @@ static inline unsigned tm_pair_hash(int x, int y) {
   unsigned h = (unsigned)x * 0x9e3779b1u + (unsigned)y;
   h = (h ^ (h >> 15)) * 0x85ebca6bu;
   return h ^ (h >> 13);
+}
+#ifdef __HIPCC__
+__host__ __device__
+#endif
+static inline unsigned tm_pair_place(int x, int y, unsigned n) {
+  return (unsigned)(((unsigned long long)tm_pair_hash(x, y) * n) >> 32);
 }
 
 // How motif edge j (j >= 1) extends a partial match.
@@ -73,12 +80,12 @@ typedef struct {
   const int *outR, *outPos, *outNbr;  // out CSR: offsets, positions (outEdgesV), destinations
   const int *inR, *inPos, *inNbr;     // in CSR: offsets, positions (inEdgesV), sources
   const int *outPairNbr, *outPairPos; // per node, out-list re-sorted by (dst, position)
-  // The pair table: open addressing by tm_pair_hash, linear probing, pmask + 1
-  // entries (a power of two, at least twice the distinct pairs) of 4 ints:
+  // The pair table: open addressing by tm_pair_hash, linear probing, psize
+  // entries (at least twice the distinct pairs) of 4 ints:
   // {x, y, s0, s1}, the pair x -> y holding slots [s0, s1) of the pair index;
   // x = -1: empty
   const int *ptab;
-  unsigned pmask;
+  unsigned psize;
   const int *outSelf;     // slot of position p in out(src of p)
   const int *inSelf;      // slot of position p in in(dst of p)
   const int *outNext;     // first slot of out(dst of p) with position > p

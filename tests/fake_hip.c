@@ -72,6 +72,7 @@ static hipError_t drop(void *p) {
 
 hipError_t hipMalloc(void **p, size_t n) { return take(p, n, 0); }
 hipError_t hipFree(void *p) { return drop(p); }
+hipError_t hipMemGetInfo(size_t *f, size_t *a) { *a = limit; *f = limit > used ? limit - used : 0; return hipSuccess; }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned f) { (void)f; return fail_host ? ret(hipErrorOutOfMemory) : take(p, n, 1); }
 hipError_t hipHostFree(void *p) { return drop(p); }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind k) { (void)k; memmove(d, s, n); return hipSuccess; }

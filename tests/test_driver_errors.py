@@ -173,3 +173,22 @@ for call, words in ((build, 3 + 6 * 2 + 2 + 3 + 2 + 8 * nv / n), (order, 5)):
         call()
     assert fake.fake_used() == 0
 """ % nv)
+
+
+@pytest.mark.parametrize("E", [30_000, 70_000, 300_000])
+def test_the_pair_table_takes_two_entries_per_edge_where_memory_is_short(E):
+    """Of 16 bytes, however many of the pairs are distinct: a graph that fills the memory is not refused for it."""
+    run("""
+E = %d
+fake.fake_pairs(1)
+g = graph(E, max(4, E // 4))
+few = g.info()["device_bytes"]
+g.close()
+fake.fake_limit(few + 64 * E + (1 << 20))  # (the upload's own keys and sort among it)
+for pairs in (E // 2 + 1, 2 * E // 3, E):
+    fake.fake_pairs(pairs)
+    g = graph(E, max(4, E // 4))
+    more = g.info()["device_bytes"] - few + 64
+    assert 32 * pairs <= more <= max(64, 32 * E), (pairs, more / E)
+    g.close()
+""" % E)
