@@ -107,7 +107,7 @@ __global__ void __launch_bounds__(256) check_slots_kernel(const tm_edge *__restr
     const int x = side ? Eg[p].v : Eg[p].u;
     if (x >= 0 && x < V) {
       if (s < R[x] || s >= R[x + 1]) b |= V_CSR << 3;
-      else if (s > R[x] && P[s - 1] >= p) b |= V_CSR << 4;
+      else if (s > max(R[x], 0) && P[s - 1] >= p) b |= V_CSR << 4;
     }
   }
   if (b) atomicOr(bad, b << (side * V_CSR_SIDE));
