@@ -291,11 +291,12 @@ bool launch_next(tm_server *s, int k) {
   return true;
 }
 
-// Collect a lane whose launch has completed; called with s->mu held.
-void complete(tm_server *s, int k) {
+// Collect a lane whose launch has completed, or failed with `he` (the pinned
+// results are then an earlier launch's); called with s->mu held.
+void complete(tm_server *s, int k, hipError_t he) {
   Lane &ln = s->lane[k];
   Slot &sl = s->g->slot[k];
-  const tm_status st = collect(s->g, sl, 0);
+  const tm_status st = he == hipSuccess ? collect(s->g, sl, 0) : lane_error("server launch", he);
   const std::vector<uint64_t> counts(sl.s.h_counts, sl.s.h_counts + ln.ids.size());  // (a cut below reuses them)
   for (size_t i = 0; i < ln.ids.size(); i++) {
     Request &r = *s->reqs[ln.ids[i]];
@@ -369,11 +370,11 @@ void dispatcher(tm_server *s, std::mutex *ready_mu, std::condition_variable *rea
       if (!ln.busy) continue;
       const hipError_t q = hipEventQuery(ln.done);
       if (q == hipSuccess) {
-        complete(s, k);
+        complete(s, k, hipSuccess);
         progress = true;
       } else if (q != hipErrorNotReady) {
         (void)hipEventSynchronize(ln.done);  // an error: drain the lane, report per request
-        complete(s, k);
+        complete(s, k, q);
         progress = true;
       } else {
         busy++;

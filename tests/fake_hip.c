@@ -22,7 +22,7 @@ static int pending[MAXS], nstream;   /* launches and copies not waited for, per 
 static hipError_t last;
 static size_t used, peak, limit = (size_t)-1;
 static char fail_kernel[64];
-static int fail_kernel_after, fail_host, fail_record, fail_sync, fail_stream;
+static int fail_kernel_after, fail_host, fail_record, fail_sync, fail_stream, fail_query;
 static unsigned long long head_pairs;
 static int word_on, word;           /* what a 4-byte copy to the host brings */
 static char trace[1 << 16];
@@ -32,6 +32,7 @@ void fake_fail_kernel(const char *part, int after) { snprintf(fail_kernel, sizeo
 void fake_fail_host(int on) { fail_host = on; }
 void fake_fail_record(int on) { fail_record = on; }
 void fake_fail_sync(int stream) { fail_sync = 1; fail_stream = stream; }
+void fake_fail_query(int n) { fail_query = n; }
 void fake_limit(size_t bytes) { limit = bytes; }
 void fake_word(int v) { word_on = 1; word = v; }
 void fake_pairs(unsigned long long n) { head_pairs = n; }
@@ -94,7 +95,7 @@ hipError_t hipEventCreate(hipEvent_t *e) { *e = (hipEvent_t)(size_t)++events; re
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned f) { (void)f; return hipEventCreate(e); }
 hipError_t hipEventDestroy(hipEvent_t e) { (void)e; return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) { (void)e; (void)s; if (fail_record > 0 && --fail_record == 0) return ret(hipErrorUnknown); return hipSuccess; }
-hipError_t hipEventQuery(hipEvent_t e) { (void)e; return hipSuccess; }
+hipError_t hipEventQuery(hipEvent_t e) { (void)e; return fail_query > 0 && fail_query-- ? ret(hipErrorUnknown) : hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t e) { (void)e; return hipSuccess; }
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t a, hipEvent_t b) { (void)a; (void)b; *ms = 1; return hipSuccess; }
 hipError_t hipGetLastError(void) { hipError_t e = last; last = hipSuccess; return e; }

@@ -192,3 +192,19 @@ for pairs in (E // 2 + 1, 2 * E // 3, E):
     assert 32 * pairs <= more <= max(64, 32 * E), (pairs, more / E)
     g.close()
 """ % E)
+
+
+@pytest.mark.parametrize("cap", [-1, 50])
+def test_a_failed_served_launch_is_not_answered_with_an_earlier_one(cap):
+    """When the wait for a launch reports an error, its results were never written."""
+    run("""
+g = graph()
+s = abi.Server(g, slots=1)
+assert s.wait(s.submit(MOT, 100, %d), 5000)["status"] == 0
+fake.fake_fail_query(1)
+r = s.wait(s.submit(MOT, 100, %d), 5000)
+assert r["status"] == 3, r
+assert s.wait(s.submit(MOT, 100, %d), 5000)["status"] == 0
+s.close()
+g.close()
+""" % (cap, cap, cap))
