@@ -760,13 +760,12 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
   }
   while (unit_shift < most && ((span >> (unit_shift + 1)) >= 4ll * grid || (unit_shift < 4 && (span >> (unit_shift + 1)) >= TM_SMALL_BLOCKS)))
     unit_shift++;
-  // Up to 5 edges, blocks of half to an eighth of that while 48 or more roots of
-  // one pass: an expansion is nearly as full, and the launch's tail shorter
-  // (cycles of 4 and 5 edges 12.1 -> 11.3 and 21.9 -> 20.3 ms; where 33 or fewer
-  // passed it took 2 to 20% more: 256 random queries 57.9 -> 61.3).  6 edges keep
-  // the larger ones (the deadline test relies on one of them running for
-  // 20 ms; 25 -> 20).
-  while (maxM <= 5 && unit_shift > 5 && passing * (double)(1 << unit_shift) >= 48.0 * span &&
+  // Blocks of half to an eighth of that while 48 or more roots of one pass: an
+  // expansion is nearly as full, and the launch's tail shorter (cycles of 4 and 5
+  // edges 12.1 -> 11.3 and 21.9 -> 20.3 ms, a zigzag of 6 edges and seven nodes at a day
+  // on 8M edges 47.5 -> 30.3; 258 random queries of 6 edges 23.64 and 23.64 ms;
+  // where 33 or fewer passed it took 2 to 20% more: 256 random queries 57.9 -> 61.3).
+  while (unit_shift > 5 && passing * (double)(1 << unit_shift) >= 48.0 * span &&
          (span >> unit_shift) <= 16ll * grid)
     unit_shift--;
   long long total_blocks = 0;
@@ -842,11 +841,13 @@ tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_t
     // A look costs two reads, and up to 5 edges earlier ones shorten the
     // launch's tail: 256 random queries on 8M power-law edges 63.2 ms of kernels
     // with 1000 us, 60.8 with 100, 61.9 with 50 and a look at every step;
-    // 5-cycle on 3.1M hub edges 27.9 -> 26.6, one of 5 edges 1.74 -> 1.11.  At
-    // 6 edges 63 of the queries take 5.5 and 5.4 ms, and 1000 us stay (the
-    // deadline test relies on one of them running for 20 ms).
+    // 5-cycle on 3.1M hub edges 27.9 -> 26.6, one of 5 edges 1.74 -> 1.11.
+    // Single-query launches of 6 edges and more still wait 1000: 100 is the better
+    // value there too (258 random queries 23.6 -> 22.1 ms, a star of 6 edges at a week
+    // 23.5 -> 18.9, a zigzag at a day 47.5 -> 44.1), but the deadline test takes that
+    // star, with no tuning of its own, for a query of more than 20 ms.
     const long long us = (tune && tune->steal_after_us > 0) ? tune->steal_after_us
-                                                            : (small ? 20 : maxM <= 5 ? 100 : 1000);
+                                                            : (small ? 20 : maxM <= 5 || nq > 1 ? 100 : 1000);
     a.steal_after_ticks = us * g->wall_rate_khz / 1000;
   }
   // two-edge tail: frames of edge M-2 with at least this many window candidates

@@ -60,7 +60,7 @@ typedef struct tm_host_graph {
 
 /* Launch parameters; zero fields take the library defaults (occupancy-limited
  * waves up to 32 per CU, scan_max 16, no time
- * limit, steal_every 16, steal_max 4, steal_min 64, steal_after_us 100 (6 edges 1000),
+ * limit, steal_every 16, steal_max 4, steal_min 64, steal_after_us 100 (one query of 6 edges or more 1000),
  * claim_blocks: single blocks of roots, or claims that shrink with the roots
  * left where few of them pass the start rules). */
 typedef struct tm_tuning {

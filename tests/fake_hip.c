@@ -36,6 +36,9 @@ void fake_fail_query(int n) { fail_query = n; }
 void fake_limit(size_t bytes) { limit = bytes; }
 void fake_word(int v) { word_on = 1; word = v; }
 void fake_pairs(unsigned long long n) { head_pairs = n; }
+static int gaps;                      /* edges in every rule's gap histogram */
+void fake_gaps(int n) { gaps = n; }
+long long fake_steal_ticks(void) { return mined.steal_after_ticks; }
 int fake_unit_shift(void) { return mined.unit_shift; }
 int fake_claim_blocks(void) { return mined.claim_blocks; }
 size_t fake_used(void) { return used; }
@@ -79,6 +82,8 @@ hipError_t hipHostFree(void *p) { return drop(p); }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind k) { (void)k; memmove(d, s, n); return hipSuccess; }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t t) {
   if (word_on && n == 4 && k == hipMemcpyDeviceToHost) *(int *)d = word; else memmove(d, s, n);
+  if (gaps && n == sizeof(unsigned) * TM_NTFIRST * 33 && k == hipMemcpyDeviceToHost)
+    for (int r = 0; r < TM_NTFIRST; r++) ((unsigned *)d)[33 * r + 3] = gaps;
   pending[sid(t)]++;
   return hipSuccess;
 }

@@ -18,6 +18,7 @@ fake.fake_used.restype = fake.fake_peak.restype = ctypes.c_size_t
 fake.fake_trace.restype = ctypes.c_char_p
 fake.fake_limit.argtypes = [ctypes.c_size_t]
 fake.fake_pairs.argtypes = [ctypes.c_ulonglong]
+fake.fake_steal_ticks.restype = ctypes.c_longlong
 sys.path[:0] = [%r, %r]
 import numpy as np
 from everest_amd import abi

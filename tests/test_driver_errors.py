@@ -208,3 +208,23 @@ assert s.wait(s.submit(MOT, 100, %d), 5000)["status"] == 0
 s.close()
 g.close()
 """ % (cap, cap, cap))
+
+
+def test_launch_rules_are_the_same_for_deep_motifs():
+    """Block sizes go by how many roots pass, whatever the motif's edges; queries of one launch share their
+    deepest one's stack, not a wait of its own."""
+    run("""
+E = 400_000
+fake.fake_gaps(E)
+g = graph(E, E // 20)
+chain = [(0, 1, 0), (1, 2, 1), (2, 0, 2), (0, 3, 3), (3, 1, 4), (1, 0, 5), (2, 3, 6), (3, 0, 7)]
+for waves in (0, 2):
+    shift = []
+    for M in (4, 5, 6, 7, 8):
+        g.count(chain[:M], 3600, tune=abi.tuning(waves_per_cu=waves, sweep=-1))
+        shift.append(fake.fake_unit_shift())
+    assert len(set(shift)) == 1, shift
+g.batch_count([(chain[:3], 3600), (chain[:6], 3600)], tune=abi.tuning(batch_mode=2))
+assert fake.fake_steal_ticks() == 100 * 100, fake.fake_steal_ticks()
+g.close()
+""")
