@@ -776,11 +776,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
   const int home_stripe = blockIdx.x & (TM_STRIPES - 1);
   int cstripe = home_stripe;  // the stripe that counts this wavefront's busy credit
   int at_stripe = home_stripe;  // the stripe it claims from
-  // The blocks go to the stripes in turn, a 64th of them at a time: a stripe's
+  // The blocks go to the stripes in turn, a 64th of a query's at a time: a stripe's
   // wavefronts (one XCD's) work close to each other in time, where hubs'
   // windows overlap in its L2 (single blocks in turn: 28% slower for
-  // 0->1, 1->2, 2->3 on 2M hub edges), and a busy period is shared by all.
-  const int nblocks = (int)args.total_blocks, seg = max(1, nblocks / (8 * TM_STRIPES));
+  // 0->1, 1->2, 2->3 on 2M hub edges), and a busy period is shared by all, as is
+  // a heavy query among many (a 64th of all blocks at a time held it in one or two
+  // stripes: 63 queries of 6 edges on 8M edges in one launch 10.1 ms
+  // with claims of 1024 roots in query order, 21.4 so, 6.1 now).
+  const int nblocks = (int)args.total_blocks, seg = max(1, nblocks / (8 * TM_STRIPES * (MULTI ? args.nq : 1)));
   bool scout = false;           // looks at the other stripes and may wait for donations
   long long look_t0 = work_t0;  // wall clock when it last looked for idle wavefronts, or took its work
   bool told = false;       // told the stripes that it waits

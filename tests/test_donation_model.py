@@ -13,13 +13,13 @@ STRIPES = 8
 
 class Launch:
     def __init__(self, rng, grid, work, claim_blocks, cap=None, idle_cap=4, scouts=2, steal_max=2, steal_min=1,
-                 drop_claim=True, root_query=0):
+                 drop_claim=True, root_query=0, nq=1):
         """work[b]: candidates of root block b (0: no root of it passes).  drop_claim and root_query: what a
         wavefront that sees the stop flag does with its claim (True: drops it), and the query word of a record of
         root blocks (None: the donor's own)."""
         self.rng, self.grid, self.work, self.cap = rng, grid, work, cap
         self.nblocks = len(work)
-        self.seg = max(1, self.nblocks // (8 * STRIPES))
+        self.seg = max(1, self.nblocks // (8 * STRIPES * nq))   # (nq queries in the launch)
         self.claim_blocks, self.idle_cap, self.scouts = claim_blocks, idle_cap, scouts
         self.steal_max, self.steal_min = steal_max, steal_min
         self.drop_claim, self.root_query = drop_claim, root_query
@@ -222,7 +222,7 @@ def random_launch(rng, listing, **kw):
     cap = int(rng.integers(1, max(2, int(work.sum())))) if listing else None
     return Launch(rng, int(rng.integers(1, 40)), work.tolist(), int(rng.integers(1, 33)), cap,
                   idle_cap=int(rng.integers(1, 8)), scouts=int(rng.integers(1, 4)),
-                  steal_max=int(rng.integers(1, 3)), **kw)
+                  steal_max=int(rng.integers(1, 3)), nq=int(rng.integers(1, 6)), **kw)
 
 
 def settle(L):
@@ -262,3 +262,20 @@ def test_a_claim_kept_at_the_stop_flag_loses_a_credit():
     with pytest.raises(AssertionError, match="a record of"):
         for _ in range(600):
             settle(random_launch(rng, True, drop_claim=False, root_query=None))
+
+
+def test_every_query_of_a_launch_is_spread_over_the_stripes():
+    """The blocks of any one query: no stripe holds more than twice its share (a stripe's wavefronts alone take a
+    heavy query's blocks there)."""
+    rng = np.random.default_rng(8)
+    for _ in range(60):
+        nq = int(rng.integers(1, 200))
+        per = int(rng.integers(64, 500))
+        L = Launch(rng, 40, [0] * (nq * per), 1, nq=nq)
+        stripe = np.zeros(L.nblocks, dtype=int)
+        for k in range(STRIPES):
+            for i in range(L.blocks_of(k)):
+                stripe[L.block(k, i)] = k
+        for q in range(nq):
+            share = np.bincount(stripe[q * per:(q + 1) * per], minlength=STRIPES) / per
+            assert share.max() <= 2 / STRIPES, (nq, per, q, share)
