@@ -31,9 +31,10 @@ AXES = [
     ("sb_flush", [0, -1, 48, 64]),          # survivor compaction (0 = 32 where it costs no occupancy)
     ("sb_inline", [0, 16, 48]),             # survivors a step expands itself with none buffered (0 = 32)
     ("scan_max", [0, 8, 32]),               # last-edge ranges scanned up to this size (0 = 16)
-    ("claim_blocks", [0, 1, 2, 8, 32]),     # 256-root blocks per claim (0 = half of what is left, shared out)
+    ("claim_blocks", [0, 1, 2, 8, 32]),     # 256 roots each per claim (0 = single blocks where many roots pass, else half
+                                            # of what is left, shared out)
     ("waves_per_cu", [0, 16, 24]),          # resident wavefronts per CU (0 = occupancy-limited, <= 32)
-    ("steal_after_us", [0, 250, 4000]),     # donation trigger (0 = 100 us, 6 edges 1000)
+    ("steal_after_us", [0, 250, 4000]),     # donation trigger (0 = 100 us, 6 edges and more 1000)
     ("steal_min", [0, 16, 256]),            # smallest donated half-frame (0 = 64 candidates)
     ("steal_max", [0, 2, 8]),               # frames donated per look (0 = 4)
 ]

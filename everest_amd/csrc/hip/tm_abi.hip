@@ -914,7 +914,7 @@ tm_status enqueue(tm_graph *g, Slot &sl, const Plan &pl, bool timing, bool count
       return st;
   }
   // the window sweep after the mining kernel on the same stream: it adds
-  // its queries' counts to the slots the reset kernel cleared
+  // its queries' counts to the slots the stage kernel cleared
   for (size_t i = 0; i < pl.sweep.size(); i += TM_SWEEP_MAXQ) {
     SweepBatch b;
     b.n = (int)std::min<size_t>(TM_SWEEP_MAXQ, pl.sweep.size() - i);

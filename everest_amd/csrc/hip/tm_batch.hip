@@ -104,7 +104,7 @@ tm_status tm_batch_prepare(tm_graph *g, int32_t nq, const int32_t *num_edges, co
   // an eager tm_batch_count after them did not finish.  The cause is not
   // established (the captured launches share scheduler state and the
   // donation ring with eager launches; whether the kernel boundaries inside
-  // a replayed graph make the reset kernel's stores visible to the next
+  // a replayed graph make the first kernel's stores visible to the next
   // launch on every XCD is not known here).  Until it is, prepared batches
   // are refused rather than risk a hang; tm_batch_count is unaffected.
   if (!tm_batch_graphs_enabled())

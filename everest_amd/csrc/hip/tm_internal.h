@@ -129,8 +129,9 @@ struct Plan {
 tm_status plan(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_tuning *tune, int instr, bool multi,
                tm_launch_fn fn, void *user, Plan *pl);
 // Enqueue a planned launch on the slot's stream: ring clear when the
-// generation wraps (host side), reset kernel, mining kernel (between the
-// slot's timing events when timing), statistics kernel.
+// generation wraps (host side), stage kernel (tables from the pinned staging,
+// scheduler cleared), mining and sweep kernels (between the slot's timing
+// events when timing), finish kernel (counters summed, results to the pinned side).
 tm_status enqueue(tm_graph *g, Slot &sl, const Plan &pl, bool timing, bool count);
 // plan + enqueue (multi: the batch kernel; fn: a caller's kernel).
 tm_status launch(tm_graph *g, Slot &sl, int q0, int nq, bool enumerate, const tm_tuning *tune, int instr,

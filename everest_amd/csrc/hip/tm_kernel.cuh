@@ -743,7 +743,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
 
   const tm_graph_view &g = *args.gv;
   tm_sched *sched = args.sched;
-  const int gen = ld_rlx(&sched->gen);  // advanced by the reset kernel before this launch
+  const int gen = ld_rlx(&sched->gen);  // advanced by the stage kernel before this launch
   const unsigned long long lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
 
   unsigned long long cnt = 0;
@@ -1043,7 +1043,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     for (int i = 0; i < MAXN; i++) m[i] = 0;
     if (top == 0 && sbn == 0) {
       // ---------------------------------------------------- root dispatch
-      // The launch's roots form one space of blocks of 16 to 1024 roots
+      // The launch's roots form one space of blocks of 4 to 1024 roots
       // (args.unit_shift), query after query.  Lane l holds roots 4 l .. 4 l + 3
       // of each 256-root row of a block and reads their gaps under each of the
       // query's rules with one 16-byte load, all rows of a rule in flight
@@ -1816,7 +1816,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
   if (lane == 0 && !is_idle) add_rlx(&sched->stripe[cstripe].busy, -1);  // left early holding work (error or deadline)
   if (lane == 0 && waiter) add_rlx(&sched->waiters, -1);
   // work counters: plain stores into this wavefront's own slot, summed by a
-  // one-block kernel after the launch (no same-address atomics from every wave)
+  // the finish kernel after the launch (no same-address atomics from every wave)
   {
     unsigned long long v = 0;
     switch (lane) {

@@ -143,7 +143,7 @@ typedef struct {
   int error;        // bit 0: frame stack overflow, bit 1: empty frame, bit 2: deadline passed,
                     // bit 3: a donated frame never became ready
   int abort;        // set once the deadline passed: every wavefront stops
-  long long t0;     // wall clock at launch (set by the reset kernel)
+  long long t0;     // wall clock at launch (set by the stage kernel)
   unsigned long long stats[16];  // work counters (see TM_STAT_*), summed after the launch
   int summed;       // blocks of the finish kernel done with them
   int pad5[31];
@@ -155,7 +155,7 @@ typedef struct {
   int pad1[31];
   int waiters;      // wavefronts waiting for donations (at most idle_cap)
   int pad4[31];
-  int gen;          // launch generation of the donation ring: the reset kernel advances it,
+  int gen;          // launch generation of the donation ring: the stage kernel advances it,
                     // so replays of a captured launch get fresh tags
   int pad3[31];
 } tm_sched;
@@ -211,7 +211,7 @@ typedef struct {
   const tm_query_dev *queries;
   // 4 ints per query: (delta, root_beg, root_end, start rule of edge 1)
   const int *qtab;
-  // The launch's roots as one space of blocks of 1 << unit_shift roots (16 to
+  // The launch's roots as one space of blocks of 1 << unit_shift roots (4 to
   // 1024), query after query: query q owns blocks [block_prefix[q],
   // block_prefix[q + 1]), its block i starting at root (root_beg & ~3) +
   // (i << unit_shift) (nq + 1 entries).

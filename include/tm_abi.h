@@ -329,9 +329,9 @@ tm_status tm_set_class_tuning(tm_graph *g, int32_t cls, const tm_tuning *tune);
  * Count many motif queries on one graph in one call.  Query q uses edges
  * msrc/mdst[q * TM_MAX_MOTIF_EDGES ...], num_edges[q], deltas[q] and roots
  * [0, E - num_edges[q] + 1).  counts[q] receives the exact count, equal to
- * tm_count of the same query.  The queries are grouped by stack depth; each
- * group is one persistent launch of the batch kernel with the whole GPU, the
- * groups one after another.  No
+ * tm_count of the same query.  tm_tuning.batch_mode chooses between a launch
+ * per query, over the graph's launch slots in turn (0), and launches of the
+ * batch kernel, one per stack depth after another (1) or one for all (2).  No
  * reference counterpart: the reference runs one generated worker per query
  * (system/batch-query.py:12-19).
  */
@@ -342,8 +342,9 @@ tm_status tm_batch_count(tm_graph *g, int32_t nq, const int32_t *num_edges,
 /*
  * tm_batch_count for callers that cannot allocate device memory: code under
  * HIP graph capture, serving loops and harnesses that own every device
- * allocation.  No counterpart in the reference.  Same queries, launches and
- * results as tm_batch_count, for at most TM_NOALLOC_MAXQ queries per call
+ * allocation.  No counterpart in the reference.  Same queries and results
+ * as tm_batch_count, launched as its batch_mode 1, for at most
+ * TM_NOALLOC_MAXQ queries per call
  * (TM_ERR_ARG beyond).  Every device buffer of its launches (scheduler
  * state, query tables, counts, per-wavefront counters, a donation ring of
  * up to 2^15 records) lives in one static device array of
@@ -361,8 +362,8 @@ tm_status tm_batch_count_noalloc(tm_graph *g, int32_t nq, const int32_t *num_edg
 
 /*
  * A prepared batch: the queries of tm_batch_count planned once, their tables
- * uploaded, and the whole set of per-class launches (reset, mining kernel,
- * statistics, result copies, on the graph's slot streams) captured into one
+ * uploaded, and the whole set of per-class launches (stage, search and finish
+ * kernels, on the graph's slot streams) captured into one
  * HIP graph; tm_batch_run replays it.  The graph records no memset: every
  * clear is a kernel.  Counts equal tm_batch_count's.  While a prepared batch
  * exists, other calls on its graph may run between its replays (each launch
