@@ -201,7 +201,7 @@ __global__ void rgap_kernel(const tm_edge *__restrict__ Eg, int E, const int *t0
   for (int k = 0; k < TM_NTFIRST; k++) {
     const int f = tf[k][p];
     unsigned gap = 0xffffffffu;
-    if (e.u != e.v && f != 0x7fffffff) {
+    if (e.u != e.v) {  // (no next edge looks like one at the last time there is, which may be one: it passes)
       const long long d = (long long)f - e.t;
       gap = d > 0x7fffffffll ? 0x7fffffffu : (unsigned)d;
     }

@@ -189,7 +189,7 @@ __device__ __forceinline__ int pend_of(const tm_graph_view &g, long long tl, Met
   if (k >= g.nbuckets) return g.E;
   int lo = g.bucket[k], hi = g.bucket[k + 1];
   if (mt) mt->b += 8;
-  return upper_bound_i(g.T, lo, hi, (int)tl, mt);
+  return upper_bound_i(g.T, lo, hi, tl < 0x7fffffffll ? (int)tl : 0x7fffffff, mt);  // (a bucket may reach past the last time)
 }
 
 // first index in [lo, hi) with a[i] >= x, probing outward from lo
