@@ -201,7 +201,8 @@ __global__ void rgap_kernel(const tm_edge *__restrict__ Eg, int E, const int *t0
   for (int k = 0; k < TM_NTFIRST; k++) {
     const int f = tf[k][p];
     unsigned gap = 0xffffffffu;
-    if (e.u != e.v) {  // (no next edge looks like one at the last time there is, which may be one: it passes)
+    // (no next edge looks like one at the last time there is: where the graph has such edges, it passes)
+    if (e.u != e.v && (f != 0x7fffffff || Eg[E - 1].t == 0x7fffffff)) {
       const long long d = (long long)f - e.t;
       gap = d > 0x7fffffffll ? 0x7fffffffu : (unsigned)d;
     }
@@ -209,7 +210,7 @@ __global__ void rgap_kernel(const tm_edge *__restrict__ Eg, int E, const int *t0
   }
 }
 
-// Per rule, the root gaps by their number of bits (none: not counted).
+// Per rule, the root gaps by their number of bits (no gap: not counted).
 __global__ void __launch_bounds__(256) gap_hist_kernel(const unsigned *__restrict__ rgap, int epad, int E,
                                                        unsigned *__restrict__ hist) {
   __shared__ unsigned h[TM_NTFIRST * 33];

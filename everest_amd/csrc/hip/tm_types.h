@@ -100,8 +100,9 @@ typedef struct {
   // a pointer table).
   const int *stf;
   // Root gaps, one array per TM_T_* rule: tfirst - T[p] clamped to INT_MAX,
-  // or 0xffffffff when p is a self-loop or has no candidate; a root passes a
-  // query with that rule for edge 1 iff gap <= delta.  Padded with
+  // or 0xffffffff when p is a self-loop or has no candidate (unless the graph has
+  // edges at time INT_MAX, the mark of none); a root is dropped from a query
+  // with that rule unless gap <= delta.  Padded with
   // 0xffffffff to a multiple of 256 entries plus 256, so a 256-root block
   // read as one 16-byte load per lane never leaves the array.
   const unsigned *rgap;    // TM_NTFIRST arrays of epad entries, one allocation
