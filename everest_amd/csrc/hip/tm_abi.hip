@@ -1442,9 +1442,9 @@ tm_status tm_graph_upload(int32_t device, const tm_host_graph *hg, tm_graph **ou
   hipLaunchKernelGGL(low_word_kernel, dim3((E + 255) / 256), dim3(256), 0, s, skey, (int *)vw.outPairNbr, E);
   TMPCHK(hipGetLastError());
   {
-    // the pair table, at most half full: the next power of two (about 0.4 full; a
-    // 5-cycle on 3.1M hub edges takes 1% more at 0.5) where that is an eighth of
-    // the free memory at most, else no more than two entries per edge: a graph
+    // the pair table, at most half full: the next power of two (about 0.4 full, for
+    // fewer probes: a 5-cycle on 3.1M hub edges 0.5% faster than at 0.5) where that
+    // is an eighth of the free memory at most, else no more than two entries per edge: a graph
     // that fills the memory gets 8 words an edge, not up to 16
     unsigned long long pairs = 0, *d_pairs = okey;  // (okey is not needed any more)
     TMPCHK(hipMemsetAsync(d_pairs, 0, sizeof(pairs), s));
